@@ -222,59 +222,52 @@ int embed_launch(janus_ctx *ctx, const janus_weight *table, const uint32_t *h_id
 
 // ---- greedy argmax --------------------------------------------------------------
 // TIE_LAST: the last maximal index (Iterator::max_by, model/sampler.rs:784-795);
-// NaN entries never win. TIE_WGSL: the 256-lane scan and strict '>' tree of
-// argmax.wgsl:26-126 reproduced lane for lane.
-__global__ __launch_bounds__(1024) void argmax_last_kernel(const float *__restrict__ logits, int32_t *__restrict__ out,
-                                                           uint32_t vocab) {
+// NaN entries never win. TIE_WGSL: the 256-lane scan from -1e38 and strict '>'
+// tree of argmax.wgsl:26-126: among equal values the smallest
+// (bitrev8(i % 256), i) wins, and without a value above -1e38 index 0.
+//
+// One 1024-thread workgroup per row, 16 loads of a thread in flight: a row's
+// scan is bound by memory round trips (one load in flight per thread of a
+// 256-thread workgroup took 34 us for 32000 logits; this takes 6).
+template <bool WGSL>
+__global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ logits, int32_t *__restrict__ out,
+                                                      uint32_t vocab) {
     __shared__ float sv[16];
-    __shared__ int32_t si[16];
+    __shared__ uint64_t sp[16];
     const float *l = logits + (size_t)blockIdx.x * vocab;
-    float bv = -INFINITY;
-    int32_t bi = -1;
-    for (uint32_t i = threadIdx.x; i < vocab; i += 1024u) {
-        float v = l[i];
-        if (v > bv || (v == bv && (int32_t)i > bi)) { bv = v; bi = (int32_t)i; }
+    // preference among equal values, smaller first; none: nothing chosen yet
+    constexpr uint64_t none = ~0ull;
+    auto pref = [](uint32_t i) -> uint64_t {
+        return WGSL ? ((uint64_t)__builtin_bitreverse32(i << 24) << 32) | i : (uint64_t)(uint32_t)~i;
+    };
+    float bv = WGSL ? -1e38f : -INFINITY;
+    uint64_t bp = none;
+    auto take = [&](float v, uint64_t p) {
+        if (v > bv || (v == bv && p < bp)) { bv = v; bp = p; }
+    };
+    for (uint32_t base = threadIdx.x; base < vocab; base += 16 * 1024u) {
+        float v[16];
+#pragma unroll
+        for (uint32_t u = 0; u < 16; ++u) v[u] = base + u * 1024u < vocab ? l[base + u * 1024u] : NAN;
+#pragma unroll
+        for (uint32_t u = 0; u < 16; ++u)
+            if (!WGSL || v[u] > -1e38f) take(v[u], pref(base + u * 1024u));
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        float ov = shfl_xor(bv, o);
-        int32_t oi = shfl_xor(bi, o);
-        if (ov > bv || (ov == bv && oi > bi)) { bv = ov; bi = oi; }
-    }
-    if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
+    for (int o = 32; o > 0; o >>= 1) take(shfl_xor(bv, o), shfl_xor(bp, o));
+    if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; sp[threadIdx.x >> 6] = bp; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; ++w)
-            if (sv[w] > bv || (sv[w] == bv && si[w] > bi)) { bv = sv[w]; bi = si[w]; }
-        out[blockIdx.x] = bi < 0 ? 0 : bi;
+        for (int w = 1; w < 16; ++w) take(sv[w], sp[w]);
+        out[blockIdx.x] = bp == none ? 0 : WGSL ? (int32_t)(uint32_t)bp : (int32_t)~(uint32_t)bp;
     }
-}
-
-__global__ __launch_bounds__(256) void argmax_wgsl_kernel(const float *__restrict__ logits, int32_t *__restrict__ out,
-                                                          uint32_t vocab) {
-    __shared__ float sv[256];
-    __shared__ int32_t si[256];
-    const float *l = logits + (size_t)blockIdx.x * vocab;
-    const uint32_t t = threadIdx.x;
-    float mv = -1e38f;
-    int32_t mi = 0;
-    for (uint32_t i = t; i < vocab; i += 256)
-        if (l[i] > mv) { mv = l[i]; mi = (int32_t)i; }
-    sv[t] = mv;
-    si[t] = mi;
-    __syncthreads();
-    for (uint32_t stride = 128; stride >= 2; stride >>= 1) {
-        if (t < stride && sv[t + stride] > sv[t]) { sv[t] = sv[t + stride]; si[t] = si[t + stride]; }
-        __syncthreads();
-    }
-    if (t == 0) out[blockIdx.x] = sv[1] > sv[0] ? si[1] : si[0];
 }
 
 int argmax_launch(janus_ctx *ctx, const float *logits, int32_t *out, uint32_t vocab, uint32_t batch, int tie) {
     if (tie == JANUS_TIE_WGSL)
-        hipLaunchKernelGGL(argmax_wgsl_kernel, dim3(batch), dim3(256), 0, ctx->stream, logits, out, vocab);
+        hipLaunchKernelGGL(argmax_kernel<true>, dim3(batch), dim3(1024), 0, ctx->stream, logits, out, vocab);
     else
-        hipLaunchKernelGGL(argmax_last_kernel, dim3(batch), dim3(1024), 0, ctx->stream, logits, out, vocab);
+        hipLaunchKernelGGL(argmax_kernel<false>, dim3(batch), dim3(1024), 0, ctx->stream, logits, out, vocab);
     JANUS_LAUNCH_CHECK(ctx);
     return JANUS_OK;
 }

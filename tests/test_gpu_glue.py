@@ -137,6 +137,30 @@ def test_argmax_kat_and_tie_rules(engine):
             assert got_wgsl[b] == O.argmax_wgsl(logits[b])
 
 
+@pytest.mark.parametrize("v", [1, 63, 1023, 1024, 1025, 16384, 16385, 32000, 128257])
+def test_argmax_edges_of_the_scan(engine, v):
+    """Sizes around the workgroup's 1024 lanes and its 16384-logit round; ties
+    at the first and last index, signed zeros, infinities, NaN, and rows with
+    no value above -1e38, against the oracle's two rules."""
+    rng = np.random.default_rng(v)
+    rows = np.stack([rng.standard_normal(v), np.full(v, -2e38), np.zeros(v), rng.standard_normal(v),
+                     np.full(v, -np.inf), rng.standard_normal(v)]).astype(np.float32)
+    rows[0, [0, v - 1]] = 9.0
+    rows[2, ::2] = -0.0
+    rows[3, v // 2] = np.nan
+    rows[5, [v // 3, v - 1]] = np.inf
+    out = torch.zeros(6, dtype=torch.int32, device=DEV)
+    for rule, want in ((ops.TIE_LAST, O.argmax_last), (ops.TIE_WGSL, O.argmax_wgsl)):
+        ops.argmax(engine, T(rows), out, v, 6, rule)
+        got = out.cpu().tolist()
+        for b in range(6):
+            if rule == ops.TIE_LAST and b == 3:   # NaN never wins
+                clean = np.where(np.isnan(rows[b]), -np.inf, rows[b])
+                assert got[b] == (O.argmax_last(clean) if v > 1 else 0)
+            else:
+                assert got[b] == want(rows[b]), (rule, b)
+
+
 def test_repetition_penalty(engine):
     rng = np.random.default_rng(4)
     logits = rng.standard_normal(1000).astype(np.float32)
