@@ -131,6 +131,8 @@ int janus_weight_dequant(janus_ctx *ctx, const janus_weight *w, float *d_out);
 /* C[b, i, :] = A[b, i, :] . W^T for b < batch, i < m; A is [batch*m][k] of
  * a_dtype (F32 or F16), C is [batch*m][n] of c_dtype (F32 or F16). Rows
  * batch*m == 1 run the GEMV kernels; up to 64 rows run the small-M MFMA GEMM
+ * (F32 rows as three exact bfloat16 parts; two F32 rows, or three of a small
+ * product, run the GEMV kernels row by row)
  * (the reference's M>1 quantized fallback, quantized.rs:77-90, is replaced
  * by a correct product). k and n must match the weight. */
 int janus_gemm_auto(janus_ctx *ctx, const void *a, int a_dtype, const janus_weight *w,

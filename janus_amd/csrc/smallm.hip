@@ -1,5 +1,6 @@
 // smallm.hip -- products with 2..64 activation rows (ragged decode batches):
-// the dequant-fused fp16 MFMA GEMM.
+// the dequant-fused MFMA GEMM, on binary16 activations or on binary32 ones
+// split into three bfloat16 parts.
 //
 // Replaces the reference's M>1 quantised path, which hands quantised bytes
 // to the f16 GEMM (crates/janus-engine/src/compute/ops/quantized.rs:77-90,
@@ -46,6 +47,8 @@ namespace janus {
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 typedef float f16x __attribute__((ext_vector_type(16)));
 
 constexpr int WAVES = 4;   // row groups per workgroup
@@ -103,6 +106,151 @@ __device__ __forceinline__ h8 unpack_i8x8(uint32_t lo, uint32_t hi) {
     return (h8){p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
 }
 
+// ---- binary32 activations: three bfloat16 parts ---------------------------------
+// A finite binary32 x is exactly x1 + x2 + x3 with bfloat16 parts of 8
+// significant bits each (x1 = the upper 16 bits of x, x2 those of x - x1, x3
+// the rest), over the whole binary32 range, and the quantised weights are
+// exact bfloat16 integers. So a product of binary32 activations is three
+// v_mfma_f32_32x32x16_bf16 per operand pair, every partial product exact and
+// every sum binary32, with nothing rounded on the way in: the weights are read
+// once for all rows instead of once per row by the M = 1 kernel.
+
+// Bytes (b0, b1) / (b2, b3) of v (each below 16) as exact bfloat16 integers
+// (OCP e4m3 byte b < 16 is b * 2^-9; the conversion scales it by 512).
+template <bool HI> __device__ __forceinline__ b2 nib8_bf16(uint32_t v) {
+    return __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, HI);
+}
+
+// The upper halves of two floats as a bfloat16 pair (exact for integers below 256).
+__device__ __forceinline__ uint32_t pack_hi16(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
+// A T32 word of 8 nibbles -> 8 bfloat16 integers in the order e0 e4 e1 e5 e2
+// e6 e3 e7 (the byte order of the word's low and high nibbles); the
+// activations are staged in the same order (SplitOrder).
+__device__ __forceinline__ b8 unpack_nib8_b(uint32_t u) {
+    const uint32_t lo = u & 0x0f0f0f0fu, hi = (u >> 4) & 0x0f0f0f0fu;
+    const b2 p0 = nib8_bf16<false>(lo), p1 = nib8_bf16<true>(lo), p2 = nib8_bf16<false>(hi), p3 = nib8_bf16<true>(hi);
+    return (b8){p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
+}
+
+__device__ __forceinline__ b8 as_b8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_bit_cast(b8, make_uint4(a, b, c, d));
+}
+
+// Q5_K word I: the fifth bits join the nibble bytes (bit 4), then bytes -> bfloat16.
+template <int I>
+__device__ __forceinline__ b8 unpack_nib8_q5_b(uint32_t u, uint32_t fifth) {
+    const uint32_t f = fifth >> I;
+    const uint32_t lo = (u & 0x0f0f0f0fu) | ((f << 4) & 0x10101010u);
+    const uint32_t hi = ((u >> 4) & 0x0f0f0f0fu) | (f & 0x10101010u);
+    auto pair = [](uint32_t v, int s) { return pack_hi16((float)((v >> s) & 255u), (float)((v >> (s + 8)) & 255u)); };
+    return as_b8(pair(lo, 0), pair(lo, 16), pair(hi, 0), pair(hi, 16));
+}
+
+// 8 int8 (two words) -> 8 bfloat16 integers, natural order.
+__device__ __forceinline__ b8 unpack_i8x8_b(uint32_t lo, uint32_t hi) {
+    auto pair = [](uint32_t v, int s) {
+        return pack_hi16((float)(int)(int8_t)(v >> s), (float)(int)(int8_t)(v >> (s + 8)));
+    };
+    return as_b8(pair(lo, 0), pair(lo, 16), pair(hi, 0), pair(hi, 16));
+}
+
+// 8 finite binary16 weights -> their upper 8 bits and the remaining 3, both
+// exact bfloat16 (natural order).
+__device__ __forceinline__ void split_f16x8(const uint4 &q, b8 &hi, b8 &lo) {
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+    uint32_t a[4], b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float e = h2f((uint16_t)(w[i] & 0xffffu)), o = h2f((uint16_t)(w[i] >> 16));
+        a[i] = pack_hi16(e, o);
+        b[i] = pack_hi16(e - __uint_as_float(__float_as_uint(e) & 0xffff0000u),
+                         o - __uint_as_float(__float_as_uint(o) & 0xffff0000u));
+    }
+    hi = as_b8(a[0], a[1], a[2], a[3]);
+    lo = as_b8(b[0], b[1], b[2], b[3]);
+}
+
+// x[0..8) -> its three bfloat16 parts, 8 values each in one 16-byte word.
+// ORDER4: in the order of unpack_nib8_b, else natural. An infinite x is all in
+// the first part; a NaN stays a NaN in the second. Returns whether an x is
+// infinite.
+template <bool ORDER4>
+__device__ __forceinline__ bool split_x8(const float (&x)[8], uint4 (&part)[3]) {
+    float r[8];
+    float top = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        r[i] = x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u);
+        top = fmaxf(top, fabsf(x[i]));
+    }
+    if (top == INFINITY) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (fabsf(x[i]) == INFINITY) r[i] = 0.0f;
+    }
+    float s[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[i] = r[i] - __uint_as_float(__float_as_uint(r[i]) & 0xffff0000u);
+    auto pack = [](const float (&v)[8]) {
+        return ORDER4 ? make_uint4(pack_hi16(v[0], v[4]), pack_hi16(v[1], v[5]), pack_hi16(v[2], v[6]), pack_hi16(v[3], v[7]))
+                      : make_uint4(pack_hi16(v[0], v[1]), pack_hi16(v[2], v[3]), pack_hi16(v[4], v[5]), pack_hi16(v[6], v[7]));
+    };
+    part[0] = pack(x);
+    part[1] = pack(r);
+    part[2] = pack(s);
+    return top == INFINITY;
+}
+
+// The finite values of 8 bfloat16, infinities as 0.
+__device__ __forceinline__ b8 strip_inf(b8 x) {
+    uint4 v = __builtin_bit_cast(uint4, x);
+    uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if ((u[i] & 0x7fffu) == 0x7f80u) u[i] &= 0xffff0000u;
+        if ((u[i] & 0x7fff0000u) == 0x7f800000u) u[i] &= 0xffffu;
+    }
+    return as_b8(u[0], u[1], u[2], u[3]);
+}
+
+__device__ __forceinline__ f16x mfma_b(b8 a, b8 b, f16x c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// One 32-element block of one M-tile: t + (the three parts of A, rows at ap,
+// `plane` halves apart) x (b0: elements 0-15, b1: 16-31). From t = 0 the
+// smallest part goes first (only the leading part's two sums round at full
+// size). FROM_OFFSET: t is the block's offset term, as large as the sums
+// themselves; the leading part cancels most of it first.
+template <bool FROM_OFFSET>
+__device__ __forceinline__ f16x block_b(const _Float16 *ap, uint32_t plane, b8 b0, b8 b1, f16x t) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int part = FROM_OFFSET ? i : 2 - i;
+        t = mfma_b(*(const b8 *)(ap + part * plane), b0, t);
+        t = mfma_b(*(const b8 *)(ap + part * plane + 16), b1, t);
+    }
+    return t;
+}
+
+// The 16 per-row values of a lane's tile rows from s (one float per row): rows
+// 8 j + 4 h + 0..3 (the MFMA C layout).
+__device__ __forceinline__ f16x tile_rows(const float *s, int h) {
+    f16x t;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const jf4 v = *(const jf4 *)(s + 8 * j + 4 * h);
+        t[4 * j] = v.x;
+        t[4 * j + 1] = v.y;
+        t[4 * j + 2] = v.z;
+        t[4 * j + 3] = v.w;
+    }
+    return t;
+}
+
 __device__ __forceinline__ f16x mfma(h8 a, h8 b, f16x c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
@@ -114,6 +262,7 @@ struct GemmArgs {
     const uint8_t *side;   // T32 side data (scales / headers)
     const uint32_t *q5h;   // Q5_K fifth bits [G][C][64]
     const _Float16 *a;     // activations [rows][k]
+    const float *a32;      // binary32 activations (X32 kernels; a is null then)
     void *c;               // output [rows][n]
     const float *resid;    // [rows][n] or null (may alias c)
     float *ws;             // split-K partials [ksplit][Mpad][Npad]
@@ -142,10 +291,43 @@ template <int MT> struct Deferred {
     float d;      // and its scale (0 before the first block)
 };
 
+// acc += the pending block's scaled results; t with scale d becomes pending.
+template <int MT>
+__device__ __forceinline__ void apply_deferred(f16x (&acc)[MT], Deferred<MT> &pend, const f16x (&t)[MT], float d) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) pend.t[mt] = t[mt];
+    pend.d = d;
+}
+
 struct GQ4_0 {
     static constexpr int CK = 64;
     static constexpr bool DEFER = true;
+    static constexpr bool ORDER4 = true;
+    static constexpr float XSUM = -8.0f;   // X32: per-block sums are staged times this
     struct W { uint4 q; uint32_t s; };
+    // One chunk on binary32 activations: As holds their three bfloat16 parts
+    // (`plane` halves apart). The offset -8 enters as the first accumulator,
+    // -8 * sum(x) of the block, so the weights stay the integers 0..15.
+    template <int MT>
+    __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
+                                   uint32_t, int lane, const float *Ss, f16x (&acc)[MT], Deferred<MT> &pend) {
+        const int h = lane >> 5, r = lane & 31;
+        const uint32_t q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const b8 b0 = unpack_nib8_b(q[2 * b]), b1 = unpack_nib8_b(q[2 * b + 1]);
+            f16x t[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                t[mt] = block_b<true>(As + (size_t)(mt * 32 + r) * pitch + kl + b * 32 + 8 * h, plane, b0, b1,
+                                tile_rows(Ss + (size_t)(kl / 32 + b) * (MT * 32) + mt * 32, h));
+            apply_deferred<MT>(acc, pend, t, h2f((uint16_t)(b ? (w.s >> 16) : (w.s & 0xffffu))));
+        }
+    }
     // g and c are wavefront-uniform: the chunk base is scalar, the lane adds
     // a 32-bit offset
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
@@ -205,7 +387,21 @@ struct GQ4_0 {
 
 struct GQ8_0 {
     static constexpr int CK = 32;
+    static constexpr bool ORDER4 = false;
+    static constexpr float XSUM = 0.0f;   // no sums
     struct W { uint4 q; uint16_t s; };
+    // see GQ4_0::mma_x32
+    template <int MT>
+    __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
+                                   uint32_t, int lane, const float *, f16x (&acc)[MT], Deferred<MT> &pend) {
+        const int h = lane >> 5, r = lane & 31;
+        const b8 b0 = unpack_i8x8_b(w.q.x, w.q.y), b1 = unpack_i8x8_b(w.q.z, w.q.w);
+        f16x t[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+            t[mt] = block_b<false>(As + (size_t)(mt * 32 + r) * pitch + kl + 8 * h, plane, b0, b1, (f16x){});
+        apply_deferred<MT>(acc, pend, t, h2f_q8(w.s));
+    }
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
         const size_t ch = (size_t)g * a.chunks + c;
         W w;
@@ -235,7 +431,43 @@ struct GQ8_0 {
 // the m term uses the per-(row, sub-block) activation sums staged in LDS.
 struct GQ4_K {
     static constexpr int CK = 64;
+    static constexpr bool ORDER4 = true;
+    static constexpr float XSUM = -8.0f;
     struct W { uint4 q; uint4 hdr; };
+    // binary32 activations (three bfloat16 parts, GQ4_0::mma_x32). The staged
+    // sums are -8 sum(x) (Q5_K: -16), so the MFMA result is that of the centred
+    // values q - 8 and ds * (q . x) - dm * sum(x) = ds * t + (dm - 8 ds) / 8 * staged:
+    // the two large terms of a block mostly cancel before they are rounded.
+    // c: chunk of the row group.
+    template <int MT, class G = GQ4_K>
+    __device__ static void mma_x32(const typename G::W &w, const _Float16 *As, uint32_t plane, uint32_t pitch,
+                                   uint32_t kl, uint32_t c, int lane, const float *Ss, f16x (&acc)[MT],
+                                   Deferred<MT> &) {
+        const int h = lane >> 5, r = lane & 31;
+        const float d = h2f((uint16_t)(w.hdr.x & 0xffffu)), dmin = h2f((uint16_t)(w.hdr.x >> 16));
+        const int j = (int)(c & 3);   // chunk index within the super-block
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            float sc, mn;
+            scale_min(w.hdr, 2 * j + b, sc, mn);
+            const float ds = d * sc, dm = dmin * mn;
+            const float cs = fmaf(G::XSUM, ds, dm) * (-1.0f / G::XSUM);   // the power of two is exact
+            b8 b0, b1;
+            G::unpack_b(w, b, b0, b1);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const f16x s = tile_rows(Ss + (size_t)(kl / 32 + b) * (MT * 32) + mt * 32, h);
+                const f16x t =
+                    block_b<true>(As + (size_t)(mt * 32 + r) * pitch + kl + b * 32 + 8 * h, plane, b0, b1, s);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(cs, s[v], fmaf(ds, t[v], acc[mt][v]));
+            }
+        }
+    }
+    __device__ static void unpack_b(const W &w, int b, b8 &b0, b8 &b1) {
+        b0 = unpack_nib8_b(b ? w.q.z : w.q.x);
+        b1 = unpack_nib8_b(b ? w.q.w : w.q.y);
+    }
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
         const size_t ch = (size_t)g * a.chunks + c;
         W w;
@@ -289,7 +521,18 @@ struct GQ4_K {
 // dmin*m with q in 0..31, the m term from the staged activation sums.
 struct GQ5_K {
     static constexpr int CK = 64;
+    static constexpr bool ORDER4 = true;
+    static constexpr float XSUM = -16.0f;
     struct W { uint4 q; uint4 hdr; uint32_t fifth; };
+    template <int MT>
+    __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
+                                   uint32_t c, int lane, const float *Ss, f16x (&acc)[MT], Deferred<MT> &pend) {
+        GQ4_K::mma_x32<MT, GQ5_K>(w, As, plane, pitch, kl, c, lane, Ss, acc, pend);
+    }
+    __device__ static void unpack_b(const W &w, int b, b8 &b0, b8 &b1) {
+        b0 = b ? unpack_nib8_q5_b<2>(w.q.z, w.fifth) : unpack_nib8_q5_b<0>(w.q.x, w.fifth);
+        b1 = b ? unpack_nib8_q5_b<3>(w.q.w, w.fifth) : unpack_nib8_q5_b<1>(w.q.y, w.fifth);
+    }
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
         const size_t ch = (size_t)g * a.chunks + c;
         W w;
@@ -351,7 +594,32 @@ template <> struct NeedsSums<GQ5_K> { static constexpr bool value = true; };
 
 struct GF16 {
     static constexpr int CK = 16;
+    static constexpr bool ORDER4 = false;
+    static constexpr float XSUM = 0.0f;
     struct W { uint4 q; };
+    // binary32 activations: the weight is two bfloat16 parts, so a 16-wide
+    // chunk is six MFMAs. The product of the two leading parts goes to acc,
+    // the five small ones (below 2^-7 of it) to pend.t, added at the end, so
+    // their roundings stay at their own size. inf: an activation may be
+    // infinite; it then meets only the leading weight part (the other may be 0).
+    template <int MT>
+    __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
+                                   uint32_t inf, int lane, const float *, f16x (&acc)[MT], Deferred<MT> &pend) {
+        const int h = lane >> 5, r = lane & 31;
+        b8 hi, lo;
+        split_f16x8(w.q, hi, lo);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const _Float16 *ap = As + (size_t)(mt * 32 + r) * pitch + kl + 8 * h;
+            const b8 x1 = *(const b8 *)ap, x2 = *(const b8 *)(ap + plane), x3 = *(const b8 *)(ap + 2 * plane);
+            acc[mt] = mfma_b(x1, hi, acc[mt]);
+            pend.t[mt] = mfma_b(x3, lo, pend.t[mt]);
+            pend.t[mt] = mfma_b(x3, hi, pend.t[mt]);
+            pend.t[mt] = mfma_b(x2, lo, pend.t[mt]);
+            pend.t[mt] = mfma_b(x2, hi, pend.t[mt]);
+            pend.t[mt] = mfma_b(inf ? strip_inf(x1) : x1, lo, pend.t[mt]);
+        }
+    }
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
         const size_t ch = (size_t)g * a.chunks + c;
         W w;
@@ -548,6 +816,16 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_mfma_kernel(GemmArgs a) 
             __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * Mpad + out_row(mt, v, lane)) * Npad + n);
 }
 
+// Bytes of one staging buffer of gemm_pipe_kernel: the activations (three
+// bfloat16 planes with X32) and, where the format needs them, the per-block sums.
+template <class F, int MT, int KR, bool X32>
+constexpr uint32_t pipe_buf() {
+    constexpr uint32_t abytes = (uint32_t)MT * 32 * (KR + 8) * 2 * (X32 ? 3 : 1);
+    constexpr bool sums = X32 ? F::XSUM != 0.0f : NeedsSums<F>::value;
+    constexpr bool flag = X32 && std::is_same<F, GF16>::value;   // an infinite activation was staged
+    return (abytes + (sums ? (uint32_t)(KR / 32) * MT * 32 * 4 : flag ? 4u : 0u) + 15u) / 16u * 16u;
+}
+
 // Sums the split-K partials in split order and applies the epilogue.
 // Cross-pass pipelined form of gemm_mfma_kernel (quantised and F16 weights),
 // with the pass length KR fixed at compile time. A is double-buffered in LDS:
@@ -558,10 +836,13 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_mfma_kernel(GemmArgs a) 
 // previous pass and the barrier between them. One barrier per pass (two for
 // Q4_K, whose activation sums are built from the staged pass). Products,
 // scale rounding, slice order and outputs are those of gemm_mfma_kernel.
-template <class F, int MT, int KW, int KR>
+// X32: binary32 activations, split into three bfloat16 parts as they are
+// stored to LDS (three planes per buffer); their per-block sums come from the
+// staging lanes themselves, so there is no separate pass over the stage.
+template <class F, int MT, int KW, int KR, bool X32>
 __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr bool SUMS = NeedsSums<F>::value;
+    constexpr bool SUMS = NeedsSums<F>::value && !X32;
     constexpr int NT = 64 * WAVES * KW;   // threads
     constexpr int PC = KR / F::CK;        // chunks per pass
     constexpr int CPW = PC / KW;          // chunks per wavefront per pass
@@ -570,8 +851,10 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
     constexpr int SEGS = KR / 8;          // 16-byte segments per row of a pass
     constexpr int SPT = MP * SEGS / NT;   // segments per thread
     static_assert(CPW >= 1 && CPW * KW == PC && SPT >= 1 && SPT * NT == MP * SEGS, "pass shape");
-    constexpr uint32_t ABYTES = (uint32_t)MP * PITCH * 2;
-    constexpr uint32_t BUF = (ABYTES + (SUMS ? (uint32_t)(KR / 32) * MP * 4 : 0u) + 15u) / 16u * 16u;
+    constexpr uint32_t PLANE = (uint32_t)MP * PITCH;   // halves of one staged part
+    constexpr uint32_t ABYTES = PLANE * 2 * (X32 ? 3 : 1);
+    constexpr uint32_t BUF = pipe_buf<F, MT, KR, X32>();
+    constexpr bool FLAG = X32 && std::is_same<F, GF16>::value;   // one word per buffer after the activations
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar chunk bases
     const int rgw = wave % WAVES, kw = wave / WAVES;
@@ -589,7 +872,7 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
     for (int mt = 0; mt < MT; ++mt) pend.t[mt] = (f16x){};
     pend.d = 0.0f;
     typename F::W w[CPW];
-    uint4 sv[SPT];
+    uint4 sv[SPT * (X32 ? 2 : 1)];
 
     // Every wavefront issues the same sequence of loads whatever the shape
     // (addresses clamped into range, out-of-range A zeroed when stored,
@@ -602,7 +885,13 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
         for (int i = 0; i < SPT; ++i) {
             const uint32_t s = threadIdx.x + NT * i;
             const uint32_t m = min(s / SEGS, a.rows - 1), col = min(kbase + (s % SEGS) * 8, a.k - 8);
-            sv[i] = *(const uint4 *)(a.a + (size_t)m * a.k + col);
+            if constexpr (X32) {
+                const uint4 *p = (const uint4 *)(a.a32 + (size_t)m * a.k + col);
+                sv[2 * i] = p[0];
+                sv[2 * i + 1] = p[1];
+            } else {
+                sv[i] = *(const uint4 *)(a.a + (size_t)m * a.k + col);
+            }
         }
     };
     auto store_a = [&](uint32_t p) {
@@ -612,6 +901,28 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
         for (int i = 0; i < SPT; ++i) {
             const uint32_t s = threadIdx.x + NT * i;
             const bool ok = s / SEGS < a.rows && kbase + (s % SEGS) * 8 < a.k;
+            if constexpr (X32) {
+                const uint4 lo = sv[2 * i], hi = sv[2 * i + 1];
+                const uint32_t u[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = ok ? __uint_as_float(u[e]) : 0.0f;
+                uint4 part[3];
+                const bool inf = split_x8<F::ORDER4>(x, part);
+                if (FLAG && inf) *(uint32_t *)(smem + (p & 1) * BUF + ABYTES) = 1u;
+                _Float16 *at = As + (s / SEGS) * PITCH + (s % SEGS) * 8;
+#pragma unroll
+                for (int j = 0; j < 3; ++j) *(uint4 *)(at + j * PLANE) = part[j];
+                if constexpr (F::XSUM != 0.0f) {
+                    // the four lanes of a quad hold one 32-element block
+                    float t = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+                    t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0xb1, 0xf, 0xf, false));
+                    t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x4e, 0xf, 0xf, false));
+                    float *Ss = (float *)(smem + (p & 1) * BUF + ABYTES);
+                    if (!(threadIdx.x & 3)) Ss[(s % SEGS) / 4 * MP + s / SEGS] = F::XSUM * t;
+                }
+                continue;
+            }
             *(uint4 *)(As + (s / SEGS) * PITCH + (s % SEGS) * 8) = ok ? sv[i] : make_uint4(0u, 0u, 0u, 0u);
         }
     };
@@ -640,21 +951,41 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
         const _Float16 *As = (const _Float16 *)(smem + (p & 1) * BUF);
         const float *Ss = (const float *)(smem + (p & 1) * BUF + ABYTES);
         const uint32_t c1 = min(a.chunks, (p + 1) * PC), m0 = p * PC + kw * CPW;
+        // X32: a pass is summed on its own and then added, so the sum over K
+        // takes one long rounding per pass and not one per block
+        f16x part[MT];
+        if constexpr (X32)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) part[mt] = (f16x){};
+        // F16: Ss is the flag of an infinite activation in the staged passes
+        const uint32_t inf = X32 && FLAG ? __builtin_amdgcn_readfirstlane(*(const uint32_t *)Ss) : 0u;
 #pragma unroll
         for (int i = 0; i < CPW; ++i) {
             if (m0 + i < c1) {
-                if constexpr (Defers<F>::value)
+                if constexpr (X32)
+                    F::template mma_x32<MT>(w[i], As, PLANE, PITCH, (uint32_t)(kw * CPW + i) * F::CK,
+                                            FLAG ? inf : m0 + i, lane, Ss, part, pend);
+                else if constexpr (Defers<F>::value)
                     F::template mma_deferred<MT>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, acc, pend);
                 else
                     F::template mma<MT>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, Ss, 0, acc);
             }
             if (decltype(load_next)::value) w[i] = F::load(a, gl, chunk_of(p + 1, i), lane);
         }
+        if constexpr (X32)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[mt][v] += part[mt][v];
     };
 
     if (p_begin < p_end) {
         const uint32_t last = p_end - 1;
         load_a(p_begin);
+        if constexpr (FLAG) {   // never cleared again: a set flag costs later passes time, not results
+            if (threadIdx.x < 2) *(uint32_t *)(smem + threadIdx.x * BUF + ABYTES) = 0u;
+            __syncthreads();
+        }
 #pragma unroll
         for (int i = 0; i < CPW; ++i) w[i] = F::load(a, gl, chunk_of(p_begin, i), lane);
         store_a(p_begin);
@@ -676,7 +1007,8 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
         }
         pass(last, std::false_type{});
     }
-    if constexpr (Defers<F>::value) flush_deferred<MT>(acc, pend);
+    if constexpr (X32 && std::is_same<F, GF16>::value) pend.d = 1.0f;   // the small parts
+    if constexpr (X32 ? !NeedsSums<F>::value : Defers<F>::value) flush_deferred<MT>(acc, pend);
 
     if (KW > 1) {
         float *red = (float *)smem;
@@ -710,29 +1042,30 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
             __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * MP + out_row(mt, v, lane)) * Npad + n);
 }
 
-// LDS bytes of gemm_pipe_kernel: two A buffers (with Q4_K sums), at least the
-// K-slice reduction area.
-template <class F, int MT, int KW, int KR>
+// LDS bytes of gemm_pipe_kernel: two staging buffers, at least the K-slice
+// reduction area.
+template <class F, int MT, int KW, int KR, bool X32>
 constexpr size_t pipe_lds() {
-    constexpr size_t abytes = (size_t)MT * 32 * (KR + 8) * 2;
-    constexpr size_t buf = (abytes + (NeedsSums<F>::value ? (size_t)(KR / 32) * MT * 32 * 4 : 0) + 15) / 16 * 16;
+    constexpr size_t buf = pipe_buf<F, MT, KR, X32>();
     constexpr size_t red = (size_t)WAVES * KW * 16 * 64 * 4;
+    static_assert(2 * buf <= 160 * 1024 && red <= 160 * 1024, "LDS");
     return 2 * buf > red ? 2 * buf : red;
 }
 
-template <class F, int MT, int KW, int KR>
+template <class F, int MT, int KW, int KR, bool X32 = false>
 void launch_pipe(janus_ctx *ctx, dim3 grid, const GemmArgs &a) {
     // thread-safe one-time set-up (a function-local static's initialiser)
     static const bool attr_set = [] {
-        (void)hipFuncSetAttribute((const void *)gemm_pipe_kernel<F, MT, KW, KR>,
+        (void)hipFuncSetAttribute((const void *)gemm_pipe_kernel<F, MT, KW, KR, X32>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         return true;
     }();
     (void)attr_set;
-    constexpr size_t lds = pipe_lds<F, MT, KW, KR>();
-    hipLaunchKernelGGL((gemm_pipe_kernel<F, MT, KW, KR>), grid, dim3(64 * WAVES * KW), lds, ctx->stream, a);
+    constexpr size_t lds = pipe_lds<F, MT, KW, KR, X32>();
+    hipLaunchKernelGGL((gemm_pipe_kernel<F, MT, KW, KR, X32>), grid, dim3(64 * WAVES * KW), lds, ctx->stream, a);
 }
 
+// Sums the split-K partials in split order and applies the epilogue.
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, uint32_t Mpad) {
     const uint32_t Npad = (a.n + 31) / 32 * 32;
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -872,22 +1205,26 @@ __global__ void t32_q8_0_kernel(const uint8_t *__restrict__ qs, const uint16_t *
     if (lane < 32) dside[ch * 32 + lane] = s;
 }
 
+// nonfinite is set when any weight is infinite or NaN (cleared by the caller).
 __global__ void t32_f16_kernel(const uint16_t *__restrict__ src, uint8_t *dq, uint32_t n, uint32_t k, uint32_t G,
-                               uint32_t C) {
+                               uint32_t C, uint32_t *nonfinite) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (size_t)G * C * 64) return;
     const int lane = (int)(t & 63), h = lane >> 5;
     const size_t ch = t >> 6;
     const uint32_t g = (uint32_t)(ch / C), c = (uint32_t)(ch % C);
     const uint32_t r = g * 32 + (lane & 31);
-    uint16_t out[8] = {0};
-    if (r < n)
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t kk = c * 16 + 8 * h + e;
-            if (kk < k) out[e] = src[(size_t)r * k + kk];
-        }
-    uint4 v;
-    std::memcpy(&v, out, 16);
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t k0 = c * 16 + 8 * h;
+    if (r < n && k0 < k) {   // k % 8 == 0 (mfma_gemm_supported): whole 16-byte groups
+        v = *(const uint4 *)(src + (size_t)r * k + k0);
+        const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            bad |= (u[i] & 0x7c00u) == 0x7c00u || (u[i] & 0x7c000000u) == 0x7c000000u;
+        if (bad) *nonfinite = 1u;
+    }
     *(uint4 *)(dq + t * 16) = v;
 }
 
@@ -912,6 +1249,8 @@ int t32_ensure(janus_ctx *ctx, janus_weight *w) {
     const size_t fifth = w->type == JANUS_DT_Q5_K ? (size_t)G * C * 64 * 4 : 0;
     void *mem = nullptr;
     JANUS_HIP_CHECK(ctx, hipMalloc(&mem, qbytes + side + fifth + 256));
+    uint32_t *nonfinite = (uint32_t *)((uint8_t *)mem + qbytes + side + fifth);   // all multiples of 64 bytes
+    uint32_t bad = 0;
     uint8_t *dq = (uint8_t *)mem, *ds = (uint8_t *)mem + qbytes;
     uint32_t *df = (uint32_t *)((uint8_t *)mem + qbytes + side);
     const size_t threads = (size_t)G * C * 64;
@@ -932,8 +1271,10 @@ int t32_ensure(janus_ctx *ctx, janus_weight *w) {
                            w->k, G, C);
         break;
     default:
+        (void)hipMemsetAsync(nonfinite, 0, 4, ctx->stream);
         hipLaunchKernelGGL(t32_f16_kernel, grid, block, 0, ctx->stream, (const uint16_t *)w->qs, dq, w->n, w->k, G,
-                           C);
+                           C, nonfinite);
+        (void)hipMemcpyAsync(&bad, nonfinite, 4, hipMemcpyDeviceToHost, ctx->stream);
         break;
     }
     hipError_t e = hipGetLastError();
@@ -947,6 +1288,7 @@ int t32_ensure(janus_ctx *ctx, janus_weight *w) {
     w->t32_side = ds;
     w->t32_q5h = fifth ? df : nullptr;
     w->t32_chunks = C;
+    w->t32_nonfinite = bad != 0;
     return JANUS_OK;
 }
 
@@ -1069,6 +1411,83 @@ int launch_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, GemmPart
     case JANUS_DT_Q4_K: return launch_mfma<GQ4_K, MT>(ctx, a, w, parts);
     case JANUS_DT_Q5_K: return launch_mfma<GQ5_K, MT>(ctx, a, w, parts);
     default: return launch_mfma<GF16, MT>(ctx, a, w, parts);
+    }
+}
+
+// Splits the product for gemm_pipe_kernel on binary32 activations: fills the
+// plan fields of a and returns the workspace bytes (0: no K split). MT M-tiles
+// of 32 rows, KR-long passes. The staged parts fill most of a CU's LDS, so one
+// workgroup runs per CU: K is split as far as the workgroups still fit in one
+// round.
+template <class F, int MT, int KR>
+size_t plan_x32(const janus_ctx *ctx, GemmArgs &a, const janus_weight *w, dim3 &grid) {
+    const uint32_t G = (w->n + 31) / 32, tiles = (G + WAVES - 1) / WAVES;
+    a.chunks = w->t32_chunks;
+    a.pass_chunks = KR / F::CK;
+    a.total_passes = (a.chunks + a.pass_chunks - 1) / a.pass_chunks;
+    uint32_t ks = (uint32_t)ctx->num_cus / tiles;
+    if (ks > a.total_passes) ks = a.total_passes;
+    if (ks < 1) ks = 1;
+    a.passes_per_wg = (a.total_passes + ks - 1) / ks;
+    a.ksplit = (a.total_passes + a.passes_per_wg - 1) / a.passes_per_wg;
+    grid = dim3(tiles, a.ksplit);
+    return a.ksplit > 1 ? (size_t)a.ksplit * MT * 32 * G * 32 * 4 : 0;
+}
+
+// Binary32 rows take the MFMA kernel where it beats a GEMV per row. Per call,
+// two rows: 19-32 us per-row against 19-29 us at 14336x4096 and 4096x14336 (no
+// clear winner); three rows: 29 / 26 / 34 / 60 us per-row (Q4_0, Q8_0 4096x14336,
+// Q4_K, F16 14336x4096) against 23 / 24 / 26 / 31; 16 rows 144 / 229 / 172 / 315
+// against 23 / 25 / 25 / 31; 64 rows 565-1248 against 40-58. Launch-bound sizes
+// (256 to 1024 square) cost 4-8 us against 2.4-3.5 us a row, so they gain from
+// three rows too, but three rows below 2^20 weights stay with the row kernels:
+// their results equal single calls bit for bit, and the time at stake is 3 us.
+bool x32_pays(const janus_weight *w, uint32_t rows) {
+    return rows > 3 || (rows == 3 && (uint64_t)w->n * w->k >= (1u << 20));
+}
+
+bool capturing(const janus_ctx *ctx) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
+
+// Binary32 rows on the MFMA kernel. *ran stays false, with nothing launched
+// and no error, when the workspace cannot grow (out of memory, or inside a
+// capture): the caller then runs one GEMV per row, which needs none.
+template <class F, int MT, int KW = gemm_kw<F, MT>()>
+int launch_x32(janus_ctx *ctx, GemmArgs a, const janus_weight *w, bool *ran) {
+    constexpr int KR = MT == 1 ? 256 : 128;
+    dim3 grid;
+    const size_t need = plan_x32<F, MT, KR>(ctx, a, w, grid);
+    if (need > ctx->gemm_ws_bytes) {
+        if (capturing(ctx)) return JANUS_OK;
+        if (ensure_gemm_ws(ctx, need)) {
+            (void)hipGetLastError();
+            ctx->last_error.clear();
+            return JANUS_OK;
+        }
+    }
+    a.ws = (float *)ctx->gemm_ws;
+    *ran = true;
+    launch_pipe<F, MT, KW, KR, true>(ctx, grid, a);
+    JANUS_LAUNCH_CHECK(ctx);
+    if (a.ksplit > 1) {
+        const size_t total = (size_t)a.rows * w->n;
+        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, a,
+                           (uint32_t)(MT * 32));
+        JANUS_LAUNCH_CHECK(ctx);
+    }
+    return JANUS_OK;
+}
+
+template <int MT>
+int launch_x32_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, bool *ran) {
+    switch (w->type) {
+    case JANUS_DT_Q4_0: return launch_x32<GQ4_0, MT>(ctx, a, w, ran);
+    case JANUS_DT_Q8_0: return launch_x32<GQ8_0, MT>(ctx, a, w, ran);
+    case JANUS_DT_Q4_K: return launch_x32<GQ4_K, MT>(ctx, a, w, ran);
+    case JANUS_DT_Q5_K: return launch_x32<GQ5_K, MT>(ctx, a, w, ran);
+    default: return launch_x32<GF16, MT>(ctx, a, w, ran);
     }
 }
 
@@ -1287,7 +1706,27 @@ int smallm_gemm_launch(janus_ctx *ctx, const void *a, int a_dt, const janus_weig
         const GemmArgs g = make_args(w, a, c, c_dt == JANUS_DT_F16, rows, residual);
         return rows <= 32 ? launch_mt<1>(ctx, g, w, nullptr) : launch_mt<2>(ctx, g, w, nullptr);
     }
-    // f32 activations keep the reference's dtype: one GEMV launch per row
+    // f32 activations keep the reference's precision: three bfloat16 parts on
+    // the MFMA kernel where the weight's tile copy can be had (built outside any
+    // capture; a binary16 weight with an infinity or NaN has no exact parts),
+    // else one GEMV launch per row
+    if (a_dt == JANUS_DT_F32 && mfma_gemm_supported(JANUS_DT_F16, w) && x32_pays(w, rows)) {
+        bool tiles = w->t32 != nullptr;
+        if (!tiles && !capturing(ctx)) {
+            tiles = mfma_gemm_prepare(ctx, w) == JANUS_OK;
+            if (!tiles) {   // no memory for the copy
+                (void)hipGetLastError();
+                ctx->last_error.clear();
+            }
+        }
+        if (tiles && !w->t32_nonfinite) {
+            GemmArgs g = make_args(w, nullptr, c, c_dt == JANUS_DT_F16, rows, residual);
+            g.a32 = (const float *)a;
+            bool ran = false;
+            const int e = rows <= 32 ? launch_x32_mt<1>(ctx, g, w, &ran) : launch_x32_mt<2>(ctx, g, w, &ran);
+            if (e || ran) return e;
+        }
+    }
     const size_t as = act_bytes(a_dt) * w->k, cs = act_bytes(c_dt) * w->n;
     for (uint32_t r = 0; r < rows; ++r) {
         int e = gemv_dispatch(ctx, (const uint8_t *)a + r * as, a_dt, w, (uint8_t *)c + r * cs, c_dt,

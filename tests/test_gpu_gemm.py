@@ -154,3 +154,115 @@ def test_f32_activations_keep_the_reference_dtype(engine):
         y = torch.empty(n, device=DEV)
         ops.gemm_auto(engine, a[r].contiguous(), w, y, 1, 1, k, n)
         assert torch.equal(y, c[r])
+
+
+def _check_f32_against_f64(y, wf, x, bound=1e-5):
+    x, w = x.double().cpu(), torch.from_numpy(wf).double()
+    err = (y.double().cpu() - x @ w.T).abs()
+    assert bool((err <= bound * (x.abs() @ w.abs().T) + 1e-30).all()), float((err / (x.abs() @ w.abs().T)).max())
+
+
+@pytest.mark.parametrize("ggml_type", [2, 8, 12, 13, 1])
+@pytest.mark.parametrize("rows", [3, 4, 31, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(33, 256), (200, 512), (4096, 1280), (1000, 4352)])
+def test_f32_rows_on_mfma_match_f64(engine, ggml_type, rows, n, k):
+    """binary32 activations as three exact bfloat16 parts: one and two M
+    tiles, partial row groups and K passes, K split over workgroups. The
+    parts and products are exact, so the M = 1 kernels' bound for binary32
+    sums holds (1e-5 of sum |w x|); values from 2^-40 to 2^20 keep their
+    digits, and a repeated call gives the same bits."""
+    _, w = _weight(engine, ggml_type, n, k, 700 + ggml_type + n)
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randn(rows, k, generator=g) * torch.exp2(torch.randint(-40, 21, (rows, 1), generator=g).float())
+    x[:, ::7] *= 2.0 ** -12
+    a, c, again = x.to(DEV), torch.empty(rows, n, device=DEV), torch.empty(rows, n, device=DEV)
+    ops.gemm_auto(engine, a, w, c, rows, 1, k, n)
+    ops.gemm_auto(engine, a, w, again, rows, 1, k, n)
+    assert torch.equal(c, again)
+    _check_f32_against_f64(c, w.dequant().cpu().numpy(), x)
+
+
+@pytest.mark.parametrize("ggml_type,n,k", [(2, 70, 96), (8, 70, 96), (8, 96, 160), (2, 6176, 4160), (1, 70, 1032)])
+def test_f32_rows_on_mfma_ragged_k(engine, ggml_type, n, k):
+    """K that ends inside a pass, a 64-wide chunk, or (F16) a 16-wide one."""
+    _, w = _weight(engine, ggml_type, n, k, 900 + n + k)
+    x = torch.randn(5, k, generator=torch.Generator().manual_seed(k))
+    resid = torch.randn(5, n, device=DEV)
+    base, out = torch.empty(5, n, device=DEV), resid.clone()
+    ops.gemm_auto(engine, x.to(DEV), w, base, 5, 1, k, n)
+    ops.gemm_residual(engine, x.to(DEV), w, out, out, 5)
+    assert torch.equal(out, base + resid)
+    h = torch.empty(5, n, device=DEV, dtype=torch.float16)
+    ops.gemm_auto(engine, x.to(DEV), w, h, 5, 1, k, n)
+    assert torch.equal(h, base.to(torch.float16))
+    _check_f32_against_f64(base, w.dequant().cpu().numpy(), x)
+
+
+@pytest.mark.parametrize("ggml_type", [2, 8, 12, 13, 1])
+def test_f32_rows_with_infinities_and_nan_match_single_rows(engine, ggml_type):
+    """Rows holding an infinity or a NaN: no finite value where a single call
+    gives none, the same infinity where it gives one (Q8_0's row kernel turns
+    infinities into NaN through its offset; here they stay), a NaN row all
+    NaN, and the other rows are left alone."""
+    n, k = 256, 512
+    _, w = _weight(engine, ggml_type, n, k, 31)
+    x = torch.randn(6, k, generator=torch.Generator().manual_seed(2))
+    x[1, 77] = float("inf")
+    x[2, 300] = float("-inf")
+    x[4, 5] = float("nan")
+    a, c = x.to(DEV), torch.empty(6, n, device=DEV)
+    ops.gemm_auto(engine, a, w, c, 6, 1, k, n)
+    for r in (1, 2, 4):
+        y = torch.empty(n, device=DEV)
+        ops.gemm_auto(engine, a[r].contiguous(), w, y, 1, 1, k, n)
+        assert torch.equal(y.isfinite(), c[r].isfinite())
+        assert torch.equal(y[y.isinf()], c[r][y.isinf()])
+        assert r != 4 or bool(c[r].isnan().all())
+    keep = [0, 3, 5]
+    _check_f32_against_f64(c[keep], w.dequant().cpu().numpy(), x[keep])
+
+
+def test_f32_rows_with_nonfinite_f16_weights_match_single_rows(engine):
+    """A binary16 weight with an infinity has no exact parts: such a weight
+    keeps the row kernels, bit for bit."""
+    n, k, rows = 128, 512, 7
+    rng = np.random.default_rng(6)
+    bits = synth.f16_bits(rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)).copy()
+    bits.reshape(n, k)[17, 3], bits.reshape(n, k)[40, 500] = 0x7C00, 0x7E00
+    w = ops.GpuTensor(engine, 1, n, k, bits)
+    a, c = torch.randn(rows, k, device=DEV), torch.empty(rows, n, device=DEV)
+    ops.gemm_auto(engine, a, w, c, rows, 1, k, n)
+    for r in range(rows):
+        y = torch.empty(n, device=DEV)
+        ops.gemm_auto(engine, a[r].contiguous(), w, y, 1, 1, k, n)
+        assert torch.equal(y.view(torch.int32), c[r].view(torch.int32))
+
+
+def test_f32_rows_first_used_inside_a_capture(engine):
+    """The first call on a weight may come inside a stream capture: nothing
+    can be allocated there, so the row kernels run; a later eager call builds
+    the tile copy. Both match f64, and every replay repeats its result."""
+    n, k, rows = 1000, 1024, 9
+    eng = ops.ComputeEngine(0)
+    _, w = _weight(eng, 2, n, k, 77)
+    a, c = torch.randn(rows, k, device=DEV), torch.empty(rows, n, device=DEV)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        eng.bind_stream(s)
+        ops.gemm_auto(eng, a, w, c, rows, 1, k, n)
+    eng.bind_stream(torch.cuda.current_stream())
+    eager = torch.empty(rows, n, device=DEV)
+    wf = w.dequant().cpu().numpy()
+    for _ in range(3):
+        c.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _check_f32_against_f64(c, wf, a)
+        ops.gemm_auto(eng, a, w, eager, rows, 1, k, n)
+        torch.cuda.synchronize()
+        _check_f32_against_f64(eager, wf, a)
+    del w, g
+    eng.sync()
+    eng.close()
