@@ -207,8 +207,9 @@ int embed_launch(janus_ctx *ctx, const janus_weight *table, const uint32_t *h_id
                  uint32_t batch, float *out) {
     const uint32_t hidden = table->k, vocab = table->n;
     const uint32_t gx = (hidden + 255) / 256 < 16 ? (hidden + 255) / 256 : 16;
-    for (uint32_t b0 = 0; b0 < batch; b0 += 64) {
-        uint32_t nb = batch - b0 < 64 ? batch - b0 : 64;
+    const uint32_t per = h_ids ? 64u : 32768u;   // host ids: what the kernel arguments hold
+    for (uint32_t b0 = 0; b0 < batch; b0 += per) {
+        uint32_t nb = batch - b0 < per ? batch - b0 : per;
         EmbedIds ids;
         std::memset(&ids, 0, sizeof(ids));
         if (h_ids)

@@ -179,6 +179,8 @@ int smallm_gemm_launch(janus_ctx *ctx, const void *a, int a_dt, const janus_weig
 // weight's tile copy (allocates: call outside graph capture).
 bool mfma_gemm_supported(int a_dt, const janus_weight *w);
 int mfma_gemm_prepare(janus_ctx *ctx, const janus_weight *w);
+// Frees the tile copy (nothing enqueued may still read it).
+void mfma_gemm_release(const janus_weight *w);
 
 // Split-K partials of one MFMA product: ws[ksplit][mpad][npad] (f32), and
 // beside them in the same workspace a small per-row area for the epilogues
@@ -189,13 +191,20 @@ struct GemmPartials {
     uint32_t ksplit, mpad, npad;
     float *ss;
 };
-// Batched products (binary16 rows, 1..64) whose epilogue kernel sums the
-// partials and finishes the step:
+// c = a . W^T (+ residual, which may be c) for any number of rows; above 64
+// the weight must be mfma_rows_supported.
+int gemm_rows(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, float *c, uint32_t rows,
+              const float *residual);
+// Whether the MFMA GEMM takes rows of a_dt on this weight (for F32 rows known
+// for certain once the tile copy exists).
+bool mfma_rows_supported(int a_dt, const janus_weight *w);
+// Batched products (rows of a_dt, any number; gemm_residual_norm: binary16,
+// at most 64) whose epilogue kernel sums the partials and finishes the step:
 //  gemm_qkv_rope: rows of the fused QKV weight (RoPE pairs of the q heads,
 //    of the k heads, then v) -> q rotated (f32 [rows][q_pairs * 2]), k rotated
 //    and v appended to the cache row rowbase[m] + pos[m] (kv_row elements;
 //    m * max_seq + pos[m] when rowbase is null).
-//  gemm_swiglu: interleaved gate/up rows -> act (binary16 [rows][n / 2]).
+//  gemm_swiglu: interleaved gate/up rows -> act ([rows][n / 2] of a_dt).
 //  gemm_residual_norm: out = resid + product (f32, may alias resid), then
 //    xn = RMSNorm(out) * gamma (binary16), one workgroup per row.
 struct QkvEpilogue {
@@ -206,9 +215,9 @@ struct QkvEpilogue {
     const int32_t *rowbase;   // KV row base per row (null: m * max_seq)
     uint32_t q_pairs, k_pairs, half_hd, kv_row, max_seq;
 };
-int gemm_qkv_rope(janus_ctx *ctx, const void *a16, const janus_weight *w, uint32_t rows, const QkvEpilogue &e,
+int gemm_qkv_rope(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, uint32_t rows, const QkvEpilogue &e,
                   int kv_f16);
-int gemm_swiglu(janus_ctx *ctx, const void *a16, const janus_weight *w, uint32_t rows, void *act16);
+int gemm_swiglu(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, uint32_t rows, void *act);
 bool resnorm_supported(uint32_t hidden);
 int gemm_residual_norm(janus_ctx *ctx, const void *a16, const janus_weight *w, uint32_t rows, const float *resid,
                        float *out, const float *gamma, float eps, void *xn16);

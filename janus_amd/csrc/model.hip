@@ -99,6 +99,16 @@ struct janus_model {
         int32_t token;
     } *h_stream = nullptr;
     hipEvent_t stream_ev[2] = {nullptr, nullptr};
+    // prompt chunks (prefill_chunk): activations of up to `rows` prompt tokens,
+    // allocated with the first prompt that uses them
+    struct Prefill {
+        uint32_t rows = 0;
+        bool ready = false, off = false;   // off: no memory, or a weight without the MFMA path
+        float *hidden = nullptr, *h1 = nullptr, *q = nullptr;
+        void *xn = nullptr, *att = nullptr, *act = nullptr;   // act_dtype
+        float *k = nullptr, *v = nullptr, *gate = nullptr, *up = nullptr;   // layers without the fused weights
+        int32_t *pos = nullptr, *lens = nullptr, *rowbase = nullptr;
+    } pf;
 };
 
 namespace {
@@ -367,14 +377,14 @@ int forward_batch(janus_model *m, const uint32_t *h_ids, const int32_t *d_ids, u
         void *vc = (uint8_t *)m->vcache + (size_t)l * m->layer_kv_elems * kv_elem_bytes(c.kv_dtype);
         const QkvEpilogue qe{m->q, kc, vc, m->rope, m->d_pos, m->d_rowbase, c.heads * half, c.kv_heads * half, half,
                              kvd, c.max_seq_len};
-        if ((e = gemm_qkv_rope(ctx, m->xn, L.qkv, nseq, qe, kv16))) return e;
+        if ((e = gemm_qkv_rope(ctx, m->xn, JANUS_DT_F16, L.qkv, nseq, qe, kv16))) return e;
         if ((e = attention_launch(ctx, m->q, kc, vc, c.kv_dtype, m->attn16, nseq, c.heads, c.kv_heads, c.head_dim, 0,
                                   c.max_seq_len, m->d_rowbase, m->d_lens, max_len, 1.0f / sqrtf((float)c.head_dim),
                                   1)))
             return e;
         if ((e = gemm_residual_norm(ctx, m->attn16, L.o, nseq, m->hidden, m->h1, L.ffn_norm, c.rms_eps, m->xn)))
             return e;
-        if ((e = gemm_swiglu(ctx, m->xn, L.gu, nseq, m->act))) return e;
+        if ((e = gemm_swiglu(ctx, m->xn, JANUS_DT_F16, L.gu, nseq, m->act))) return e;
         const float *next = l + 1 < c.layers ? m->layers[l + 1].attn_norm : m->out_norm;
         if ((e = gemm_residual_norm(ctx, m->act, L.down, nseq, m->h1, m->hidden, next, c.rms_eps, m->xn))) return e;
     }
@@ -590,6 +600,156 @@ struct Request {
     uint32_t n;
 };
 
+// ---- prompts in chunks ------------------------------------------------------------
+// The reference feeds a prompt token by token (generation.rs:161-173) and uses
+// none of those steps' logits. Here up to kPrefillRows prompt tokens of one
+// sequence go through the layers together as rows: their products read each
+// weight once per chunk, and each row attends its own prefix (a row's K/V is
+// in the cache before the attention of its layer runs), so the K/V rows are
+// those of the token-by-token steps up to the order of binary32 sums. The
+// output head runs with the step that follows.
+constexpr uint32_t kPrefillRows = 512;
+constexpr uint32_t kPrefillMin = 4;   // shorter prompts: as few replays of the captured step
+
+__global__ void prefill_rows_kernel(int32_t *pos, int32_t *lens, int32_t *rowbase, uint32_t p0, uint32_t n,
+                                    uint32_t base) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    pos[i] = (int32_t)(p0 + i);
+    lens[i] = (int32_t)(p0 + i + 1);
+    rowbase[i] = (int32_t)base;
+}
+
+void prefill_free(janus_model *m) {
+    janus_model::Prefill &f = m->pf;
+    for (void *p : {(void *)f.hidden, (void *)f.h1, (void *)f.q, f.xn, f.att, f.act, (void *)f.k, (void *)f.v,
+                    (void *)f.gate, (void *)f.up, (void *)f.pos, (void *)f.lens, (void *)f.rowbase})
+        if (p) (void)hipFree(p);
+    m->pf = janus_model::Prefill();
+}
+
+// Tile copies and activations for prompt chunks, once per model. False, with
+// what was allocated here given back, when a weight has no MFMA path or memory
+// is short: prompts then run token by token.
+bool prefill_ready(janus_model *m) {
+    janus_model::Prefill &f = m->pf;
+    if (f.ready || f.off) return f.ready;
+    janus_ctx *ctx = m->ctx;
+    const janus_model_config &c = m->cfg;
+    bool ok = ctx->fused_step, split = false;
+    std::vector<const janus_weight *> built;
+    for (const auto &L : m->layers) {
+        std::vector<const janus_weight *> ws{L.o, L.down};
+        if (L.qkv) ws.push_back(L.qkv);
+        else ws.insert(ws.end(), {L.q, L.k, L.v});
+        if (L.gu) ws.push_back(L.gu);
+        else ws.insert(ws.end(), {L.gate, L.up});
+        split = split || !L.qkv || !L.gu;
+        for (const janus_weight *w : ws) {
+            if (!w->t32) built.push_back(w);
+            ok = ok && mfma_gemm_supported(JANUS_DT_F16, w) && mfma_gemm_prepare(ctx, w) == JANUS_OK &&
+                 mfma_rows_supported(c.act_dtype, w);
+        }
+    }
+    const size_t R = c.max_seq_len < kPrefillRows ? c.max_seq_len : kPrefillRows, kvd = (size_t)c.kv_heads * c.head_dim;
+    const size_t ab = act_bytes(c.act_dtype);
+    auto alloc = [&](void **p, size_t bytes) { return hipMalloc(p, bytes < 256 ? 256 : bytes) == hipSuccess; };
+    ok = ok && alloc((void **)&f.hidden, R * c.hidden * 4) && alloc((void **)&f.h1, R * c.hidden * 4) &&
+         alloc((void **)&f.q, R * c.hidden * 4) && alloc(&f.xn, R * c.hidden * ab) &&
+         alloc(&f.att, R * c.hidden * ab) && alloc(&f.act, R * c.ffn * ab) && alloc((void **)&f.pos, R * 4) &&
+         alloc((void **)&f.lens, R * 4) && alloc((void **)&f.rowbase, R * 4);
+    if (split)
+        ok = ok && alloc((void **)&f.k, R * kvd * 4) && alloc((void **)&f.v, R * kvd * 4) &&
+             alloc((void **)&f.gate, R * c.ffn * 4) && alloc((void **)&f.up, R * c.ffn * 4);
+    if (!ok) {
+        (void)hipGetLastError();   // a failed allocation
+        ctx->last_error.clear();
+        for (const janus_weight *w : built) mfma_gemm_release(w);
+        prefill_free(m);
+        f.off = true;
+        return false;
+    }
+    f.rows = (uint32_t)R;
+    f.ready = true;
+    return true;
+}
+
+// n prompt tokens d_ids[0, n) of the sequence in KV slot `slot` at positions
+// p0 .. p0 + n - 1 (n <= pf.rows) through every layer: the operations and
+// order of forward_rows, without the output head.
+int prefill_chunk(janus_model *m, const int32_t *d_ids, uint32_t p0, uint32_t n, uint32_t slot) {
+    janus_ctx *ctx = m->ctx;
+    const janus_model_config &c = m->cfg;
+    const janus_model::Prefill &f = m->pf;
+    const uint32_t kvd = c.kv_heads * c.head_dim, half = c.head_dim / 2;
+    const int dt = c.act_dtype;
+    const bool a16 = dt == JANUS_DT_F16;
+    int e;
+    hipLaunchKernelGGL(prefill_rows_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, f.pos, f.lens, f.rowbase,
+                       p0, n, slot * c.max_seq_len);
+    JANUS_LAUNCH_CHECK(ctx);
+    if ((e = embed_launch(ctx, m->tok_embd, nullptr, d_ids, n, f.hidden))) return e;
+    for (uint32_t l = 0; l < c.layers; ++l) {
+        const janus_model::Layer &L = m->layers[l];
+        void *kc = (uint8_t *)m->kcache + (size_t)l * m->layer_kv_elems * kv_elem_bytes(c.kv_dtype);
+        void *vc = (uint8_t *)m->vcache + (size_t)l * m->layer_kv_elems * kv_elem_bytes(c.kv_dtype);
+        if ((e = rmsnorm_launch(ctx, f.hidden, f.xn, dt, L.attn_norm, n, c.hidden, c.rms_eps))) return e;
+        if (L.qkv) {
+            const QkvEpilogue qe{f.q, kc, vc, m->rope, f.pos, f.rowbase, c.heads * half, c.kv_heads * half, half, kvd,
+                                 c.max_seq_len};
+            if ((e = gemm_qkv_rope(ctx, f.xn, dt, L.qkv, n, qe, c.kv_dtype == JANUS_DT_F16))) return e;
+        } else {
+            if ((e = gemm_rows(ctx, f.xn, dt, L.q, f.q, n, nullptr))) return e;
+            if ((e = gemm_rows(ctx, f.xn, dt, L.k, f.k, n, nullptr))) return e;
+            if ((e = gemm_rows(ctx, f.xn, dt, L.v, f.v, n, nullptr))) return e;
+            if ((e = rope_launch(ctx, f.q, f.q, m->rope, n, c.heads, c.head_dim, 0, f.pos))) return e;
+            if ((e = rope_launch(ctx, f.k, f.k, m->rope, n, c.kv_heads, c.head_dim, 0, f.pos))) return e;
+            if ((e = kv_update_launch(ctx, f.k, f.v, kc, vc, c.kv_dtype, n, kvd, 0, c.max_seq_len, f.rowbase, f.pos)))
+                return e;
+        }
+        for (uint32_t r = 0; r < n; r += 64) {
+            const uint32_t nb = n - r < 64 ? n - r : 64;
+            void *out = (uint8_t *)f.att + (size_t)r * c.hidden * act_bytes(dt);
+            if ((e = attention_launch(ctx, f.q + (size_t)r * c.hidden, kc, vc, c.kv_dtype, out, nb, c.heads, c.kv_heads,
+                                      c.head_dim, 0, c.max_seq_len, f.rowbase + r, f.lens + r, p0 + r + nb,
+                                      1.0f / sqrtf((float)c.head_dim), a16)))
+                return e;
+        }
+        if ((e = gemm_rows(ctx, f.att, dt, L.o, f.h1, n, f.hidden))) return e;
+        if ((e = rmsnorm_launch(ctx, f.h1, f.xn, dt, L.ffn_norm, n, c.hidden, c.rms_eps))) return e;
+        if (L.gu) {
+            if ((e = gemm_swiglu(ctx, f.xn, dt, L.gu, n, f.act))) return e;
+        } else {
+            if ((e = gemm_rows(ctx, f.xn, dt, L.gate, f.gate, n, nullptr))) return e;
+            if ((e = gemm_rows(ctx, f.xn, dt, L.up, f.up, n, nullptr))) return e;
+            if ((e = elementwise_launch(ctx, EW_SWIGLU, f.gate, f.up, f.act, dt, n * c.ffn))) return e;
+        }
+        if ((e = gemm_rows(ctx, f.act, dt, L.down, f.hidden, n, f.h1))) return e;
+    }
+    return JANUS_OK;
+}
+
+// Puts the first `want` tokens of the prompt in d_prompts[slot] through the
+// layers in equal chunks. *done is `want`, or 0 when they have to run token by
+// token (a short prompt, no MFMA path, no memory).
+int prefill(janus_model *m, uint32_t slot, uint32_t want, uint32_t *done) {
+    *done = 0;
+    if (want < kPrefillMin || !prefill_ready(m)) return JANUS_OK;
+    const uint32_t chunks = (want + m->pf.rows - 1) / m->pf.rows, size = (want + chunks - 1) / chunks;
+    for (uint32_t p = 0; p < want; p += size) {
+        const uint32_t n = want - p < size ? want - p : size;
+        const int e = prefill_chunk(m, m->d_prompts + (size_t)slot * m->cfg.max_seq_len + p, p, n, slot);
+        if (e == JANUS_E_OOM) {   // a workspace could not grow: the steps rewrite what the chunks wrote
+            (void)hipGetLastError();
+            m->ctx->last_error.clear();
+            return JANUS_OK;
+        }
+        if (e) return e;
+    }
+    *done = want;
+    return JANUS_OK;
+}
+
 // The prompt checks of Model::generate (generation.rs:146-150; positions 0..n-1, :161-173).
 int check_request(janus_model *m, const Request &q) {
     const janus_model_config &c = m->cfg;
@@ -603,8 +763,9 @@ int check_request(janus_model *m, const Request &q) {
     return JANUS_OK;
 }
 
-// Puts request q into row r of `in`: its prompt copied to the device, its
-// occurrence counts cleared, its first prompt token at position 0 of KV slot r.
+// Puts request q into row r of `in`: its prompt copied to the device and put
+// through the layers in chunks where that pays, its occurrence counts cleared,
+// its next token and position in KV slot r.
 int admit_row(janus_model *m, uint32_t r, const Request &q, uint32_t max_tokens, int eos_mode, RowInit &in,
               std::vector<int32_t> &tmp) {
     janus_ctx *ctx = m->ctx;
@@ -614,8 +775,12 @@ int admit_row(janus_model *m, uint32_t r, const Request &q, uint32_t max_tokens,
                                         hipMemcpyHostToDevice, ctx->stream));
     JANUS_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));   // tmp is reused
     JANUS_HIP_CHECK(ctx, hipMemsetAsync(m->d_counts + (size_t)r * c.vocab, 0, (size_t)c.vocab * 4, ctx->stream));
-    in.token[r] = (int32_t)q.prompt[0];
-    in.pos[r] = 0;
+    // the whole prompt when a position is left for the re-fed last token (which
+    // the row then starts with), else all but the last prompt token
+    uint32_t done = 0;
+    if (int e = prefill(m, r, q.n < c.max_seq_len ? q.n : q.n - 1, &done)) return e;
+    in.token[r] = (int32_t)q.prompt[done < q.n ? done : q.n - 1];
+    in.pos[r] = (int32_t)done;
     in.rowbase[r] = (int32_t)(r * c.max_seq_len);
     in.ctl[r] = RowDev{(int32_t)q.n, (int32_t)max_tokens, 0, 0, eos_mode, 0};
     in.mask[r / 32] |= 1u << (r % 32);
@@ -656,7 +821,7 @@ int run_requests(janus_model *m, const std::vector<Request> &reqs, uint32_t max_
             parked[r] = 0;
             if (int e = admit_row(m, r, reqs[next_req++], max_tokens, eos_mode, in, tmp)) return e;
             hrows[r] = in.ctl[r];
-            hpos[r] = 0;
+            hpos[r] = in.pos[r];
             any_new = true;
         }
         uint32_t nrows = 0;
@@ -691,7 +856,7 @@ int run_requests(janus_model *m, const std::vector<Request> &reqs, uint32_t max_
             if (need < 1) need = 1;
             if ((uint64_t)need < k) k = (uint32_t)need;
         }
-        // hpos holds each row's position (admitted and parked rows start at 0)
+        // hpos holds each row's position (parked rows are at 0)
         int32_t top = 0;
         for (uint32_t r = 0; r < nrows; ++r) top = hpos[r] > top ? hpos[r] : top;
         if (int e = replay(m, nrows, k, (uint32_t)top + 1)) return e;
@@ -744,14 +909,15 @@ int run_stream(janus_model *m, const Request &q, uint32_t max_tokens, janus_toke
     if (int e = set_rows(m, in)) return e;
     // every bucket the request can reach, captured before the first step so
     // that no capture stalls the stream of tokens
+    const uint32_t done = (uint32_t)in.pos[0];   // prompt tokens already in the cache
     {
         const uint64_t reach = (uint64_t)q.n + max_tokens + 1;
-        if (int e = replay_prepare(m, 1, 1, reach < m->cfg.max_seq_len ? (uint32_t)reach : m->cfg.max_seq_len))
+        if (int e = replay_prepare(m, 1, done + 1, reach < m->cfg.max_seq_len ? (uint32_t)reach : m->cfg.max_seq_len))
             return e;
     }
-    // prefill: positions 0 .. n-1; the last of these steps queues the re-fed
-    // last prompt token at position n (or ends the row at max_seq_len)
-    if (int e = replay(m, 1, q.n, 1)) return e;
+    // the rest of the prompt, up to position n-1; the last of these steps queues
+    // the re-fed last prompt token at position n (or ends the row at max_seq_len)
+    if (int e = replay(m, 1, q.n - done, done + 1)) return e;
     // step i samples token i (the step at position n + i at most); at most
     // max_tokens steps can sample one
     auto issue = [&](uint32_t i) -> int {
@@ -884,6 +1050,7 @@ void janus_model_destroy(janus_model *m) {
     for (hipEvent_t ev : m->stream_ev)
         if (ev) (void)hipEventDestroy(ev);
     if (m->h_stream) (void)hipHostFree(m->h_stream);
+    prefill_free(m);
     for (auto &L : m->layers) {
         for (janus_weight *w : {L.q, L.k, L.v, L.o, L.gate, L.up, L.down, L.qkv, L.gu}) janus_weight_free(m->ctx, w);
         (void)hipFree(L.attn_norm);
@@ -933,6 +1100,7 @@ int janus_model_set_tensor(janus_model *m, const char *cname, int type, uint32_t
     free_graphs(m);
     m->fused_ready = false;
     m->tiles_ready = false;
+    prefill_free(m);   // the new tensor may change whether prompts run in chunks
     for (auto &L : m->layers) {
         janus_weight_free(ctx, L.qkv);
         janus_weight_free(ctx, L.gu);
@@ -1078,8 +1246,19 @@ int janus_model_generate(janus_model *m, const uint32_t *prompt, uint32_t n_prom
     m->h_sampler.mode = std::fabs(penalty - 1.0f) < 0.01f ? SAMPLE_WGSL : SAMPLE_PENALTY;
     m->h_sampler.penalty = penalty;
     if (max_tokens == 0) {
-        // prefill only (generation.rs:161-173), then a loop of zero steps
-        for (uint32_t i = 0; i < n_prompt; ++i)
+        // prefill only (generation.rs:161-173), then a loop of zero steps; the
+        // last token's step leaves its logits
+        uint32_t done = 0;
+        if (n_prompt > kPrefillMin && janus_model_validate(m) == JANUS_OK &&
+            check_request(m, Request{prompt, n_prompt}) == JANUS_OK) {
+            std::vector<int32_t> ids(prompt, prompt + n_prompt);
+            JANUS_HIP_CHECK(m->ctx, hipMemcpyAsync(m->d_prompts, ids.data(), (size_t)n_prompt * 4, hipMemcpyHostToDevice,
+                                                   m->ctx->stream));
+            JANUS_HIP_CHECK(m->ctx, hipStreamSynchronize(m->ctx->stream));   // ids goes out of scope
+            m->graph_nseq = 0;   // d_prompts no longer holds a running loop's prompt
+            if (int e = prefill(m, 0, n_prompt - 1, &done)) return e;
+        }
+        for (uint32_t i = done; i < n_prompt; ++i)
             if (int e = janus_model_forward(m, &prompt[i], &i, 1)) return e;
         return upload_sampler(m);
     }

@@ -272,11 +272,12 @@ struct GemmArgs {
     uint32_t passes_per_wg;
     uint32_t total_passes;
     uint32_t ksplit;
+    uint32_t tiles, mtiles;   // gemm_pipe_kernel: weight tiles of 32 NW rows, M tiles of 32 MT rows
     uint32_t pitch;        // LDS row pitch of A, in halves
     int c_f16;
     int to_ws;             // write partials to ws even when ksplit == 1 (epilogue kernels read them)
     uint32_t seg_shift;    // log2 of the 8-half A segments per row of a pass (pass length / 8)
-    int swiglu;            // ksplit == 1 only: rows (2j, 2j+1) are (gate_j, up_j); c = silu(gate)*up, binary16 [rows][n/2]
+    int swiglu;            // ksplit == 1 only: rows (2j, 2j+1) are (gate_j, up_j); c = silu(gate)*up [rows][n/2]
 };
 
 // ---- formats ------------------------------------------------------------------
@@ -291,13 +292,46 @@ template <int MT> struct Deferred {
     float d;      // and its scale (0 before the first block)
 };
 
-// acc += the pending block's scaled results; t with scale d becomes pending.
+// Keeps the arithmetic on a result tile where it is written: without it the
+// compiler sinks the scale FMAs of a whole pass behind its MFMAs, and the
+// block results held for them spill.
 template <int MT>
+__device__ __forceinline__ void pin(f16x (&acc)[MT]) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[mt]));
+}
+
+// PIN keeps the arithmetic on a result tile where it is written. In the
+// branch-free passes of the wide kernel the compiler otherwise sinks the scale
+// FMAs of a whole pass behind its MFMAs and spills the block results held for
+// them (28672x4096 at 512 rows: 1.8 ms against 0.17).
+template <int MT, bool PIN>
+__device__ __forceinline__ void pin(f16x (&acc)[MT]) {
+    if constexpr (PIN)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[mt]));
+}
+
+// acc += the pending block's scaled results; t with scale d becomes pending
+// (from three M tiles on t is applied at once: the tiles' MFMAs cover each
+// other's latency, and a second set of results does not fit the registers).
+template <int MT, bool PIN = false>
 __device__ __forceinline__ void apply_deferred(f16x (&acc)[MT], Deferred<MT> &pend, const f16x (&t)[MT], float d) {
+    if constexpr (MT >= 3) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(d, t[mt][v], acc[mt][v]);
+        pin<MT>(acc);
+        pin<MT, PIN>(acc);
+        return;
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
+    pin<MT>(acc);
+    pin<MT, PIN>(acc);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) pend.t[mt] = t[mt];
     pend.d = d;
@@ -312,7 +346,7 @@ struct GQ4_0 {
     // One chunk on binary32 activations: As holds their three bfloat16 parts
     // (`plane` halves apart). The offset -8 enters as the first accumulator,
     // -8 * sum(x) of the block, so the weights stay the integers 0..15.
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t, int lane, const float *Ss, f16x (&acc)[MT], Deferred<MT> &pend) {
         const int h = lane >> 5, r = lane & 31;
@@ -325,7 +359,7 @@ struct GQ4_0 {
             for (int mt = 0; mt < MT; ++mt)
                 t[mt] = block_b<true>(As + (size_t)(mt * 32 + r) * pitch + kl + b * 32 + 8 * h, plane, b0, b1,
                                 tile_rows(Ss + (size_t)(kl / 32 + b) * (MT * 32) + mt * 32, h));
-            apply_deferred<MT>(acc, pend, t, h2f((uint16_t)(b ? (w.s >> 16) : (w.s & 0xffffu))));
+            apply_deferred<MT, PIN>(acc, pend, t, h2f((uint16_t)(b ? (w.s >> 16) : (w.s & 0xffffu))));
         }
     }
     // g and c are wavefront-uniform: the chunk base is scalar, the lane adds
@@ -337,7 +371,7 @@ struct GQ4_0 {
         w.s = *(const uint32_t *)(a.side + ch * 128 + (uint32_t)(lane & 31) * 4u);
         return w;
     }
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma_deferred(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                         f16x (&acc)[MT], Deferred<MT> &pend) {
         const int h = lane >> 5, r = lane & 31;
@@ -354,16 +388,10 @@ struct GQ4_0 {
                 t[mt] = mfma(lds_h8(ap), b0, (f16x){});
                 t[mt] = mfma(lds_h8(ap + 16), b1, t[mt]);
             }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) pend.t[mt] = t[mt];
-            pend.d = d;
+            apply_deferred<MT, PIN>(acc, pend, t, d);
         }
     }
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *, uint32_t, f16x (&acc)[MT]) {
         const int h = lane >> 5, r = lane & 31;
@@ -391,7 +419,7 @@ struct GQ8_0 {
     static constexpr float XSUM = 0.0f;   // no sums
     struct W { uint4 q; uint16_t s; };
     // see GQ4_0::mma_x32
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t, int lane, const float *, f16x (&acc)[MT], Deferred<MT> &pend) {
         const int h = lane >> 5, r = lane & 31;
@@ -400,7 +428,7 @@ struct GQ8_0 {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
             t[mt] = block_b<false>(As + (size_t)(mt * 32 + r) * pitch + kl + 8 * h, plane, b0, b1, (f16x){});
-        apply_deferred<MT>(acc, pend, t, h2f_q8(w.s));
+        apply_deferred<MT, PIN>(acc, pend, t, h2f_q8(w.s));
     }
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
         const size_t ch = (size_t)g * a.chunks + c;
@@ -409,7 +437,7 @@ struct GQ8_0 {
         w.s = ((const uint16_t *)a.side)[ch * 32 + (lane & 31)];
         return w;
     }
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *, uint32_t, f16x (&acc)[MT]) {
         const int h = lane >> 5, r = lane & 31;
@@ -424,6 +452,7 @@ struct GQ8_0 {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(d, t[v], acc[mt][v]);
         }
+        pin<MT>(acc);
     }
 };
 
@@ -439,7 +468,7 @@ struct GQ4_K {
     // values q - 8 and ds * (q . x) - dm * sum(x) = ds * t + (dm - 8 ds) / 8 * staged:
     // the two large terms of a block mostly cancel before they are rounded.
     // c: chunk of the row group.
-    template <int MT, class G = GQ4_K>
+    template <int MT, bool PIN = false, class G = GQ4_K>
     __device__ static void mma_x32(const typename G::W &w, const _Float16 *As, uint32_t plane, uint32_t pitch,
                                    uint32_t kl, uint32_t c, int lane, const float *Ss, f16x (&acc)[MT],
                                    Deferred<MT> &) {
@@ -462,6 +491,8 @@ struct GQ4_K {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(cs, s[v], fmaf(ds, t[v], acc[mt][v]));
             }
+            pin<MT, PIN>(acc);
+            pin<MT>(acc);
         }
     }
     __device__ static void unpack_b(const W &w, int b, b8 &b0, b8 &b1) {
@@ -482,13 +513,13 @@ struct GQ4_K {
         sc = (float)((g >> o) & 63u);
         mn = (float)((g >> (12u + o)) & 63u);
     }
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
-                               const float *Ss, uint32_t sub0, f16x (&acc)[MT]) {
+                               const float *Ss, uint32_t chunk0, f16x (&acc)[MT]) {
         const int h = lane >> 5, r = lane & 31;
         const uint32_t q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
         const float d = h2f((uint16_t)(w.hdr.x & 0xffffu)), dmin = h2f((uint16_t)(w.hdr.x >> 16));
-        const int j = (int)((kl / 64 + sub0 / 2) & 3);   // chunk index within the super-block
+        const int j = (int)((kl / 64 + chunk0) & 3);   // chunk index within the super-block (chunk0: the pass's first)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             float sc, mn;
@@ -512,6 +543,8 @@ struct GQ4_K {
                     acc[mt][4 * jj + 3] = fmaf(-dm, s4.w, fmaf(ds, t[4 * jj + 3], acc[mt][4 * jj + 3]));
                 }
             }
+            pin<MT, PIN>(acc);
+            pin<MT>(acc);
         }
     }
 };
@@ -524,10 +557,10 @@ struct GQ5_K {
     static constexpr bool ORDER4 = true;
     static constexpr float XSUM = -16.0f;
     struct W { uint4 q; uint4 hdr; uint32_t fifth; };
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t c, int lane, const float *Ss, f16x (&acc)[MT], Deferred<MT> &pend) {
-        GQ4_K::mma_x32<MT, GQ5_K>(w, As, plane, pitch, kl, c, lane, Ss, acc, pend);
+        GQ4_K::mma_x32<MT, PIN, GQ5_K>(w, As, plane, pitch, kl, c, lane, Ss, acc, pend);
     }
     __device__ static void unpack_b(const W &w, int b, b8 &b0, b8 &b1) {
         b0 = b ? unpack_nib8_q5_b<2>(w.q.z, w.fifth) : unpack_nib8_q5_b<0>(w.q.x, w.fifth);
@@ -542,12 +575,12 @@ struct GQ5_K {
         w.hdr = *(const uint4 *)(a.side + (sb * 32 + (lane & 31)) * 16);
         return w;
     }
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
-                               const float *Ss, uint32_t sub0, f16x (&acc)[MT]) {
+                               const float *Ss, uint32_t chunk0, f16x (&acc)[MT]) {
         const int h = lane >> 5, r = lane & 31;
         const float d = h2f((uint16_t)(w.hdr.x & 0xffffu)), dmin = h2f((uint16_t)(w.hdr.x >> 16));
-        const int j = (int)((kl / 64 + sub0 / 2) & 3);   // chunk index within the super-block
+        const int j = (int)((kl / 64 + chunk0) & 3);   // chunk index within the super-block (chunk0: the pass's first)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             float sc, mn;
@@ -571,6 +604,8 @@ struct GQ5_K {
                     acc[mt][4 * jj + 3] = fmaf(-dm, s4.w, fmaf(ds, t[4 * jj + 3], acc[mt][4 * jj + 3]));
                 }
             }
+            pin<MT, PIN>(acc);
+            pin<MT>(acc);
         }
     }
 };
@@ -602,7 +637,7 @@ struct GF16 {
     // the five small ones (below 2^-7 of it) to pend.t, added at the end, so
     // their roundings stay at their own size. inf: an activation may be
     // infinite; it then meets only the leading weight part (the other may be 0).
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t inf, int lane, const float *, f16x (&acc)[MT], Deferred<MT> &pend) {
         const int h = lane >> 5, r = lane & 31;
@@ -626,7 +661,7 @@ struct GF16 {
         w.q = ld_stream(a.qs + (ch * 64 + lane) * 16);
         return w;
     }
-    template <int MT>
+    template <int MT, bool PIN = false>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *, uint32_t, f16x (&acc)[MT]) {
         const int h = lane >> 5, r = lane & 31;
@@ -646,14 +681,14 @@ __device__ __forceinline__ uint32_t out_row(int mt, int v, int lane) {
 }
 
 template <int MT>
-__device__ __forceinline__ void store_tile(const GemmArgs &a, uint32_t g, int lane, const f16x (&acc)[MT]) {
+__device__ __forceinline__ void store_tile(const GemmArgs &a, uint32_t g, uint32_t m0, int lane, const f16x (&acc)[MT]) {
     const uint32_t n = g * 32 + (lane & 31);
     if (n >= a.n) return;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const uint32_t m = out_row(mt, v, lane);
+            const uint32_t m = m0 + out_row(mt, v, lane);
             if (m < a.rows) {
                 float val = acc[mt][v];
                 const size_t at = (size_t)m * a.n + n;
@@ -665,10 +700,11 @@ __device__ __forceinline__ void store_tile(const GemmArgs &a, uint32_t g, int la
 }
 
 // SwiGLU store of a finished tile: columns 2j, 2j+1 (lanes l, l^1) hold gate_j
-// and up_j of the same rows; the even lane writes silu(gate) * up as binary16
-// (the arithmetic of elementwise_kernel's SwiGLU).
+// and up_j of the same rows; the even lane writes silu(gate) * up (the
+// arithmetic of elementwise_kernel's SwiGLU).
 template <int MT>
-__device__ __forceinline__ void store_swiglu(const GemmArgs &a, uint32_t g, int lane, const f16x (&acc)[MT]) {
+__device__ __forceinline__ void store_swiglu(const GemmArgs &a, uint32_t g, uint32_t m0, int lane,
+                                             const f16x (&acc)[MT]) {
     const uint32_t n = g * 32 + (lane & 31);
     const uint32_t half = a.n / 2;
 #pragma unroll
@@ -677,10 +713,11 @@ __device__ __forceinline__ void store_swiglu(const GemmArgs &a, uint32_t g, int 
         for (int v = 0; v < 16; ++v) {
             const float mine = acc[mt][v];
             const float other = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(mine), 0xb1, 0xf, 0xf, false));
-            const uint32_t m = out_row(mt, v, lane);
+            const uint32_t m = m0 + out_row(mt, v, lane);
             if (!(lane & 1) && m < a.rows && n + 1 < a.n) {
                 const float act = mine * (1.0f / (1.0f + expf(-mine))) * other;
-                ((uint16_t *)a.c)[(size_t)m * half + n / 2] = f2h_bits(act);
+                if (a.c_f16) ((uint16_t *)a.c)[(size_t)m * half + n / 2] = f2h_bits(act);
+                else ((float *)a.c)[(size_t)m * half + n / 2] = act;
             }
         }
 }
@@ -802,8 +839,8 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_mfma_kernel(GemmArgs a) 
     }
     if (kw != 0 || !active) return;
     if (a.ksplit == 1 && !a.to_ws) {
-        if (a.swiglu) store_swiglu<MT>(a, g, lane, acc);
-        else store_tile<MT>(a, g, lane, acc);
+        if (a.swiglu) store_swiglu<MT>(a, g, 0, lane, acc);
+        else store_tile<MT>(a, g, 0, lane, acc);
         return;
     }
     // split-K: this split's tile goes to the workspace; gemm_reduce_kernel adds
@@ -826,7 +863,6 @@ constexpr uint32_t pipe_buf() {
     return (abytes + (sums ? (uint32_t)(KR / 32) * MT * 32 * 4 : flag ? 4u : 0u) + 15u) / 16u * 16u;
 }
 
-// Sums the split-K partials in split order and applies the epilogue.
 // Cross-pass pipelined form of gemm_mfma_kernel (quantised and F16 weights),
 // with the pass length KR fixed at compile time. A is double-buffered in LDS:
 // the activations of pass p + 1 are requested while pass p computes and are
@@ -834,16 +870,18 @@ constexpr uint32_t pipe_buf() {
 // registers and requests chunk i of the next pass as soon as chunk i of the
 // current one is consumed, so a pass's weights are in flight during the
 // previous pass and the barrier between them. One barrier per pass (two for
-// Q4_K, whose activation sums are built from the staged pass). Products,
+// the K-quants at most 64 binary16 rows, whose activation sums are built from
+// the staged pass; elsewhere they come from the lanes that stage a block).
+// Workgroup: NW row groups x KW K slices of a pass. Products,
 // scale rounding, slice order and outputs are those of gemm_mfma_kernel.
 // X32: binary32 activations, split into three bfloat16 parts as they are
-// stored to LDS (three planes per buffer); their per-block sums come from the
-// staging lanes themselves, so there is no separate pass over the stage.
-template <class F, int MT, int KW, int KR, bool X32>
-__global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) {
+// stored to LDS (three planes per buffer).
+template <class F, int MT, int KW, int KR, bool X32, int NW = WAVES>
+__global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
+    constexpr bool WIDE = KW == 1;   // the form for more than 64 rows
     constexpr bool SUMS = NeedsSums<F>::value && !X32;
-    constexpr int NT = 64 * WAVES * KW;   // threads
+    constexpr int NT = 64 * NW * KW;   // threads
     constexpr int PC = KR / F::CK;        // chunks per pass
     constexpr int CPW = PC / KW;          // chunks per wavefront per pass
     constexpr int MP = MT * 32;           // padded rows
@@ -857,9 +895,19 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
     constexpr bool FLAG = X32 && std::is_same<F, GF16>::value;   // one word per buffer after the activations
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar chunk bases
-    const int rgw = wave % WAVES, kw = wave / WAVES;
+    const int rgw = wave % NW, kw = wave / NW;
     const uint32_t G = (a.n + 31) / 32;
-    const uint32_t g = blockIdx.x * WAVES + rgw, ks = blockIdx.y;
+    // Workgroup -> (weight tile, M tile). With several M tiles, those of one
+    // weight tile are consecutive on one XCD (workgroup ids go round the 8
+    // XCDs), so they share the tile's weights in that XCD's L2.
+    uint32_t tile = blockIdx.x, mtile = 0;
+    if (a.mtiles > 1) {
+        const uint32_t local = blockIdx.x >> 3;
+        tile = (local / a.mtiles) * 8 + (blockIdx.x & 7u);
+        mtile = local % a.mtiles;
+        if (tile >= a.tiles) return;
+    }
+    const uint32_t g = tile * NW + rgw, ks = blockIdx.y, m0 = mtile * MP;
     const bool active = g < G;
     const uint32_t p_begin = ks * a.passes_per_wg;
     const uint32_t p_end = min(a.total_passes, p_begin + a.passes_per_wg);
@@ -871,6 +919,12 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) pend.t[mt] = (f16x){};
     pend.d = 0.0f;
+    // X32: 256 of K are summed on their own (part) and then added to acc, so
+    // the sum over K takes one long rounding per 256 and not one per block
+    f16x part[MT];
+    if constexpr (X32)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) part[mt] = (f16x){};
     typename F::W w[CPW];
     uint4 sv[SPT * (X32 ? 2 : 1)];
 
@@ -884,7 +938,7 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
 #pragma unroll
         for (int i = 0; i < SPT; ++i) {
             const uint32_t s = threadIdx.x + NT * i;
-            const uint32_t m = min(s / SEGS, a.rows - 1), col = min(kbase + (s % SEGS) * 8, a.k - 8);
+            const uint32_t m = min(m0 + s / SEGS, a.rows - 1), col = min(kbase + (s % SEGS) * 8, a.k - 8);
             if constexpr (X32) {
                 const uint4 *p = (const uint4 *)(a.a32 + (size_t)m * a.k + col);
                 sv[2 * i] = p[0];
@@ -894,13 +948,21 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
             }
         }
     };
+    // the sum t of segment s joins those of its 32-element block (the four
+    // lanes of a quad) in the stage's [sub-block][row] sums
+    auto put_sum = [&](uint32_t p, uint32_t s, float t) {
+        t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0xb1, 0xf, 0xf, false));
+        t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x4e, 0xf, 0xf, false));
+        float *Ss = (float *)(smem + (p & 1) * BUF + ABYTES);
+        if (!(threadIdx.x & 3)) Ss[(s % SEGS) / 4 * MP + s / SEGS] = t;
+    };
     auto store_a = [&](uint32_t p) {
         _Float16 *As = (_Float16 *)(smem + (p & 1) * BUF);
         const uint32_t kbase = p * KR;
 #pragma unroll
         for (int i = 0; i < SPT; ++i) {
             const uint32_t s = threadIdx.x + NT * i;
-            const bool ok = s / SEGS < a.rows && kbase + (s % SEGS) * 8 < a.k;
+            const bool ok = m0 + s / SEGS < a.rows && kbase + (s % SEGS) * 8 < a.k;
             if constexpr (X32) {
                 const uint4 lo = sv[2 * i], hi = sv[2 * i + 1];
                 const uint32_t u[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
@@ -913,20 +975,22 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
                 _Float16 *at = As + (s / SEGS) * PITCH + (s % SEGS) * 8;
 #pragma unroll
                 for (int j = 0; j < 3; ++j) *(uint4 *)(at + j * PLANE) = part[j];
-                if constexpr (F::XSUM != 0.0f) {
-                    // the four lanes of a quad hold one 32-element block
-                    float t = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
-                    t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0xb1, 0xf, 0xf, false));
-                    t += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x4e, 0xf, 0xf, false));
-                    float *Ss = (float *)(smem + (p & 1) * BUF + ABYTES);
-                    if (!(threadIdx.x & 3)) Ss[(s % SEGS) / 4 * MP + s / SEGS] = F::XSUM * t;
-                }
+                if constexpr (F::XSUM != 0.0f)
+                    put_sum(p, s, F::XSUM * (((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]))));
                 continue;
             }
-            *(uint4 *)(As + (s / SEGS) * PITCH + (s % SEGS) * 8) = ok ? sv[i] : make_uint4(0u, 0u, 0u, 0u);
+            const uint4 v = ok ? sv[i] : make_uint4(0u, 0u, 0u, 0u);
+            *(uint4 *)(As + (s / SEGS) * PITCH + (s % SEGS) * 8) = v;
+            if constexpr (SUMS && WIDE) {
+                const h8 x = __builtin_bit_cast(h8, v);
+                const float t = (((float)x[0] + (float)x[1]) + ((float)x[2] + (float)x[3])) +
+                                (((float)x[4] + (float)x[5]) + ((float)x[6] + (float)x[7]));
+                put_sum(p, s, t);
+            }
         }
     };
-    // Q4_K: per-(sub-block, row) sums of the staged activations, as gemm_mfma_kernel
+    // the sums of a staged pass, by a pass over it (with two M tiles the lanes'
+    // own sums cost the registers that let two workgroups share a CU)
     auto sums = [&](uint32_t p) {
         const _Float16 *As = (const _Float16 *)(smem + (p & 1) * BUF);
         float *Ss = (float *)(smem + (p & 1) * BUF + ABYTES);
@@ -939,6 +1003,7 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
             for (int j = 0; j < 32; ++j) t += (float)p8[j];
             Ss[i] = t;
         }
+        __syncthreads();
     };
     // chunk i of this wavefront's slice of pass p (K-tail slots repeat the
     // pass's last chunk and are not computed)
@@ -950,33 +1015,35 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
     auto pass = [&](uint32_t p, auto load_next) {
         const _Float16 *As = (const _Float16 *)(smem + (p & 1) * BUF);
         const float *Ss = (const float *)(smem + (p & 1) * BUF + ABYTES);
-        const uint32_t c1 = min(a.chunks, (p + 1) * PC), m0 = p * PC + kw * CPW;
-        // X32: a pass is summed on its own and then added, so the sum over K
-        // takes one long rounding per pass and not one per block
-        f16x part[MT];
-        if constexpr (X32)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) part[mt] = (f16x){};
+        const uint32_t c1 = min(a.chunks, (p + 1) * PC), cw = p * PC + kw * CPW;
         // F16: Ss is the flag of an infinite activation in the staged passes
         const uint32_t inf = X32 && FLAG ? __builtin_amdgcn_readfirstlane(*(const uint32_t *)Ss) : 0u;
 #pragma unroll
         for (int i = 0; i < CPW; ++i) {
-            if (m0 + i < c1) {
+            // Only the last pass can end before its last chunk. The wide form
+            // takes the others without a branch (a branch per chunk costs it a
+            // register copy of every result tile where the paths meet); with
+            // one or two M tiles the branches keep the chunks' order for less.
+            if ((WIDE && decltype(load_next)::value) || cw + i < c1) {
                 if constexpr (X32)
-                    F::template mma_x32<MT>(w[i], As, PLANE, PITCH, (uint32_t)(kw * CPW + i) * F::CK,
-                                            FLAG ? inf : m0 + i, lane, Ss, part, pend);
+                    F::template mma_x32<MT, WIDE>(w[i], As, PLANE, PITCH, (uint32_t)(kw * CPW + i) * F::CK,
+                                            FLAG ? inf : cw + i, lane, Ss, part, pend);
                 else if constexpr (Defers<F>::value)
-                    F::template mma_deferred<MT>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, acc, pend);
+                    F::template mma_deferred<MT, WIDE>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, acc, pend);
                 else
-                    F::template mma<MT>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, Ss, 0, acc);
+                    F::template mma<MT, WIDE>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, Ss, p * PC, acc);
             }
             if (decltype(load_next)::value) w[i] = F::load(a, gl, chunk_of(p + 1, i), lane);
+            if constexpr (WIDE) __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (X32)
+            if (KR >= 256 || ((p - p_begin) & 1u) || !decltype(load_next)::value)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
+                for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[mt][v] += part[mt][v];
+                    for (int v = 0; v < 16; ++v) acc[mt][v] += part[mt][v];
+                    part[mt] = (f16x){};
+                }
     };
 
     if (p_begin < p_end) {
@@ -991,19 +1058,13 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
         store_a(p_begin);
         load_a(min(p_begin + 1, last));
         __syncthreads();
-        if (SUMS) {
-            sums(p_begin);
-            __syncthreads();
-        }
+        if constexpr (SUMS && !WIDE) sums(p_begin);
         for (uint32_t p = p_begin; p < last; ++p) {
             pass(p, std::true_type{});
             store_a(p + 1);   // that buffer was last read in pass p - 1
             load_a(min(p + 2, last));
             __syncthreads();
-            if (SUMS) {
-                sums(p + 1);
-                __syncthreads();
-            }
+            if constexpr (SUMS && !WIDE) sums(p + 1);
         }
         pass(last, std::false_type{});
     }
@@ -1022,7 +1083,7 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
                     float sum = red[((size_t)rgw * 16 + v) * 64 + lane];
-                    for (int j = 1; j < KW; ++j) sum += red[((size_t)(j * WAVES + rgw) * 16 + v) * 64 + lane];
+                    for (int j = 1; j < KW; ++j) sum += red[((size_t)(j * NW + rgw) * 16 + v) * 64 + lane];
                     acc[mt][v] = sum;
                 }
             }
@@ -1030,8 +1091,8 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
     }
     if (kw != 0 || !active) return;
     if (a.ksplit == 1 && !a.to_ws) {
-        if (a.swiglu) store_swiglu<MT>(a, g, lane, acc);
-        else store_tile<MT>(a, g, lane, acc);
+        if (a.swiglu) store_swiglu<MT>(a, g, m0, lane, acc);
+        else store_tile<MT>(a, g, m0, lane, acc);
         return;
     }
     const uint32_t Npad = G * 32, n = g * 32 + (lane & 31);
@@ -1039,30 +1100,30 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_pipe_kernel(GemmArgs a) 
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-            __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * MP + out_row(mt, v, lane)) * Npad + n);
+            __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * MP * a.mtiles + m0 + out_row(mt, v, lane)) * Npad + n);
 }
 
 // LDS bytes of gemm_pipe_kernel: two staging buffers, at least the K-slice
 // reduction area.
-template <class F, int MT, int KW, int KR, bool X32>
+template <class F, int MT, int KW, int KR, bool X32, int NW>
 constexpr size_t pipe_lds() {
     constexpr size_t buf = pipe_buf<F, MT, KR, X32>();
-    constexpr size_t red = (size_t)WAVES * KW * 16 * 64 * 4;
+    constexpr size_t red = (size_t)NW * KW * 16 * 64 * 4;
     static_assert(2 * buf <= 160 * 1024 && red <= 160 * 1024, "LDS");
     return 2 * buf > red ? 2 * buf : red;
 }
 
-template <class F, int MT, int KW, int KR, bool X32 = false>
+template <class F, int MT, int KW, int KR, bool X32 = false, int NW = WAVES>
 void launch_pipe(janus_ctx *ctx, dim3 grid, const GemmArgs &a) {
     // thread-safe one-time set-up (a function-local static's initialiser)
     static const bool attr_set = [] {
-        (void)hipFuncSetAttribute((const void *)gemm_pipe_kernel<F, MT, KW, KR, X32>,
+        (void)hipFuncSetAttribute((const void *)gemm_pipe_kernel<F, MT, KW, KR, X32, NW>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         return true;
     }();
     (void)attr_set;
-    constexpr size_t lds = pipe_lds<F, MT, KW, KR, X32>();
-    hipLaunchKernelGGL((gemm_pipe_kernel<F, MT, KW, KR, X32>), grid, dim3(64 * WAVES * KW), lds, ctx->stream, a);
+    constexpr size_t lds = pipe_lds<F, MT, KW, KR, X32, NW>();
+    hipLaunchKernelGGL((gemm_pipe_kernel<F, MT, KW, KR, X32, NW>), grid, dim3(64 * NW * KW), lds, ctx->stream, a);
 }
 
 // Sums the split-K partials in split order and applies the epilogue.
@@ -1297,6 +1358,13 @@ constexpr int gemm_kw() {
     return (MT == 1 && std::is_same<F, GF16>::value) ? 4 : 2;
 }
 
+int launch_reduce(janus_ctx *ctx, const GemmArgs &a, uint32_t mpad) {
+    const size_t total = (size_t)a.rows * a.n;
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, a, mpad);
+    JANUS_LAUNCH_CHECK(ctx);
+    return JANUS_OK;
+}
+
 // kr_force / ks_force (0 = automatic) fix the pass length and the K split.
 template <class F, int MT, int KW = gemm_kw<F, MT>(), int PD = Stage<F>::PD>
 int launch_mfma(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials *parts, uint32_t kr_force = 0,
@@ -1394,12 +1462,7 @@ int launch_mfma(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials 
         parts->ss = a.ws + need / 4;
         return JANUS_OK;
     }
-    if (a.ksplit > 1) {
-        const size_t total = (size_t)a.rows * w->n;
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, a,
-                           (uint32_t)(MT * 32));
-        JANUS_LAUNCH_CHECK(ctx);
-    }
+    if (a.ksplit > 1) return launch_reduce(ctx, a, MT * 32);
     return JANUS_OK;
 }
 
@@ -1451,14 +1514,16 @@ bool capturing(const janus_ctx *ctx) {
     return hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
 }
 
-// Binary32 rows on the MFMA kernel. *ran stays false, with nothing launched
-// and no error, when the workspace cannot grow (out of memory, or inside a
-// capture): the caller then runs one GEMV per row, which needs none.
+// Binary32 rows (at most 64) on the MFMA kernel. *ran stays false, with nothing
+// launched and no error, when the workspace cannot grow (out of memory, or
+// inside a capture): the caller then runs one GEMV per row, which needs none.
 template <class F, int MT, int KW = gemm_kw<F, MT>()>
-int launch_x32(janus_ctx *ctx, GemmArgs a, const janus_weight *w, bool *ran) {
+int launch_x32(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials *parts, bool *ran) {
     constexpr int KR = MT == 1 ? 256 : 128;
     dim3 grid;
-    const size_t need = plan_x32<F, MT, KR>(ctx, a, w, grid);
+    size_t need = plan_x32<F, MT, KR>(ctx, a, w, grid);
+    const uint32_t npad = (w->n + 31) / 32 * 32;
+    if (parts) need = (size_t)a.ksplit * MT * 32 * npad * 4;
     if (need > ctx->gemm_ws_bytes) {
         if (capturing(ctx)) return JANUS_OK;
         if (ensure_gemm_ws(ctx, need)) {
@@ -1468,26 +1533,89 @@ int launch_x32(janus_ctx *ctx, GemmArgs a, const janus_weight *w, bool *ran) {
         }
     }
     a.ws = (float *)ctx->gemm_ws;
+    a.to_ws = parts != nullptr;
     *ran = true;
     launch_pipe<F, MT, KW, KR, true>(ctx, grid, a);
     JANUS_LAUNCH_CHECK(ctx);
-    if (a.ksplit > 1) {
-        const size_t total = (size_t)a.rows * w->n;
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, a,
-                           (uint32_t)(MT * 32));
-        JANUS_LAUNCH_CHECK(ctx);
+    if (parts) {
+        *parts = GemmPartials{a.ws, a.ksplit, MT * 32, npad, nullptr};
+        return JANUS_OK;
     }
+    if (a.ksplit > 1) return launch_reduce(ctx, a, MT * 32);
     return JANUS_OK;
 }
 
 template <int MT>
-int launch_x32_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, bool *ran) {
+int launch_x32_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, GemmPartials *parts, bool *ran) {
     switch (w->type) {
-    case JANUS_DT_Q4_0: return launch_x32<GQ4_0, MT>(ctx, a, w, ran);
-    case JANUS_DT_Q8_0: return launch_x32<GQ8_0, MT>(ctx, a, w, ran);
-    case JANUS_DT_Q4_K: return launch_x32<GQ4_K, MT>(ctx, a, w, ran);
-    case JANUS_DT_Q5_K: return launch_x32<GQ5_K, MT>(ctx, a, w, ran);
-    default: return launch_x32<GF16, MT>(ctx, a, w, ran);
+    case JANUS_DT_Q4_0: return launch_x32<GQ4_0, MT>(ctx, a, w, parts, ran);
+    case JANUS_DT_Q8_0: return launch_x32<GQ8_0, MT>(ctx, a, w, parts, ran);
+    case JANUS_DT_Q4_K: return launch_x32<GQ4_K, MT>(ctx, a, w, parts, ran);
+    case JANUS_DT_Q5_K: return launch_x32<GQ5_K, MT>(ctx, a, w, parts, ran);
+    default: return launch_x32<GF16, MT>(ctx, a, w, parts, ran);
+    }
+}
+
+// ---- more than 64 rows (prompts) -----------------------------------------------
+// gemm_pipe_kernel over M tiles of 32 MT rows with 8 row groups per workgroup
+// (256 weight rows) and no K slices: a staged activation tile serves all 8
+// wavefronts, and a weight chunk is unpacked once for MT MFMA pairs. MT = 4
+// for binary16 rows (2 x 35 KB of LDS), 2 for three bfloat16 parts (2 x 52 KB).
+// Bound by the VALU (one scale FMA per weight and 32 rows, 0.4 more to unpack)
+// on binary16 rows and by LDS reads of the parts on binary32 rows. Q4_0
+// 28672x4096 at 512 rows: 167 us (721 TFLOP/s) against 229 with 4 row groups
+// x 2 K slices and 186 with MT = 2; binary32 rows 411 us (875 TFLOP/s of
+// MFMA) against 464, and 556 with MT = 3. A product with too few tiles for
+// the CUs splits K over workgroups.
+constexpr int kWideKR = 128, kWideNW = 8;
+
+template <class F, int MT, bool X32>
+int launch_wide_mt(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials *parts) {
+    const uint32_t G = (w->n + 31) / 32;
+    a.tiles = (G + kWideNW - 1) / kWideNW;
+    a.mtiles = (a.rows + 32 * MT - 1) / (32 * MT);
+    a.chunks = w->t32_chunks;
+    a.pass_chunks = kWideKR / F::CK;
+    a.total_passes = (a.chunks + a.pass_chunks - 1) / a.pass_chunks;
+    const uint64_t wgs = (uint64_t)a.tiles * a.mtiles;
+    uint64_t ks = a.swiglu ? 1 : (uint64_t)ctx->num_cus / wgs;
+    if (ks > a.total_passes / 4) ks = a.total_passes / 4;
+    if (ks < 1) ks = 1;
+    a.passes_per_wg = (a.total_passes + (uint32_t)ks - 1) / (uint32_t)ks;
+    a.ksplit = (a.total_passes + a.passes_per_wg - 1) / a.passes_per_wg;
+    const uint32_t mpad = a.mtiles * MT * 32;
+    a.to_ws = parts != nullptr;
+    if (a.ksplit > 1 || parts) {
+        if (int e = ensure_gemm_ws(ctx, (size_t)a.ksplit * mpad * G * 32 * 4)) return e;
+        a.ws = (float *)ctx->gemm_ws;
+    }
+    const uint32_t gx = a.mtiles > 1 ? (a.tiles + 7) / 8 * 8 * a.mtiles : a.tiles;
+    launch_pipe<F, MT, 1, kWideKR, X32, kWideNW>(ctx, dim3(gx, a.ksplit), a);
+    JANUS_LAUNCH_CHECK(ctx);
+    if (parts) {
+        *parts = GemmPartials{a.ws, a.ksplit, mpad, G * 32, nullptr};
+        return JANUS_OK;
+    }
+    if (a.ksplit > 1) return launch_reduce(ctx, a, mpad);
+    return JANUS_OK;
+}
+
+template <class F>
+int launch_wide(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, GemmPartials *parts) {
+    if (a.a32) return launch_wide_mt<F, 2, true>(ctx, a, w, parts);
+    // the M tile with the least padded work (per workgroup, unpacking and
+    // staging cost about what 0.7 of an M subtile does)
+    auto cost = [&](uint32_t mt) { return (float)((a.rows + 32 * mt - 1) / (32 * mt)) * ((float)mt + 0.7f); };
+    return cost(4) <= cost(3) ? launch_wide_mt<F, 4, false>(ctx, a, w, parts) : launch_wide_mt<F, 3, false>(ctx, a, w, parts);
+}
+
+int launch_wide_any(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, GemmPartials *parts) {
+    switch (w->type) {
+    case JANUS_DT_Q4_0: return launch_wide<GQ4_0>(ctx, a, w, parts);
+    case JANUS_DT_Q8_0: return launch_wide<GQ8_0>(ctx, a, w, parts);
+    case JANUS_DT_Q4_K: return launch_wide<GQ4_K>(ctx, a, w, parts);
+    case JANUS_DT_Q5_K: return launch_wide<GQ5_K>(ctx, a, w, parts);
+    default: return launch_wide<GF16>(ctx, a, w, parts);
     }
 }
 
@@ -1504,6 +1632,7 @@ GemmArgs make_args(const janus_weight *w, const void *a, void *c, int c_f16, uin
     g.n = w->n;
     g.k = w->k;
     g.c_f16 = c_f16;
+    g.mtiles = 1;
     return g;
 }
 
@@ -1566,15 +1695,16 @@ __global__ __launch_bounds__(256) void epi_qkv_rope_kernel(GemmPartials p, QkvEp
     }
 }
 
-// Gate/up rows interleaved (gate_j, up_j): act[m][j] = silu(gate) * up as
-// binary16 (the SwiGLU of elementwise_kernel).
-__global__ __launch_bounds__(256) void epi_swiglu_kernel(GemmPartials p, _Float16 *act, uint32_t rows, uint32_t ffn) {
+// Gate/up rows interleaved (gate_j, up_j): act[m][j] = silu(gate) * up (the
+// SwiGLU of elementwise_kernel).
+template <typename T>
+__global__ __launch_bounds__(256) void epi_swiglu_kernel(GemmPartials p, T *act, uint32_t rows, uint32_t ffn) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (size_t)rows * ffn) return;
     const uint32_t m = (uint32_t)(idx / ffn), j = (uint32_t)(idx % ffn);
     const jf2 r = sum_pair(p, m, 2 * j);
     const float v = r.x * (1.0f / (1.0f + expf(-r.x))) * r.y;
-    ((uint16_t *)act)[idx] = f2h_bits(v);
+    act[idx] = (T)v;
 }
 
 // One 1024-thread workgroup per row: out[m] = resid[m] + product (f32, may
@@ -1678,13 +1808,21 @@ __global__ __launch_bounds__(128) void epi_norm_kernel(GemmPartials p, const flo
     }
 }
 
-int run_partials(janus_ctx *ctx, const void *a, const janus_weight *w, uint32_t rows, GemmPartials *parts) {
+int run_partials(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, uint32_t rows, GemmPartials *parts) {
     if (!mfma_gemm_supported(JANUS_DT_F16, w))
         return fail(ctx, JANUS_E_UNSUPPORTED_DTYPE, "batched epilogue: weight has no MFMA path");
-    if (rows == 0 || rows > 64) return fail(ctx, JANUS_E_INVALID_DIM, "batched epilogue: rows must be 1..64");
+    if (rows == 0) return fail(ctx, JANUS_E_INVALID_DIM, "batched epilogue: no rows");
     if (int e = mfma_gemm_prepare(ctx, w)) return e;
-    const GemmArgs g = make_args(w, a, nullptr, 0, rows, nullptr);
-    return rows <= 32 ? launch_mt<1>(ctx, g, w, parts) : launch_mt<2>(ctx, g, w, parts);
+    GemmArgs g = make_args(w, a_dt == JANUS_DT_F16 ? a : nullptr, nullptr, 0, rows, nullptr);
+    if (a_dt == JANUS_DT_F16)
+        return rows <= 32 ? launch_mt<1>(ctx, g, w, parts)
+               : rows <= 64 ? launch_mt<2>(ctx, g, w, parts) : launch_wide_any(ctx, g, w, parts);
+    if (w->t32_nonfinite) return fail(ctx, JANUS_E_UNSUPPORTED_DTYPE, "batched epilogue: weight has no exact parts");
+    g.a32 = (const float *)a;
+    if (rows > 64) return launch_wide_any(ctx, g, w, parts);
+    bool ran = false;
+    const int e = rows <= 32 ? launch_x32_mt<1>(ctx, g, w, parts, &ran) : launch_x32_mt<2>(ctx, g, w, parts, &ran);
+    return e || ran ? e : fail(ctx, JANUS_E_OOM, "batched epilogue: workspace");
 }
 
 }  // namespace
@@ -1697,6 +1835,16 @@ bool mfma_gemm_supported(int a_dt, const janus_weight *w) {
 
 int mfma_gemm_prepare(janus_ctx *ctx, const janus_weight *w) {
     return t32_ensure(ctx, const_cast<janus_weight *>(w));
+}
+
+void mfma_gemm_release(const janus_weight *cw) {
+    janus_weight *w = const_cast<janus_weight *>(cw);
+    if (w->t32) (void)hipFree(w->t32);
+    w->t32 = nullptr;
+    w->t32_qs = w->t32_side = nullptr;
+    w->t32_q5h = nullptr;
+    w->t32_chunks = 0;
+    w->t32_nonfinite = false;
 }
 
 int smallm_gemm_launch(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, void *c, int c_dt,
@@ -1723,7 +1871,8 @@ int smallm_gemm_launch(janus_ctx *ctx, const void *a, int a_dt, const janus_weig
             GemmArgs g = make_args(w, nullptr, c, c_dt == JANUS_DT_F16, rows, residual);
             g.a32 = (const float *)a;
             bool ran = false;
-            const int e = rows <= 32 ? launch_x32_mt<1>(ctx, g, w, &ran) : launch_x32_mt<2>(ctx, g, w, &ran);
+            const int e = rows <= 32 ? launch_x32_mt<1>(ctx, g, w, nullptr, &ran)
+                                     : launch_x32_mt<2>(ctx, g, w, nullptr, &ran);
             if (e || ran) return e;
         }
     }
@@ -1736,12 +1885,26 @@ int smallm_gemm_launch(janus_ctx *ctx, const void *a, int a_dt, const janus_weig
     return JANUS_OK;
 }
 
-int gemm_qkv_rope(janus_ctx *ctx, const void *a16, const janus_weight *w, uint32_t rows, const QkvEpilogue &e,
+int gemm_rows(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, float *c, uint32_t rows,
+              const float *residual) {
+    if (rows <= 64) return gemm_dispatch(ctx, a, a_dt, w, c, JANUS_DT_F32, rows, residual);
+    if (!mfma_rows_supported(a_dt, w)) return fail(ctx, JANUS_E_UNSUPPORTED_DTYPE, "gemm: weight has no MFMA path");
+    if (int e = mfma_gemm_prepare(ctx, w)) return e;
+    GemmArgs g = make_args(w, a_dt == JANUS_DT_F16 ? a : nullptr, c, 0, rows, residual);
+    if (a_dt == JANUS_DT_F32) g.a32 = (const float *)a;
+    return launch_wide_any(ctx, g, w, nullptr);
+}
+
+bool mfma_rows_supported(int a_dt, const janus_weight *w) {
+    return mfma_gemm_supported(JANUS_DT_F16, w) && !(a_dt == JANUS_DT_F32 && w->t32_nonfinite);
+}
+
+int gemm_qkv_rope(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, uint32_t rows, const QkvEpilogue &e,
                   int kv_f16) {
     if (w->n != 2 * (e.q_pairs + e.k_pairs) + e.kv_row || e.kv_row % 2)
         return fail(ctx, JANUS_E_INVALID_DIM, "qkv epilogue: row count does not match the head layout");
     GemmPartials p{};
-    if (int r = run_partials(ctx, a16, w, rows, &p)) return r;
+    if (int r = run_partials(ctx, a, a_dt, w, rows, &p)) return r;
     const size_t total = (size_t)rows * (w->n / 2);
     const dim3 grid((unsigned)((total + 255) / 256));
     if (kv_f16) hipLaunchKernelGGL(epi_qkv_rope_kernel<_Float16>, grid, dim3(256), 0, ctx->stream, p, e, rows);
@@ -1750,22 +1913,32 @@ int gemm_qkv_rope(janus_ctx *ctx, const void *a16, const janus_weight *w, uint32
     return JANUS_OK;
 }
 
-int gemm_swiglu(janus_ctx *ctx, const void *a16, const janus_weight *w, uint32_t rows, void *act16) {
+int gemm_swiglu(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, uint32_t rows, void *act) {
     if (w->n % 2) return fail(ctx, JANUS_E_INVALID_DIM, "swiglu epilogue: odd row count");
     const uint32_t tiles = (w->n + 32 * WAVES - 1) / (32 * WAVES);
-    if (w->type == JANUS_DT_Q4_0 && rows <= 32 && 4 * tiles >= 3 * (uint32_t)ctx->num_cus) {
+    const bool f16 = a_dt == JANUS_DT_F16;
+    if (rows > 64 && mfma_rows_supported(a_dt, w)) {
+        // K unsplit: SwiGLU is applied to the finished tile
+        if (int e = mfma_gemm_prepare(ctx, w)) return e;
+        GemmArgs g = make_args(w, f16 ? a : nullptr, act, f16, rows, nullptr);
+        if (!f16) g.a32 = (const float *)a;
+        g.swiglu = 1;
+        return launch_wide_any(ctx, g, w, nullptr);
+    }
+    if (f16 && w->type == JANUS_DT_Q4_0 && rows <= 32 && 4 * tiles >= 3 * (uint32_t)ctx->num_cus) {
         // enough row tiles for every CU without splitting K: 16-wavefront
         // workgroups over the whole K, SwiGLU applied to the finished tile
         if (int e = mfma_gemm_prepare(ctx, w)) return e;
-        GemmArgs g = make_args(w, a16, act16, 1, rows, nullptr);
+        GemmArgs g = make_args(w, a, act, 1, rows, nullptr);
         g.swiglu = 1;
         return launch_mfma<GQ4_0, 1, 4, 2>(ctx, g, w, nullptr, ctx->gemm_pipe ? 512 : 1024, 1);
     }
     GemmPartials p{};
-    if (int r = run_partials(ctx, a16, w, rows, &p)) return r;
+    if (int r = run_partials(ctx, a, a_dt, w, rows, &p)) return r;
     const size_t total = (size_t)rows * (w->n / 2);
-    hipLaunchKernelGGL(epi_swiglu_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, p,
-                       (_Float16 *)act16, rows, w->n / 2);
+    const dim3 grid((unsigned)((total + 255) / 256));
+    if (f16) hipLaunchKernelGGL(epi_swiglu_kernel<_Float16>, grid, dim3(256), 0, ctx->stream, p, (_Float16 *)act, rows, w->n / 2);
+    else hipLaunchKernelGGL(epi_swiglu_kernel<float>, grid, dim3(256), 0, ctx->stream, p, (float *)act, rows, w->n / 2);
     JANUS_LAUNCH_CHECK(ctx);
     return JANUS_OK;
 }
@@ -1778,7 +1951,8 @@ int gemm_residual_norm(janus_ctx *ctx, const void *a16, const janus_weight *w, u
     if (!resnorm_supported(hidden))
         return fail(ctx, JANUS_E_INVALID_DIM, "residual-norm epilogue: rows must be a multiple of 4, at most 8192");
     GemmPartials p{};
-    if (int r = run_partials(ctx, a16, w, rows, &p)) return r;
+    if (rows > 64) return fail(ctx, JANUS_E_INVALID_DIM, "residual-norm epilogue: at most 64 rows");
+    if (int r = run_partials(ctx, a16, JANUS_DT_F16, w, rows, &p)) return r;
     _Float16 *xn = (_Float16 *)xn16;
     if (ctx->epi_split) {
         const dim3 sgrid((hidden + kEpiCols - 1) / kEpiCols, rows), sblock(kEpiCols / 4);

@@ -391,3 +391,84 @@ def test_captured_steps_cross_length_buckets(monkeypatch):
         for got in (gen, stream, batch[0]):
             assert_same_or_near_tie(got, want_pen, lg_pen, 1.15)
         assert_same_or_near_tie(batch[1], want_short, lg_short, 1.15)
+
+
+def _prompt_model(kind):
+    if kind == "mixed":   # q/k/v and gate/up of different types: no fused weights
+        s = synth.make_model(61, 512, 4, 2, 768, 700, 2, synth.Q4_K, 1e-5, 500000.0,
+                             embed_type=synth.F16, head_type=synth.F16, down_type=synth.Q5_K)
+        rng = np.random.default_rng(62)
+        for t in s.tensors:
+            if t.name.endswith("attn_v.weight") or t.name.endswith("ffn_up.weight"):
+                t.ggml_type, t.data = synth.Q8_0, synth.random_q8_0(rng, t.n, t.k)
+        return s
+    return synth.make_model(63, 512, 4, 1, 1024, 700, 2, kind, 1e-5, 500000.0, embed_type=synth.F16,
+                            head_type=synth.F16)
+
+
+@pytest.mark.parametrize("act", [_lib.DT_F32, _lib.DT_F16])
+@pytest.mark.parametrize("kind", [synth.Q4_0, synth.Q8_0, synth.Q4_K, synth.Q5_K, synth.F16, "mixed"])
+def test_prompt_chunks_match_token_by_token(engine, act, kind):
+    """A prompt's K/V rows and the logits of the step after it, through the
+    chunked prompt path, against eager single-token steps: the shortest chunk,
+    one and two small M tiles, one wide tile with a ragged edge (66, 97, 130
+    rows), and two chunks (600). Binary32 activations differ only in the order
+    of binary32 sums; with binary16 ones a sum on a rounding edge moves a
+    stored value by one ulp (2^-11), which the next layer carries on."""
+    s = _prompt_model(kind)
+    n_max = 610
+    shape = (2, n_max, s.kv_heads, 128)
+    dt = torch.float16 if act == _lib.DT_F16 else torch.float32
+
+    def model():
+        m = Model(engine, s, max_seq_len=n_max, kv_dtype=act, act_dtype=act)
+        kv = [torch.zeros(shape, dtype=dt, device=DEV) for _ in range(2)]
+        m.set_kv_cache(*kv)
+        return m, kv
+
+    prompt = _prompt(64, 600, s.vocab)
+    ref, rkv = model()
+    want = {}
+    for p, t in enumerate(prompt):
+        if p in (4, 33, 66, 97, 130):
+            keep = [x[:, p].clone() for x in rkv]
+            ref.forward([prompt[p - 1]], [p])   # generate's re-fed last token
+            want[p] = ref.logits()[0]
+            for x, y in zip(rkv, keep):
+                x[:, p] = y
+        ref.forward([t], [p])
+    ref.forward([prompt[-1]], [600])
+    want[600] = ref.logits()[0]
+    ref.close()
+    tol = 1e-5 if act == _lib.DT_F32 else 2e-3
+    m, kv = model()
+    for n, lg in want.items():
+        for x in kv:
+            x.zero_()
+        m.generate(prompt[:n], 1)
+        assert _rel_err(m.logits()[0], lg) <= tol, n
+        for x, r in zip(kv, rkv):
+            d, r = x[:, :n].double() - r[:, :n].double(), r[:, :n].double()
+            assert float(d.norm() / r.norm()) <= tol, n
+            assert float(d.abs().max() / r.abs().max()) <= 4 * tol, n
+            assert not x[:, n + 1:].any()
+    m.close()
+
+
+def test_prompt_chunks_at_capacity_and_in_every_loop(engine):
+    """generate, generate_with_callback and generate_batch agree on prompts
+    that run in chunks; a prompt of max_seq_len - 1 leaves one token, one of
+    max_seq_len none; max_tokens 0 leaves the last prompt token's logits."""
+    s = _prompt_model(synth.Q4_0)
+    m = Model(engine, s, max_seq_len=80, max_batch=3)
+    prompts = [_prompt(70 + n, n, s.vocab) for n in (79, 80, 5, 41, 66)]
+    alone = [m.generate(p, 6) for p in prompts]
+    assert [len(a) for a in alone] == [1, 0, 6, 6, 6]
+    assert [m.generate_with_callback(p, 6) for p in prompts] == alone
+    assert m.generate_batch(prompts, 6) == alone
+    m.generate(prompts[3], 0)
+    got = m.logits()[0]
+    for p, t in enumerate(prompts[3]):
+        m.forward([t], [p])
+    assert _rel_err(got, m.logits()[0]) <= 1e-5
+    m.close()
