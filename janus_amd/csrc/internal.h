@@ -249,6 +249,14 @@ int attention_launch(janus_ctx *ctx, const float *q, const void *kc, const void 
                      uint32_t batch, uint32_t heads, uint32_t kv_heads, uint32_t hd, uint32_t seq_len,
                      uint32_t max_seq, const int32_t *row_base, const int32_t *seq_lens, uint32_t max_len,
                      float scale, int out_f16 = 0, float *fixed_ws = nullptr, size_t fixed_ws_bytes = 0);
+// Causal attention of n prompt rows at positions p0 .. p0 + n - 1 of one
+// sequence (prefill.hip): q [n][heads][hd] f32, kc / vc the sequence's cache
+// rows from position 0 on, row i over positions 0 .. p0 + i; out as
+// attention_launch. Allocates nothing.
+bool prefill_attention_supported(uint32_t hd);
+int prefill_attention_launch(janus_ctx *ctx, const float *q, const void *kc, const void *vc, int kv_dt, void *out,
+                             uint32_t n, uint32_t p0, uint32_t heads, uint32_t kv_heads, uint32_t hd, float scale,
+                             int out_f16);
 // Looks up, once per device, the device address of the fixed attention
 // scratch (kAttnScratchBytes) and stores it in ctx->attn_scratch. Called by
 // janus_create with the context's device current.

@@ -107,7 +107,7 @@ struct janus_model {
         float *hidden = nullptr, *h1 = nullptr, *q = nullptr;
         void *xn = nullptr, *att = nullptr, *act = nullptr;   // act_dtype
         float *k = nullptr, *v = nullptr, *gate = nullptr, *up = nullptr;   // layers without the fused weights
-        int32_t *pos = nullptr, *lens = nullptr, *rowbase = nullptr;
+        int32_t *pos = nullptr, *rowbase = nullptr;
     } pf;
 };
 
@@ -611,19 +611,17 @@ struct Request {
 constexpr uint32_t kPrefillRows = 512;
 constexpr uint32_t kPrefillMin = 4;   // shorter prompts: as few replays of the captured step
 
-__global__ void prefill_rows_kernel(int32_t *pos, int32_t *lens, int32_t *rowbase, uint32_t p0, uint32_t n,
-                                    uint32_t base) {
+__global__ void prefill_rows_kernel(int32_t *pos, int32_t *rowbase, uint32_t p0, uint32_t n, uint32_t base) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     pos[i] = (int32_t)(p0 + i);
-    lens[i] = (int32_t)(p0 + i + 1);
     rowbase[i] = (int32_t)base;
 }
 
 void prefill_free(janus_model *m) {
     janus_model::Prefill &f = m->pf;
     for (void *p : {(void *)f.hidden, (void *)f.h1, (void *)f.q, f.xn, f.att, f.act, (void *)f.k, (void *)f.v,
-                    (void *)f.gate, (void *)f.up, (void *)f.pos, (void *)f.lens, (void *)f.rowbase})
+                    (void *)f.gate, (void *)f.up, (void *)f.pos, (void *)f.rowbase})
         if (p) (void)hipFree(p);
     m->pf = janus_model::Prefill();
 }
@@ -636,7 +634,7 @@ bool prefill_ready(janus_model *m) {
     if (f.ready || f.off) return f.ready;
     janus_ctx *ctx = m->ctx;
     const janus_model_config &c = m->cfg;
-    bool ok = ctx->fused_step, split = false;
+    bool ok = ctx->fused_step && prefill_attention_supported(c.head_dim), split = false;
     std::vector<const janus_weight *> built;
     for (const auto &L : m->layers) {
         std::vector<const janus_weight *> ws{L.o, L.down};
@@ -657,7 +655,7 @@ bool prefill_ready(janus_model *m) {
     ok = ok && alloc((void **)&f.hidden, R * c.hidden * 4) && alloc((void **)&f.h1, R * c.hidden * 4) &&
          alloc((void **)&f.q, R * c.hidden * 4) && alloc(&f.xn, R * c.hidden * ab) &&
          alloc(&f.att, R * c.hidden * ab) && alloc(&f.act, R * c.ffn * ab) && alloc((void **)&f.pos, R * 4) &&
-         alloc((void **)&f.lens, R * 4) && alloc((void **)&f.rowbase, R * 4);
+         alloc((void **)&f.rowbase, R * 4);
     if (split)
         ok = ok && alloc((void **)&f.k, R * kvd * 4) && alloc((void **)&f.v, R * kvd * 4) &&
              alloc((void **)&f.gate, R * c.ffn * 4) && alloc((void **)&f.up, R * c.ffn * 4);
@@ -685,8 +683,8 @@ int prefill_chunk(janus_model *m, const int32_t *d_ids, uint32_t p0, uint32_t n,
     const int dt = c.act_dtype;
     const bool a16 = dt == JANUS_DT_F16;
     int e;
-    hipLaunchKernelGGL(prefill_rows_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, f.pos, f.lens, f.rowbase,
-                       p0, n, slot * c.max_seq_len);
+    hipLaunchKernelGGL(prefill_rows_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, f.pos, f.rowbase, p0, n,
+                       slot * c.max_seq_len);
     JANUS_LAUNCH_CHECK(ctx);
     if ((e = embed_launch(ctx, m->tok_embd, nullptr, d_ids, n, f.hidden))) return e;
     for (uint32_t l = 0; l < c.layers; ++l) {
@@ -707,14 +705,11 @@ int prefill_chunk(janus_model *m, const int32_t *d_ids, uint32_t p0, uint32_t n,
             if ((e = kv_update_launch(ctx, f.k, f.v, kc, vc, c.kv_dtype, n, kvd, 0, c.max_seq_len, f.rowbase, f.pos)))
                 return e;
         }
-        for (uint32_t r = 0; r < n; r += 64) {
-            const uint32_t nb = n - r < 64 ? n - r : 64;
-            void *out = (uint8_t *)f.att + (size_t)r * c.hidden * act_bytes(dt);
-            if ((e = attention_launch(ctx, f.q + (size_t)r * c.hidden, kc, vc, c.kv_dtype, out, nb, c.heads, c.kv_heads,
-                                      c.head_dim, 0, c.max_seq_len, f.rowbase + r, f.lens + r, p0 + r + nb,
-                                      1.0f / sqrtf((float)c.head_dim), a16)))
-                return e;
-        }
+        const size_t base = (size_t)slot * c.max_seq_len * kvd * kv_elem_bytes(c.kv_dtype);
+        if ((e = prefill_attention_launch(ctx, f.q, (const uint8_t *)kc + base, (const uint8_t *)vc + base, c.kv_dtype,
+                                          f.att, n, p0, c.heads, c.kv_heads, c.head_dim,
+                                          1.0f / sqrtf((float)c.head_dim), a16)))
+            return e;
         if ((e = gemm_rows(ctx, f.att, dt, L.o, f.h1, n, f.hidden))) return e;
         if ((e = rmsnorm_launch(ctx, f.h1, f.xn, dt, L.ffn_norm, n, c.hidden, c.rms_eps))) return e;
         if (L.gu) {

@@ -1,0 +1,337 @@
+// prefill.hip -- causal attention of a prompt chunk.
+//
+// The rows of a chunk are consecutive positions p0 .. p0 + n - 1 of one
+// sequence whose K/V rows 0 .. p0 + n - 1 are in the cache; row i attends
+// positions 0 .. p0 + i (shaders/attention.wgsl:62-186 for each row). The
+// decode kernels would read the whole prefix once per row; here a wavefront
+// holds 32 query rows of one head, and K and V tiles of 32 positions pass
+// through LDS once for the four wavefronts of a workgroup: four heads of a KV
+// head where it has that many, else two heads x two row tiles or four row tiles.
+//
+// Scores are S^T = K Q^T (positions x queries), so a lane's column is one
+// query and the running maximum and sum, the rescale and the output scale
+// are per lane; the probabilities are P.V's B operand as they lie, with the
+// position order of V's operand chosen to match.
+//  * binary16 caches: v_mfma_f32_32x32x16_f16. q is split into binary16
+//    hi + mid + lo parts after a power-of-two prescale (33 bits, as in
+//    MfmaAttn), P into hi + lo parts of 2^14 p (22 bits, as in
+//    attn_rows_kernel); V is transposed on its way into LDS.
+//  * binary32 caches: v_mfma_f32_32x32x2_f32, nothing split or rounded.
+#include <type_traits>
+
+#include "internal.h"
+
+namespace janus {
+namespace {
+
+typedef _Float16 ph8 __attribute__((ext_vector_type(8)));
+typedef float pf16 __attribute__((ext_vector_type(16)));
+
+constexpr int QT = 32, PT = 32;   // queries per wavefront, positions per tile
+
+struct PrefillArgs {
+    const float *q;        // [n][heads][D]
+    const void *kc, *vc;   // the sequence's cache rows of one layer: [pos][kv_heads][D]
+    void *out;             // [n][heads][D], f32 or binary16
+    uint32_t n, p0, heads, kv_heads;
+    float scale2;          // scale * log2(e)
+    int out_f16;
+};
+
+__device__ __forceinline__ float swap32(float v) {   // value of lane ^ 32
+    const uint32_t u = __float_as_uint(v);
+    auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __uint_as_float((__lane_id() & 32) ? p[0] : p[1]);
+}
+
+// LDS of one K/V tile. binary16: K rows padded to D + 8 halves; V transposed,
+// [dim][position] rows padded to PT + 4 halves (8-byte reads of 4 positions).
+// binary32: K rows padded to D + 4 floats, V rows as they are.
+template <typename KV, int D> struct Tile;
+template <int D> struct Tile<_Float16, D> {
+    static constexpr int KP = D + 8, VP = PT + 4;
+    static constexpr uint32_t K = PT * KP * 2, BYTES = K + D * VP * 2;
+    static constexpr int SEG = 8;   // elements of a 16-byte segment
+};
+template <int D> struct Tile<float, D> {
+    static constexpr int KP = D + 4, VP = D;
+    static constexpr uint32_t K = PT * KP * 4, BYTES = K + PT * VP * 4;
+    static constexpr int SEG = 4;
+};
+
+// HW: heads of a KV head that a workgroup's wavefronts take (1, 2 or 4); the
+// other factor of 4 is row tiles.
+template <typename KV, int D, int HW>
+__global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
+    constexpr bool F16 = std::is_same<KV, _Float16>::value;
+    typedef Tile<KV, D> T;
+    constexpr int SEG = T::SEG, SROW = D / SEG;       // 16-byte segments per row
+    constexpr int LD = PT * SROW / 256;               // K (and V) segments per thread
+    static_assert(LD >= 1 && LD * 256 == PT * SROW, "tile load");
+    constexpr int ND = D / 32;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 31, h = lane >> 5;
+    const uint32_t G = a.heads / a.kv_heads;
+    const uint32_t parts = G / HW, kvh = blockIdx.y / parts;
+    const uint32_t head = kvh * G + (blockIdx.y % parts) * HW + wave % HW;
+    // row tiles from the last (longest) to the first
+    const uint32_t groups = gridDim.x, grp = groups - 1 - blockIdx.x;
+    constexpr uint32_t TW = 4 / HW;   // row tiles per workgroup
+    const uint32_t q0 = (grp * TW + wave / HW) * QT;   // may lie beyond n: such a wavefront only helps to load
+    const uint32_t last_row = min(a.n, (grp + 1) * TW * QT) - 1;
+    const uint32_t end_all = a.p0 + last_row + 1;      // positions the workgroup passes over
+    const uint32_t kvrow = a.kv_heads * D;
+    const KV *kc = (const KV *)a.kc + (size_t)kvh * D, *vc = (const KV *)a.vc + (size_t)kvh * D;
+
+    ju4 kr[LD], vr[LD];
+    // segment j of this thread: binary16 V goes to LDS transposed in pairs of
+    // positions, so a thread takes two rows of the same dims
+    auto row_of = [&](int j, bool v) -> uint32_t {
+        const uint32_t s = threadIdx.x + 256u * j;
+        if (F16 && v) return LD >= 2 ? (threadIdx.x / SROW) * 2 + j : threadIdx.x / SROW;
+        return s / SROW;
+    };
+    auto seg_of = [&](int j, bool v) -> uint32_t {
+        const uint32_t s = threadIdx.x + 256u * j;
+        if (F16 && v) return threadIdx.x % SROW;
+        return s % SROW;
+    };
+    auto load = [&](uint32_t p) {
+#pragma unroll
+        for (int j = 0; j < LD; ++j) {
+            const uint32_t kp = min(p + row_of(j, false), end_all - 1), vp = min(p + row_of(j, true), end_all - 1);
+            kr[j] = *(const ju4 *)(kc + (size_t)kp * kvrow + seg_of(j, false) * SEG);
+            vr[j] = *(const ju4 *)(vc + (size_t)vp * kvrow + seg_of(j, true) * SEG);
+        }
+    };
+    auto store = [&](unsigned char *t) {
+#pragma unroll
+        for (int j = 0; j < LD; ++j)
+            *(ju4 *)(t + ((size_t)row_of(j, false) * T::KP + seg_of(j, false) * SEG) * sizeof(KV)) = kr[j];
+        if constexpr (!F16) {
+#pragma unroll
+            for (int j = 0; j < LD; ++j)
+                *(ju4 *)(t + T::K + ((size_t)row_of(j, true) * T::VP + seg_of(j, true) * SEG) * 4) = vr[j];
+        } else if constexpr (LD == 2) {
+            // rows r, r + 1 of dims 8 s .. 8 s + 7: one word per dim
+            uint32_t *vt = (uint32_t *)(t + T::K);
+            const ju4 a0 = vr[0], a1 = vr[LD - 1];
+            const uint32_t d0 = seg_of(0, true) * 8, r2 = row_of(0, true) / 2;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                vt[(d0 + 2 * i) * (T::VP / 2) + r2] = __builtin_amdgcn_perm(a1[i], a0[i], 0x05040100u);
+                vt[(d0 + 2 * i + 1) * (T::VP / 2) + r2] = __builtin_amdgcn_perm(a1[i], a0[i], 0x07060302u);
+            }
+        } else {   // D = 64: one row per thread
+            uint16_t *vt = (uint16_t *)(t + T::K);
+            const ju4 a0 = vr[0];
+            const uint32_t d0 = seg_of(0, true) * 8, r = row_of(0, true);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                vt[(d0 + 2 * i) * T::VP + r] = (uint16_t)(a0[i] & 0xffffu);
+                vt[(d0 + 2 * i + 1) * T::VP + r] = (uint16_t)(a0[i] >> 16);
+            }
+        }
+    };
+    load(0);
+
+    // q of this lane's query: binary16 caches: dims 16 s + 8 h + 0..7 of each
+    // 16-wide step as three parts; binary32: dims 8 s + 4 h + 0..3
+    const uint32_t qi = min(q0 + col, a.n - 1);
+    const float *qp = a.q + ((size_t)qi * a.heads + head) * D;
+    float sc2 = a.scale2;
+    ph8 qh[F16 ? D / 16 : 1], qm[F16 ? D / 16 : 1], ql[F16 ? D / 16 : 1];
+    jf4 qf[F16 ? 1 : D / 8];
+    if constexpr (F16) {
+        float qmax = 0.0f;
+#pragma unroll
+        for (int s = 0; s < D / 16; ++s) {
+            const jf4 x0 = *(const jf4 *)(qp + 16 * s + 8 * h), x1 = *(const jf4 *)(qp + 16 * s + 8 * h + 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) qmax = fmaxf(qmax, fmaxf(fabsf(x0[i]), fabsf(x1[i])));
+        }
+        qmax = fmaxf(qmax, swap32(qmax));
+        int qe = 0;
+        (void)frexpf(qmax, &qe);                  // qmax < 2^qe
+        const int sh = qe > 15 ? qe - 15 : 0;     // |q| 2^-sh < 2^15
+        const float qs = ldexpf(1.0f, -sh);
+        sc2 *= ldexpf(1.0f, sh);
+        asm volatile("" : "+v"(qp));   // q is read again (from cache) rather than held beside its parts
+#pragma unroll
+        for (int s = 0; s < D / 16; ++s) {
+            const jf4 x0 = *(const jf4 *)(qp + 16 * s + 8 * h), x1 = *(const jf4 *)(qp + 16 * s + 8 * h + 4);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float x = (i < 4 ? x0[i & 3] : x1[i & 3]) * qs;
+                const _Float16 hi = (_Float16)x;
+                const float r = x - (float)hi;
+                const _Float16 mid = (_Float16)r;
+                qh[s][i] = hi;
+                qm[s][i] = mid;
+                ql[s][i] = (_Float16)(r - (float)mid);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < D / 8; ++s) qf[s] = *(const jf4 *)(qp + 8 * s + 4 * h);
+    }
+
+    pf16 o[ND];   // O^T: dims 32 d + 8 j + 4 h + i of query col (binary16 caches: times 2^14)
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d] = (pf16){};
+    float m = -INFINITY, l = 0.0f;
+    const uint32_t my_end = a.p0 + q0 + col + 1;                         // this lane's query sees [0, my_end)
+    const uint32_t wave_end = q0 < a.n ? a.p0 + min(q0 + QT, a.n) : 0;   // uniform
+
+    store(smem);
+    uint32_t buf = 0;
+    for (uint32_t p = 0; p < end_all; p += PT) {
+        load(min(p + PT, end_all - 1));   // the last tile's request repeats a row and is not used
+        __syncthreads();
+        const unsigned char *kt = smem + buf * T::BYTES, *vt = kt + T::K;
+        if (p < wave_end) {
+            // two chains, so that an MFMA need not wait for the one before it
+            pf16 s = (pf16){}, s2 = (pf16){};
+            if constexpr (F16) {
+#pragma unroll
+                for (int t = 0; t < D / 16; ++t) {
+                    const ph8 k = *(const ph8 *)(kt + ((size_t)col * T::KP + 16 * t + 8 * h) * 2);
+                    s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, ql[t], s2, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, qh[t], s, 0, 0, 0);
+                    s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, qm[t], s2, 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < D / 8; ++t) {
+                    const jf4 k = *(const jf4 *)(kt + ((size_t)col * T::KP + 8 * t + 4 * h) * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; i += 2) {
+                        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i], qf[t][i], s, 0, 0, 0);
+                        s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i + 1], qf[t][i + 1], s2, 0, 0, 0);
+                    }
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[v] += s2[v];
+            // s[4 j + i]: position p + 8 j + 4 h + i
+            float bm = -INFINITY;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const bool live = p + 8 * (v >> 2) + 4 * h + (v & 3) < my_end;
+                s[v] = live ? s[v] * sc2 : -INFINITY;
+                bm = fmaxf(bm, s[v]);
+            }
+            bm = fmaxf(bm, swap32(bm));
+            const float mn = fmaxf(m, bm);
+            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            float sum = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                s[v] = mn == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[v] - mn);
+                sum += s[v];
+            }
+            l = l * alpha + sum;
+            m = mn;
+            if (__any(alpha != 1.0f))   // after the first tiles the maximum rarely moves
+#pragma unroll
+                for (int d = 0; d < ND; ++d)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+            if constexpr (F16) {
+                // 16 positions per step: half h holds 4 h + 0..3 and 8 + 4 h + 0..3 of them
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    ph8 hi, lo;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float x = s[8 * t + e] * 16384.0f;
+                        const _Float16 xh = (_Float16)x;
+                        hi[e] = xh;
+                        lo[e] = (_Float16)(x - (float)xh);
+                    }
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) {
+                        const unsigned char *vp = vt + ((size_t)(32 * d + col) * T::VP + 16 * t + 4 * h) * 2;
+                        const uint2 v0 = *(const uint2 *)vp, v1 = *(const uint2 *)(vp + 16);
+                        const ph8 v = __builtin_bit_cast(ph8, make_uint4(v0.x, v0.y, v1.x, v1.y));
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, lo, o[d], 0, 0, 0);
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, hi, o[d], 0, 0, 0);
+                    }
+                }
+            } else {
+                // step v: positions 8 (v / 4) + v % 4 (half 0) and that plus 4 (half 1)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) {
+                        const float x = *(const float *)(vt + ((size_t)(8 * (v >> 2) + 4 * h + (v & 3)) * T::VP + 32 * d + col) * 4);
+                        o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, s[v], o[d], 0, 0, 0);
+                    }
+            }
+        }
+        buf ^= 1u;
+        store(smem + buf * T::BYTES);   // last read before the barrier above
+    }
+    if (q0 + col >= a.n) return;
+    float lt = l + swap32(l);
+    const float inv = (F16 ? 1.0f / 16384.0f : 1.0f) / fmaxf(lt, 1e-20f);
+    const size_t at = ((size_t)(q0 + col) * a.heads + head) * D + 4 * h;
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float x0 = o[d][4 * j] * inv, x1 = o[d][4 * j + 1] * inv, x2 = o[d][4 * j + 2] * inv,
+                        x3 = o[d][4 * j + 3] * inv;
+            const size_t i = at + 32 * d + 8 * j;
+            if (a.out_f16)
+                *(uint2 *)((uint16_t *)a.out + i) = make_uint2((uint32_t)f2h_bits(x0) | ((uint32_t)f2h_bits(x1) << 16),
+                                                               (uint32_t)f2h_bits(x2) | ((uint32_t)f2h_bits(x3) << 16));
+            else *(jf4 *)((float *)a.out + i) = jf4{x0, x1, x2, x3};
+        }
+}
+
+template <typename KV, int D, int HW>
+void launch(janus_ctx *ctx, const PrefillArgs &a) {
+    static const bool attr_set = [] {   // thread-safe one-time set-up
+        (void)hipFuncSetAttribute((const void *)prefill_attn_kernel<KV, D, HW>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        return true;
+    }();
+    (void)attr_set;
+    const uint32_t rows = 4 / HW * QT, G = a.heads / a.kv_heads;
+    const dim3 grid((a.n + rows - 1) / rows, a.kv_heads * (G / HW));
+    constexpr size_t lds = 2 * Tile<KV, D>::BYTES;
+    hipLaunchKernelGGL((prefill_attn_kernel<KV, D, HW>), grid, dim3(256), lds, ctx->stream, a);
+}
+
+template <typename KV, int D>
+void launch_heads(janus_ctx *ctx, const PrefillArgs &a) {
+    const uint32_t G = a.heads / a.kv_heads;
+    if (G % 4 == 0) launch<KV, D, 4>(ctx, a);
+    else if (G % 2 == 0) launch<KV, D, 2>(ctx, a);
+    else launch<KV, D, 1>(ctx, a);
+}
+
+}  // namespace
+
+bool prefill_attention_supported(uint32_t hd) { return hd == 64 || hd == 128; }
+
+int prefill_attention_launch(janus_ctx *ctx, const float *q, const void *kc, const void *vc, int kv_dt, void *out,
+                             uint32_t n, uint32_t p0, uint32_t heads, uint32_t kv_heads, uint32_t hd, float scale,
+                             int out_f16) {
+    if (!prefill_attention_supported(hd)) return fail(ctx, JANUS_E_INVALID_DIM, "attention: head_dim must be 64 or 128");
+    if (n == 0) return JANUS_OK;
+    const PrefillArgs a{q, kc, vc, out, n, p0, heads, kv_heads, scale * 1.4426950408889634f, out_f16};
+    if (kv_dt == JANUS_DT_F16) {
+        if (hd == 64) launch_heads<_Float16, 64>(ctx, a);
+        else launch_heads<_Float16, 128>(ctx, a);
+    } else {
+        if (hd == 64) launch_heads<float, 64>(ctx, a);
+        else launch_heads<float, 128>(ctx, a);
+    }
+    JANUS_LAUNCH_CHECK(ctx);
+    return JANUS_OK;
+}
+
+}  // namespace janus

@@ -1569,10 +1569,10 @@ int launch_x32_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, Gemm
 // the CUs splits K over workgroups.
 constexpr int kWideKR = 128, kWideNW = 8;
 
-template <class F, int MT, bool X32>
+template <class F, int MT, bool X32, int NW = kWideNW, int KW = 1>
 int launch_wide_mt(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials *parts) {
     const uint32_t G = (w->n + 31) / 32;
-    a.tiles = (G + kWideNW - 1) / kWideNW;
+    a.tiles = (G + NW - 1) / NW;
     a.mtiles = (a.rows + 32 * MT - 1) / (32 * MT);
     a.chunks = w->t32_chunks;
     a.pass_chunks = kWideKR / F::CK;
@@ -1590,7 +1590,7 @@ int launch_wide_mt(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartia
         a.ws = (float *)ctx->gemm_ws;
     }
     const uint32_t gx = a.mtiles > 1 ? (a.tiles + 7) / 8 * 8 * a.mtiles : a.tiles;
-    launch_pipe<F, MT, 1, kWideKR, X32, kWideNW>(ctx, dim3(gx, a.ksplit), a);
+    launch_pipe<F, MT, KW, kWideKR, X32, NW>(ctx, dim3(gx, a.ksplit), a);
     JANUS_LAUNCH_CHECK(ctx);
     if (parts) {
         *parts = GemmPartials{a.ws, a.ksplit, mpad, G * 32, nullptr};
@@ -1602,7 +1602,21 @@ int launch_wide_mt(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartia
 
 template <class F>
 int launch_wide(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, GemmPartials *parts) {
-    if (a.a32) return launch_wide_mt<F, 2, true>(ctx, a, w, parts);
+    if (a.a32) {
+        // the form with the fewest rounds of workgroups over the CUs, weighed by
+        // what one takes: 64 rows x 8 row groups, 96 rows x 8, or 64 x 4 with
+        // two K slices (Q4_K 22016x4096 at 133 rows: 258 workgroups of the
+        // first kind need a second round for the last two)
+        const uint64_t cus = (uint64_t)ctx->num_cus;
+        auto time = [&](uint32_t rows, uint32_t nw, float unit) {
+            const uint64_t wgs = ((w->n + 31) / 32 + nw - 1) / nw * (uint64_t)((a.rows + rows - 1) / rows);
+            const uint64_t ks = a.swiglu || wgs > cus ? 1 : cus / wgs;
+            return unit * (float)((wgs * ks + cus - 1) / cus) / (float)ks;
+        };
+        const float t2 = time(64, 8, 1.0f), t3 = time(96, 8, 1.45f), t4 = time(64, 4, 0.57f);
+        if (t2 <= t3 && t2 <= t4) return launch_wide_mt<F, 2, true>(ctx, a, w, parts);
+        return t3 <= t4 ? launch_wide_mt<F, 3, true>(ctx, a, w, parts) : launch_wide_mt<F, 2, true, 4, 2>(ctx, a, w, parts);
+    }
     // the M tile with the least padded work (per workgroup, unpacking and
     // staging cost about what 0.7 of an M subtile does)
     auto cost = [&](uint32_t mt) { return (float)((a.rows + 32 * mt - 1) / (32 * mt)) * ((float)mt + 0.7f); };

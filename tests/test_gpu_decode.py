@@ -472,3 +472,32 @@ def test_prompt_chunks_at_capacity_and_in_every_loop(engine):
         m.forward([t], [p])
     assert _rel_err(got, m.logits()[0]) <= 1e-5
     m.close()
+
+
+@pytest.mark.parametrize("act", [_lib.DT_F32, _lib.DT_F16])
+@pytest.mark.parametrize("heads,kv_heads", [(4, 4), (4, 2), (8, 1), (16, 2), (4, 1)])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_prompt_attention_head_layouts(engine, act, heads, kv_heads, hd):
+    """The chunk attention's head and row-tile splits (1, 2, 4 or 8 query heads
+    per KV head) and both head sizes, at prompt lengths around its 32-row
+    tiles: the second layer's K/V rows (which hold the first layer's attention)
+    and the logits against eager token-by-token steps, tolerances as in
+    test_prompt_chunks_match_token_by_token."""
+    s = synth.make_model(90 + heads + kv_heads, heads * hd, heads, kv_heads, 256, 300, 2, synth.Q8_0, 1e-5, 10000.0,
+                         embed_type=synth.F16, head_type=synth.F16)
+    dt = torch.float16 if act == _lib.DT_F16 else torch.float32
+    kv, tol = [], 1e-5 if act == _lib.DT_F32 else 2e-3
+    m = Model(engine, s, max_seq_len=150, kv_dtype=act, act_dtype=act)
+    for _ in range(2):
+        kv.append(torch.zeros(2, 150, kv_heads, hd, dtype=dt, device=DEV))
+    m.set_kv_cache(*kv)
+    prompt = _prompt(91, 131, s.vocab)
+    for n in (5, 32, 33, 131):
+        for p, t in enumerate(prompt[:n] + [prompt[n - 1]]):
+            m.forward([t], [p])
+        want, rows = m.logits()[0], [x[:, :n].double() for x in kv]
+        m.generate(prompt[:n], 1)
+        assert _rel_err(m.logits()[0], want) <= tol, n
+        for x, r in zip(kv, rows):
+            assert float((x[:, :n].double() - r).norm() / r.norm()) <= tol, n
+    m.close()
