@@ -236,12 +236,13 @@ __device__ __forceinline__ f16x block_b(const _Float16 *ap, uint32_t plane, b8 b
     return t;
 }
 
-// The 16 per-row values of a lane's tile rows from s (one float per row): rows
-// 8 j + 4 h + 0..3 (the MFMA C layout).
+// The per-row values of a lane's tile rows from s (one float per row): rows
+// 8 j + 4 h + 0..3 (the MFMA C layout), the first VN of them.
+template <int VN>
 __device__ __forceinline__ f16x tile_rows(const float *s, int h) {
-    f16x t;
+    f16x t = (f16x){};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < VN / 4; ++j) {
         const jf4 v = *(const jf4 *)(s + 8 * j + 4 * h);
         t[4 * j] = v.x;
         t[4 * j + 1] = v.y;
@@ -312,16 +313,23 @@ __device__ __forceinline__ void pin(f16x (&acc)[MT]) {
         for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[mt]));
 }
 
+// Products with at most 8 or 16 rows use the first VN = 4 or 8 values of a
+// lane's result tile (rows 8 (v / 4) + 4 (lane / 32) + v % 4): the scale FMAs,
+// the K-slice sums and the stores stop there, and 8 or 16 rows of activations
+// are staged, read by the lanes of rows that have none modulo that many.
+template <int MT, int VN> constexpr int rows_staged() { return VN == 16 ? MT * 32 : 2 * VN; }
+template <int VN> constexpr int row_mask() { return VN == 16 ? 31 : 2 * VN - 1; }
+
 // acc += the pending block's scaled results; t with scale d becomes pending
 // (from three M tiles on t is applied at once: the tiles' MFMAs cover each
 // other's latency, and a second set of results does not fit the registers).
-template <int MT, bool PIN = false>
+template <int MT, bool PIN = false, int VN = 16>
 __device__ __forceinline__ void apply_deferred(f16x (&acc)[MT], Deferred<MT> &pend, const f16x (&t)[MT], float d) {
     if constexpr (MT >= 3) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(d, t[mt][v], acc[mt][v]);
+            for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(d, t[mt][v], acc[mt][v]);
         pin<MT>(acc);
         pin<MT, PIN>(acc);
         return;
@@ -329,7 +337,7 @@ __device__ __forceinline__ void apply_deferred(f16x (&acc)[MT], Deferred<MT> &pe
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
+        for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
     pin<MT>(acc);
     pin<MT, PIN>(acc);
 #pragma unroll
@@ -346,10 +354,10 @@ struct GQ4_0 {
     // One chunk on binary32 activations: As holds their three bfloat16 parts
     // (`plane` halves apart). The offset -8 enters as the first accumulator,
     // -8 * sum(x) of the block, so the weights stay the integers 0..15.
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t, int lane, const float *Ss, f16x (&acc)[MT], Deferred<MT> &pend) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const uint32_t q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -358,8 +366,8 @@ struct GQ4_0 {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
                 t[mt] = block_b<true>(As + (size_t)(mt * 32 + r) * pitch + kl + b * 32 + 8 * h, plane, b0, b1,
-                                tile_rows(Ss + (size_t)(kl / 32 + b) * (MT * 32) + mt * 32, h));
-            apply_deferred<MT, PIN>(acc, pend, t, h2f((uint16_t)(b ? (w.s >> 16) : (w.s & 0xffffu))));
+                                tile_rows<VN>(Ss + (size_t)(kl / 32 + b) * rows_staged<MT, VN>() + mt * 32, h));
+            apply_deferred<MT, PIN, VN>(acc, pend, t, h2f((uint16_t)(b ? (w.s >> 16) : (w.s & 0xffffu))));
         }
     }
     // g and c are wavefront-uniform: the chunk base is scalar, the lane adds
@@ -371,10 +379,10 @@ struct GQ4_0 {
         w.s = *(const uint32_t *)(a.side + ch * 128 + (uint32_t)(lane & 31) * 4u);
         return w;
     }
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma_deferred(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                         f16x (&acc)[MT], Deferred<MT> &pend) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const uint32_t q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -388,13 +396,13 @@ struct GQ4_0 {
                 t[mt] = mfma(lds_h8(ap), b0, (f16x){});
                 t[mt] = mfma(lds_h8(ap + 16), b1, t[mt]);
             }
-            apply_deferred<MT, PIN>(acc, pend, t, d);
+            apply_deferred<MT, PIN, VN>(acc, pend, t, d);
         }
     }
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *, uint32_t, f16x (&acc)[MT]) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const uint32_t q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -407,7 +415,7 @@ struct GQ4_0 {
                 f16x t = mfma(lds_h8(ap), b0, (f16x){});
                 t = mfma(lds_h8(ap + 16), b1, t);
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(d, t[v], acc[mt][v]);
+                for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(d, t[v], acc[mt][v]);
             }
         }
     }
@@ -419,16 +427,16 @@ struct GQ8_0 {
     static constexpr float XSUM = 0.0f;   // no sums
     struct W { uint4 q; uint16_t s; };
     // see GQ4_0::mma_x32
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t, int lane, const float *, f16x (&acc)[MT], Deferred<MT> &pend) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const b8 b0 = unpack_i8x8_b(w.q.x, w.q.y), b1 = unpack_i8x8_b(w.q.z, w.q.w);
         f16x t[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
             t[mt] = block_b<false>(As + (size_t)(mt * 32 + r) * pitch + kl + 8 * h, plane, b0, b1, (f16x){});
-        apply_deferred<MT, PIN>(acc, pend, t, h2f_q8(w.s));
+        apply_deferred<MT, PIN, VN>(acc, pend, t, h2f_q8(w.s));
     }
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
         const size_t ch = (size_t)g * a.chunks + c;
@@ -437,10 +445,10 @@ struct GQ8_0 {
         w.s = ((const uint16_t *)a.side)[ch * 32 + (lane & 31)];
         return w;
     }
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *, uint32_t, f16x (&acc)[MT]) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const h8 b0 = unpack_i8x8(w.q.x, w.q.y);
         const h8 b1 = unpack_i8x8(w.q.z, w.q.w);
         const float d = h2f_q8(w.s);
@@ -450,7 +458,7 @@ struct GQ8_0 {
             f16x t = mfma(lds_h8(ap), b0, (f16x){});
             t = mfma(lds_h8(ap + 16), b1, t);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(d, t[v], acc[mt][v]);
+            for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(d, t[v], acc[mt][v]);
         }
         pin<MT>(acc);
     }
@@ -468,11 +476,11 @@ struct GQ4_K {
     // values q - 8 and ds * (q . x) - dm * sum(x) = ds * t + (dm - 8 ds) / 8 * staged:
     // the two large terms of a block mostly cancel before they are rounded.
     // c: chunk of the row group.
-    template <int MT, bool PIN = false, class G = GQ4_K>
+    template <int MT, bool PIN = false, int VN = 16, class G = GQ4_K>
     __device__ static void mma_x32(const typename G::W &w, const _Float16 *As, uint32_t plane, uint32_t pitch,
                                    uint32_t kl, uint32_t c, int lane, const float *Ss, f16x (&acc)[MT],
                                    Deferred<MT> &) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const float d = h2f((uint16_t)(w.hdr.x & 0xffffu)), dmin = h2f((uint16_t)(w.hdr.x >> 16));
         const int j = (int)(c & 3);   // chunk index within the super-block
 #pragma unroll
@@ -485,11 +493,11 @@ struct GQ4_K {
             G::unpack_b(w, b, b0, b1);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                const f16x s = tile_rows(Ss + (size_t)(kl / 32 + b) * (MT * 32) + mt * 32, h);
+                const f16x s = tile_rows<VN>(Ss + (size_t)(kl / 32 + b) * rows_staged<MT, VN>() + mt * 32, h);
                 const f16x t =
                     block_b<true>(As + (size_t)(mt * 32 + r) * pitch + kl + b * 32 + 8 * h, plane, b0, b1, s);
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(cs, s[v], fmaf(ds, t[v], acc[mt][v]));
+                for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(cs, s[v], fmaf(ds, t[v], acc[mt][v]));
             }
             pin<MT, PIN>(acc);
             pin<MT>(acc);
@@ -513,10 +521,10 @@ struct GQ4_K {
         sc = (float)((g >> o) & 63u);
         mn = (float)((g >> (12u + o)) & 63u);
     }
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *Ss, uint32_t chunk0, f16x (&acc)[MT]) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const uint32_t q[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
         const float d = h2f((uint16_t)(w.hdr.x & 0xffffu)), dmin = h2f((uint16_t)(w.hdr.x >> 16));
         const int j = (int)((kl / 64 + chunk0) & 3);   // chunk index within the super-block (chunk0: the pass's first)
@@ -533,9 +541,9 @@ struct GQ4_K {
                 const _Float16 *ap = As + (size_t)(mt * 32 + r) * pitch + kl + b * 32 + 8 * h;
                 f16x t = mfma(lds_h8(ap), b0, (f16x){});
                 t = mfma(lds_h8(ap + 16), b1, t);
-                const float *sx = Ss + (size_t)sub * (MT * 32) + mt * 32 + 4 * h;
+                const float *sx = Ss + (size_t)sub * rows_staged<MT, VN>() + mt * 32 + 4 * h;
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj) {
+                for (int jj = 0; jj < VN / 4; ++jj) {
                     const jf4 s4 = *(const jf4 *)(sx + 8 * jj);
                     acc[mt][4 * jj + 0] = fmaf(-dm, s4.x, fmaf(ds, t[4 * jj + 0], acc[mt][4 * jj + 0]));
                     acc[mt][4 * jj + 1] = fmaf(-dm, s4.y, fmaf(ds, t[4 * jj + 1], acc[mt][4 * jj + 1]));
@@ -557,10 +565,10 @@ struct GQ5_K {
     static constexpr bool ORDER4 = true;
     static constexpr float XSUM = -16.0f;
     struct W { uint4 q; uint4 hdr; uint32_t fifth; };
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t c, int lane, const float *Ss, f16x (&acc)[MT], Deferred<MT> &pend) {
-        GQ4_K::mma_x32<MT, PIN, GQ5_K>(w, As, plane, pitch, kl, c, lane, Ss, acc, pend);
+        GQ4_K::mma_x32<MT, PIN, VN, GQ5_K>(w, As, plane, pitch, kl, c, lane, Ss, acc, pend);
     }
     __device__ static void unpack_b(const W &w, int b, b8 &b0, b8 &b1) {
         b0 = b ? unpack_nib8_q5_b<2>(w.q.z, w.fifth) : unpack_nib8_q5_b<0>(w.q.x, w.fifth);
@@ -575,10 +583,10 @@ struct GQ5_K {
         w.hdr = *(const uint4 *)(a.side + (sb * 32 + (lane & 31)) * 16);
         return w;
     }
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *Ss, uint32_t chunk0, f16x (&acc)[MT]) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const float d = h2f((uint16_t)(w.hdr.x & 0xffffu)), dmin = h2f((uint16_t)(w.hdr.x >> 16));
         const int j = (int)((kl / 64 + chunk0) & 3);   // chunk index within the super-block (chunk0: the pass's first)
 #pragma unroll
@@ -594,9 +602,9 @@ struct GQ5_K {
                 const _Float16 *ap = As + (size_t)(mt * 32 + r) * pitch + kl + b * 32 + 8 * h;
                 f16x t = mfma(lds_h8(ap), b0, (f16x){});
                 t = mfma(lds_h8(ap + 16), b1, t);
-                const float *sx = Ss + (size_t)sub * (MT * 32) + mt * 32 + 4 * h;
+                const float *sx = Ss + (size_t)sub * rows_staged<MT, VN>() + mt * 32 + 4 * h;
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj) {
+                for (int jj = 0; jj < VN / 4; ++jj) {
                     const jf4 s4 = *(const jf4 *)(sx + 8 * jj);
                     acc[mt][4 * jj + 0] = fmaf(-dm, s4.x, fmaf(ds, t[4 * jj + 0], acc[mt][4 * jj + 0]));
                     acc[mt][4 * jj + 1] = fmaf(-dm, s4.y, fmaf(ds, t[4 * jj + 1], acc[mt][4 * jj + 1]));
@@ -614,12 +622,12 @@ struct GQ5_K {
 template <class F, class = void> struct Defers { static constexpr bool value = false; };
 template <class F> struct Defers<F, std::void_t<decltype(F::DEFER)>> { static constexpr bool value = F::DEFER; };
 
-template <int MT>
+template <int MT, int VN = 16>
 __device__ __forceinline__ void flush_deferred(f16x (&acc)[MT], const Deferred<MT> &pend) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
+        for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
 }
 
 // formats whose mins need the per-(row, sub-block) activation sums in LDS
@@ -637,10 +645,10 @@ struct GF16 {
     // the five small ones (below 2^-7 of it) to pend.t, added at the end, so
     // their roundings stay at their own size. inf: an activation may be
     // infinite; it then meets only the leading weight part (the other may be 0).
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
                                    uint32_t inf, int lane, const float *, f16x (&acc)[MT], Deferred<MT> &pend) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         b8 hi, lo;
         split_f16x8(w.q, hi, lo);
 #pragma unroll
@@ -661,10 +669,10 @@ struct GF16 {
         w.q = ld_stream(a.qs + (ch * 64 + lane) * 16);
         return w;
     }
-    template <int MT, bool PIN = false>
+    template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma(const W &w, const _Float16 *As, uint32_t pitch, uint32_t kl, int lane,
                                const float *, uint32_t, f16x (&acc)[MT]) {
-        const int h = lane >> 5, r = lane & 31;
+        const int h = lane >> 5, r = lane & row_mask<VN>();
         const h8 b = __builtin_bit_cast(h8, w.q);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma(lds_h8(As + (size_t)(mt * 32 + r) * pitch + kl + 8 * h), b, acc[mt]);
@@ -855,12 +863,13 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_mfma_kernel(GemmArgs a) 
 
 // Bytes of one staging buffer of gemm_pipe_kernel: the activations (three
 // bfloat16 planes with X32) and, where the format needs them, the per-block sums.
-template <class F, int MT, int KR, bool X32>
+template <class F, int MT, int KR, bool X32, int VN>
 constexpr uint32_t pipe_buf() {
-    constexpr uint32_t abytes = (uint32_t)MT * 32 * (KR + 8) * 2 * (X32 ? 3 : 1);
+    constexpr uint32_t rows = rows_staged<MT, VN>();
+    constexpr uint32_t abytes = rows * (KR + 8) * 2 * (X32 ? 3 : 1);
     constexpr bool sums = X32 ? F::XSUM != 0.0f : NeedsSums<F>::value;
     constexpr bool flag = X32 && std::is_same<F, GF16>::value;   // an infinite activation was staged
-    return (abytes + (sums ? (uint32_t)(KR / 32) * MT * 32 * 4 : flag ? 4u : 0u) + 15u) / 16u * 16u;
+    return (abytes + (sums ? (uint32_t)(KR / 32) * rows * 4 : flag ? 4u : 0u) + 15u) / 16u * 16u;
 }
 
 // Cross-pass pipelined form of gemm_mfma_kernel (quantised and F16 weights),
@@ -876,7 +885,7 @@ constexpr uint32_t pipe_buf() {
 // scale rounding, slice order and outputs are those of gemm_mfma_kernel.
 // X32: binary32 activations, split into three bfloat16 parts as they are
 // stored to LDS (three planes per buffer).
-template <class F, int MT, int KW, int KR, bool X32, int NW = WAVES>
+template <class F, int MT, int KW, int KR, bool X32, int NW = WAVES, int VN = 16>
 __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr bool WIDE = KW == 1;   // the form for more than 64 rows
@@ -884,14 +893,15 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     constexpr int NT = 64 * NW * KW;   // threads
     constexpr int PC = KR / F::CK;        // chunks per pass
     constexpr int CPW = PC / KW;          // chunks per wavefront per pass
-    constexpr int MP = MT * 32;           // padded rows
+    constexpr int MP = rows_staged<MT, VN>();   // padded rows
     constexpr int PITCH = KR + 8;         // LDS row pitch in halves
     constexpr int SEGS = KR / 8;          // 16-byte segments per row of a pass
-    constexpr int SPT = MP * SEGS / NT;   // segments per thread
-    static_assert(CPW >= 1 && CPW * KW == PC && SPT >= 1 && SPT * NT == MP * SEGS, "pass shape");
+    constexpr int SPT = (MP * SEGS + NT - 1) / NT;   // segments per thread
+    constexpr bool PART = SPT * NT != MP * SEGS;     // the last wavefronts stage nothing
+    static_assert(CPW >= 1 && CPW * KW == PC && (!PART || SPT == 1) && MP * SEGS % 64 == 0, "pass shape");
     constexpr uint32_t PLANE = (uint32_t)MP * PITCH;   // halves of one staged part
     constexpr uint32_t ABYTES = PLANE * 2 * (X32 ? 3 : 1);
-    constexpr uint32_t BUF = pipe_buf<F, MT, KR, X32>();
+    constexpr uint32_t BUF = pipe_buf<F, MT, KR, X32, VN>();
     constexpr bool FLAG = X32 && std::is_same<F, GF16>::value;   // one word per buffer after the activations
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar chunk bases
@@ -959,6 +969,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     auto store_a = [&](uint32_t p) {
         _Float16 *As = (_Float16 *)(smem + (p & 1) * BUF);
         const uint32_t kbase = p * KR;
+        if (PART && threadIdx.x >= MP * SEGS) return;
 #pragma unroll
         for (int i = 0; i < SPT; ++i) {
             const uint32_t s = threadIdx.x + NT * i;
@@ -1026,12 +1037,12 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
             // one or two M tiles the branches keep the chunks' order for less.
             if ((WIDE && decltype(load_next)::value) || cw + i < c1) {
                 if constexpr (X32)
-                    F::template mma_x32<MT, WIDE>(w[i], As, PLANE, PITCH, (uint32_t)(kw * CPW + i) * F::CK,
+                    F::template mma_x32<MT, WIDE, VN>(w[i], As, PLANE, PITCH, (uint32_t)(kw * CPW + i) * F::CK,
                                             FLAG ? inf : cw + i, lane, Ss, part, pend);
                 else if constexpr (Defers<F>::value)
-                    F::template mma_deferred<MT, WIDE>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, acc, pend);
+                    F::template mma_deferred<MT, WIDE, VN>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, acc, pend);
                 else
-                    F::template mma<MT, WIDE>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, Ss, p * PC, acc);
+                    F::template mma<MT, WIDE, VN>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, Ss, p * PC, acc);
             }
             if (decltype(load_next)::value) w[i] = F::load(a, gl, chunk_of(p + 1, i), lane);
             if constexpr (WIDE) __builtin_amdgcn_sched_barrier(0);
@@ -1041,7 +1052,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[mt][v] += part[mt][v];
+                    for (int v = 0; v < VN; ++v) acc[mt][v] += part[mt][v];
                     part[mt] = (f16x){};
                 }
     };
@@ -1069,7 +1080,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
         pass(last, std::false_type{});
     }
     if constexpr (X32 && std::is_same<F, GF16>::value) pend.d = 1.0f;   // the small parts
-    if constexpr (X32 ? !NeedsSums<F>::value : Defers<F>::value) flush_deferred<MT>(acc, pend);
+    if constexpr (X32 ? !NeedsSums<F>::value : Defers<F>::value) flush_deferred<MT, VN>(acc, pend);
 
     if (KW > 1) {
         float *red = (float *)smem;
@@ -1077,11 +1088,11 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
         for (int mt = 0; mt < MT; ++mt) {
             __syncthreads();
 #pragma unroll
-            for (int v = 0; v < 16; ++v) red[((size_t)wave * 16 + v) * 64 + lane] = acc[mt][v];
+            for (int v = 0; v < VN; ++v) red[((size_t)wave * 16 + v) * 64 + lane] = acc[mt][v];
             __syncthreads();
             if (kw == 0) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
+                for (int v = 0; v < VN; ++v) {
                     float sum = red[((size_t)rgw * 16 + v) * 64 + lane];
                     for (int j = 1; j < KW; ++j) sum += red[((size_t)(j * NW + rgw) * 16 + v) * 64 + lane];
                     acc[mt][v] = sum;
@@ -1099,31 +1110,52 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-            __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * MP * a.mtiles + m0 + out_row(mt, v, lane)) * Npad + n);
+        for (int v = 0; v < VN; ++v)
+            __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * (MT * 32) * a.mtiles + m0 + out_row(mt, v, lane)) * Npad + n);
 }
 
 // LDS bytes of gemm_pipe_kernel: two staging buffers, at least the K-slice
 // reduction area.
-template <class F, int MT, int KW, int KR, bool X32, int NW>
+template <class F, int MT, int KW, int KR, bool X32, int NW, int VN>
 constexpr size_t pipe_lds() {
-    constexpr size_t buf = pipe_buf<F, MT, KR, X32>();
+    constexpr size_t buf = pipe_buf<F, MT, KR, X32, VN>();
     constexpr size_t red = (size_t)NW * KW * 16 * 64 * 4;
     static_assert(2 * buf <= 160 * 1024 && red <= 160 * 1024, "LDS");
     return 2 * buf > red ? 2 * buf : red;
 }
 
-template <class F, int MT, int KW, int KR, bool X32 = false, int NW = WAVES>
+constexpr size_t kHalfLds = 81 * 1024;   // more than half of a CU's 160 KB
+template <class F, int MT, int KW, int KR, bool X32 = false, int NW = WAVES, int VN = 16>
 void launch_pipe(janus_ctx *ctx, dim3 grid, const GemmArgs &a) {
     // thread-safe one-time set-up (a function-local static's initialiser)
     static const bool attr_set = [] {
-        (void)hipFuncSetAttribute((const void *)gemm_pipe_kernel<F, MT, KW, KR, X32, NW>,
+        (void)hipFuncSetAttribute((const void *)gemm_pipe_kernel<F, MT, KW, KR, X32, NW, VN>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         return true;
     }();
     (void)attr_set;
-    constexpr size_t lds = pipe_lds<F, MT, KW, KR, X32, NW>();
-    hipLaunchKernelGGL((gemm_pipe_kernel<F, MT, KW, KR, X32, NW>), grid, dim3(64 * NW * KW), lds, ctx->stream, a);
+    // Where the workgroups do not outnumber the CUs, each asks for more than
+    // half of a CU's LDS: the dispatcher otherwise puts two on one CU and
+    // leaves another idle.
+    size_t lds = pipe_lds<F, MT, KW, KR, X32, NW, VN>();
+    if (grid.x * grid.y <= (uint32_t)ctx->num_cus && lds < kHalfLds) lds = kHalfLds;
+    hipLaunchKernelGGL((gemm_pipe_kernel<F, MT, KW, KR, X32, NW, VN>), grid, dim3(64 * NW * KW), lds, ctx->stream, a);
+}
+
+// Whether gemm_pipe_kernel has a form for at most 8 and 16 rows: one M tile of a
+// quantised weight (14336x4096 at 8 binary16 rows: Q4_0 15.7 -> 13.4 us, Q5_K
+// 21.8 -> 17.8; 11008x4096 Q4_K at 16 binary32 rows 25.7 -> 18.4). F16 weights
+// have no scales to save and measured slower (32000x4096: 54 -> 66 us).
+template <class F, int MT> constexpr bool trims_rows() { return MT == 1 && !std::is_same<F, GF16>::value; }
+
+// gemm_pipe_kernel for the row count: at most 8, 16 or 32 rows of one M tile.
+template <class F, int MT, int KW, int KR, bool X32>
+void launch_pipe_rows(janus_ctx *ctx, dim3 grid, const GemmArgs &a) {
+    if constexpr (trims_rows<F, MT>()) {
+        if (a.rows <= 8) return launch_pipe<F, MT, KW, KR, X32, WAVES, 4>(ctx, grid, a);
+        if (a.rows <= 16) return launch_pipe<F, MT, KW, KR, X32, WAVES, 8>(ctx, grid, a);
+    }
+    launch_pipe<F, MT, KW, KR, X32>(ctx, grid, a);
 }
 
 // Sums the split-K partials in split order and applies the epilogue.
@@ -1392,6 +1424,11 @@ int launch_mfma(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials 
         if (ctx->gemm_pipe && !kr_force && !ks_force) {
             const uint32_t pp = (w->t32_chunks * F::CK + 255) / 256;
             uint32_t pks = ((uint32_t)ctx->num_cus * 11 + 10 * tiles - 1) / (10 * tiles);
+            // two M tiles: as many workgroups as run at once, one per CU for
+            // Q4_0 (158 registers), two for the other formats (14336x4096 at 33
+            // rows: Q4_0 26.4 -> 21.2 us with 224 workgroups instead of 336,
+            // Q5_K 31.2 -> 28.5 with 448)
+            if (MT == 2) pks = (uint32_t)ctx->num_cus * (std::is_same<F, GQ4_0>::value ? 1u : 2u) / tiles;
             if (pks > pp) pks = pp;
             if (pks < 1) pks = 1;
             if ((pp + pks - 1) / pks >= 3) {
@@ -1445,7 +1482,7 @@ int launch_mfma(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials 
     {
         if (pipe && a.passes_per_wg > 1) {
             piped = true;
-            if (kr == 256) launch_pipe<F, MT, KW, 256>(ctx, grid, a);
+            if (kr == 256) launch_pipe_rows<F, MT, KW, 256, false>(ctx, grid, a);
             else if (kr == 512) launch_pipe<F, MT, KW, 512>(ctx, grid, a);
             else if (MT == 1 && kr == 1024) launch_pipe<F, MT, KW, 1024 / MT>(ctx, grid, a);
             else piped = false;
@@ -1479,9 +1516,11 @@ int launch_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, GemmPart
 
 // Splits the product for gemm_pipe_kernel on binary32 activations: fills the
 // plan fields of a and returns the workspace bytes (0: no K split). MT M-tiles
-// of 32 rows, KR-long passes. The staged parts fill most of a CU's LDS, so one
-// workgroup runs per CU: K is split as far as the workgroups still fit in one
-// round.
+// of 32 rows, KR-long passes. The staged parts of 32 and more rows fill most of
+// a CU's LDS, so one workgroup runs per CU and K is split as far as the
+// workgroups still fit in one round; with at most 16 rows two run, and K is
+// split until there are two per CU (11008x4096 at 16 rows: 18.4 us against
+// 20.4 with 344 workgroups and 23.0 with 172).
 template <class F, int MT, int KR>
 size_t plan_x32(const janus_ctx *ctx, GemmArgs &a, const janus_weight *w, dim3 &grid) {
     const uint32_t G = (w->n + 31) / 32, tiles = (G + WAVES - 1) / WAVES;
@@ -1489,6 +1528,7 @@ size_t plan_x32(const janus_ctx *ctx, GemmArgs &a, const janus_weight *w, dim3 &
     a.pass_chunks = KR / F::CK;
     a.total_passes = (a.chunks + a.pass_chunks - 1) / a.pass_chunks;
     uint32_t ks = (uint32_t)ctx->num_cus / tiles;
+    if (trims_rows<F, MT>() && a.rows <= 16) ks = (2 * (uint32_t)ctx->num_cus + tiles - 1) / tiles;
     if (ks > a.total_passes) ks = a.total_passes;
     if (ks < 1) ks = 1;
     a.passes_per_wg = (a.total_passes + ks - 1) / ks;
@@ -1535,7 +1575,7 @@ int launch_x32(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials *
     a.ws = (float *)ctx->gemm_ws;
     a.to_ws = parts != nullptr;
     *ran = true;
-    launch_pipe<F, MT, KW, KR, true>(ctx, grid, a);
+    launch_pipe_rows<F, MT, KW, KR, true>(ctx, grid, a);
     JANUS_LAUNCH_CHECK(ctx);
     if (parts) {
         *parts = GemmPartials{a.ws, a.ksplit, MT * 32, npad, nullptr};

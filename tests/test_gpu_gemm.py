@@ -83,6 +83,22 @@ def test_pipelined_gemm_shapes_match_f64(engine, ggml_type, rows, n, k):
     _check_against_f64(outs[0].numpy(), w.dequant().cpu().numpy(), a16)
 
 
+@pytest.mark.parametrize("ggml_type", [2, 8, 12, 13])
+@pytest.mark.parametrize("rows", [2, 8, 9, 16, 17])
+@pytest.mark.parametrize("n,k", [(6144, 4096), (6176, 4352)])
+def test_pipelined_gemm_row_trimmed_forms(engine, ggml_type, rows, n, k):
+    """The pipelined kernel's forms for at most 8 and 16 rows (the scale FMAs,
+    the stage and the stores stop at the row count), at their edges, with a
+    partial row-group tile and a K split."""
+    raw, w = _weight(engine, ggml_type, n, k, 600 + ggml_type + rows)
+    a16 = _acts(rows, k, 13 * rows + n)
+    c = torch.full((rows + 1, n), 7.0, device=DEV)
+    ops.gemm_auto(engine, a16.to(DEV), w, c, rows, 1, k, n)
+    torch.cuda.synchronize()
+    assert bool((c[rows] == 7.0).all())
+    _check_against_f64(c[:rows].cpu().numpy(), w.dequant().cpu().numpy(), a16)
+
+
 @pytest.mark.parametrize("ggml_type", [2, 8])
 @pytest.mark.parametrize("rows", [32, 40])
 def test_pipelined_gemm_ragged_k_and_partial_tile(engine, ggml_type, rows):
@@ -163,11 +179,11 @@ def _check_f32_against_f64(y, wf, x, bound=1e-5):
 
 
 @pytest.mark.parametrize("ggml_type", [2, 8, 12, 13, 1])
-@pytest.mark.parametrize("rows", [3, 4, 31, 32, 33, 64])
+@pytest.mark.parametrize("rows", [3, 4, 8, 9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("n,k", [(33, 256), (200, 512), (4096, 1280), (1000, 4352)])
 def test_f32_rows_on_mfma_match_f64(engine, ggml_type, rows, n, k):
-    """binary32 activations as three exact bfloat16 parts: one and two M
-    tiles, partial row groups and K passes, K split over workgroups. The
+    """binary32 activations as three exact bfloat16 parts: at most 8, 16 and 32
+    rows of an M tile, two M tiles, partial row groups and K passes, K split over workgroups. The
     parts and products are exact, so the M = 1 kernels' bound for binary32
     sums holds (1e-5 of sum |w x|); values from 2^-40 to 2^20 keep their
     digits, and a repeated call gives the same bits."""
