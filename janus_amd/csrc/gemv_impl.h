@@ -1689,9 +1689,28 @@ int launch_lds32(janus_ctx *ctx, const GemvArgs &a, bool norm) {
     return JANUS_OK;
 }
 
+// F16 rows of 9 to 32 units per lane on binary32 x (k of 4104 to 16384: a long
+// ffn_down loaded from Q6_K): the whole row is in flight at once,
+// single-buffered, and x is read from LDS at use. They took the per-launch
+// kernel, which stages x behind four rows' loads in every 256-thread
+// workgroup: 4096x14336 43.0 -> 22.5 us (5.2 TB/s), 4096x11008 34.2 -> 17.9,
+// 4096x8192 unchanged at 13.7. (With binary16 x the register kernel holds
+// such rows' x and is as fast: 21.7 us at 4096x14336.)
+inline int launch_f16_long(janus_ctx *ctx, const GemvArgs &a, int bpl, bool &done) {
+    done = bpl <= 32;
+    if (!done) return JANUS_OK;
+    if (bpl <= 12) return launch_lds32<FF16, 12, 1>(ctx, a, false);
+    if (bpl <= 16) return launch_lds32<FF16, 16, 1>(ctx, a, false);
+    if (bpl <= 22) return launch_lds32<FF16, 22, 1>(ctx, a, false);
+    if (bpl <= 28) return launch_lds32<FF16, 28, 1>(ctx, a, false);
+    return launch_lds32<FF16, 32, 1>(ctx, a, false);
+}
+
 template <class F>
 int launch_lds32_fmt(janus_ctx *ctx, const GemvArgs &a, bool norm, bool pair, bool &done) {
     const int bpl = (int)((a.units + 63) / 64);
+    if constexpr (std::is_same<F, FF16>::value)
+        if (bpl > 8 && !norm && !pair) return launch_f16_long(ctx, a, bpl, done);
     done = bpl <= 8;
     if (!done) return JANUS_OK;
     if (pair) {

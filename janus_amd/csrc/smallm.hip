@@ -1545,7 +1545,9 @@ size_t plan_x32(const janus_ctx *ctx, GemmArgs &a, const janus_weight *w, dim3 &
 // (256 to 1024 square) cost 4-8 us against 2.4-3.5 us a row, so they gain from
 // three rows too, but three rows below 2^20 weights stay with the row kernels:
 // their results equal single calls bit for bit, and the time at stake is 3 us.
+// Rows longer than the row kernels take (2048 units) stay with them, refused.
 bool x32_pays(const janus_weight *w, uint32_t rows) {
+    if (w->k / (w->type == JANUS_DT_F16 ? 8u : 32u) > 2048u) return false;
     return rows > 3 || (rows == 3 && (uint64_t)w->n * w->k >= (1u << 20));
 }
 

@@ -243,3 +243,33 @@ def test_gemv_error_is_unbiased_across_rows(engine, ggml_type, xdt, m):
     mean, rms = float(np.mean(np.abs(means))), float(np.mean(rmss))
     assert rms < 2e-8, (means, rmss)
     assert mean < 0.25 * rms + 1e-10, (means, rmss)
+
+
+@pytest.mark.parametrize("k", [4104, 6144, 6152, 8200, 11008, 11272, 14336, 16384])
+def test_f16_long_rows_with_f32_x(engine, k):
+    """Binary16 rows of 9 to 32 units per lane on binary32 x, full and ragged,
+    with the residual form; the M = 1 kernels' bound for binary32 sums."""
+    n = 515
+    rng = np.random.default_rng(k)
+    w = ops.GpuTensor(engine, 1, n, k, synth.f16_bits(rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)))
+    x = torch.from_numpy(rng.standard_normal(k, dtype=np.float32)).cuda()
+    y = torch.full((n + 1,), 7.0, device="cuda:0")
+    ops.gemm_auto(engine, x, w, y, 1, 1, k, n)
+    wf, x64 = w.dequant().double(), x.double()
+    assert bool(((y[:n].double() - wf @ x64).abs() <= 1e-5 * (wf.abs() @ x64.abs())).all()) and y[n].item() == 7.0
+    r = torch.randn(n, device="cuda:0")
+    out = torch.empty(n, device="cuda:0")
+    ops.gemm_residual(engine, x, w, r, out, 1)
+    assert torch.equal(out, y[:n] + r)
+
+
+@pytest.mark.parametrize("rows", [1, 5])
+def test_f16_rows_beyond_the_gemv_limit_stay_refused_with_f32_x(engine, rows):
+    """k above 16384 is refused on binary32 x, for one row and for several
+    (which could run on MFMA)."""
+    n, k = 8, 16392
+    w = ops.GpuTensor(engine, 1, n, k, np.zeros((n, k), np.uint16))
+    x, y = torch.zeros(rows, k, device="cuda:0"), torch.zeros(rows, n, device="cuda:0")
+    with pytest.raises(ops.JanusError) as ei:
+        ops.gemm_auto(engine, x, w, y, rows, 1, k, n)
+    assert ei.value.status == 2
