@@ -293,15 +293,6 @@ template <int MT> struct Deferred {
     float d;      // and its scale (0 before the first block)
 };
 
-// Keeps the arithmetic on a result tile where it is written: without it the
-// compiler sinks the scale FMAs of a whole pass behind its MFMAs, and the
-// block results held for them spill.
-template <int MT>
-__device__ __forceinline__ void pin(f16x (&acc)[MT]) {
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(acc[mt]));
-}
-
 // PIN keeps the arithmetic on a result tile where it is written. In the
 // branch-free passes of the wide kernel the compiler otherwise sinks the scale
 // FMAs of a whole pass behind its MFMAs and spills the block results held for
@@ -330,7 +321,6 @@ __device__ __forceinline__ void apply_deferred(f16x (&acc)[MT], Deferred<MT> &pe
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(d, t[mt][v], acc[mt][v]);
-        pin<MT>(acc);
         pin<MT, PIN>(acc);
         return;
     }
@@ -338,7 +328,6 @@ __device__ __forceinline__ void apply_deferred(f16x (&acc)[MT], Deferred<MT> &pe
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(pend.d, pend.t[mt][v], acc[mt][v]);
-    pin<MT>(acc);
     pin<MT, PIN>(acc);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) pend.t[mt] = t[mt];
@@ -460,7 +449,7 @@ struct GQ8_0 {
 #pragma unroll
             for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(d, t[v], acc[mt][v]);
         }
-        pin<MT>(acc);
+        pin<MT, PIN>(acc);
     }
 };
 
@@ -500,7 +489,6 @@ struct GQ4_K {
                 for (int v = 0; v < VN; ++v) acc[mt][v] = fmaf(cs, s[v], fmaf(ds, t[v], acc[mt][v]));
             }
             pin<MT, PIN>(acc);
-            pin<MT>(acc);
         }
     }
     __device__ static void unpack_b(const W &w, int b, b8 &b0, b8 &b1) {
@@ -552,7 +540,6 @@ struct GQ4_K {
                 }
             }
             pin<MT, PIN>(acc);
-            pin<MT>(acc);
         }
     }
 };
@@ -613,7 +600,6 @@ struct GQ5_K {
                 }
             }
             pin<MT, PIN>(acc);
-            pin<MT>(acc);
         }
     }
 };
@@ -710,7 +696,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &a, uint32_t g, uint32
 // SwiGLU store of a finished tile: columns 2j, 2j+1 (lanes l, l^1) hold gate_j
 // and up_j of the same rows; the even lane writes silu(gate) * up (the
 // arithmetic of elementwise_kernel's SwiGLU).
-template <int MT>
+template <int MT, bool F32OUT>
 __device__ __forceinline__ void store_swiglu(const GemmArgs &a, uint32_t g, uint32_t m0, int lane,
                                              const f16x (&acc)[MT]) {
     const uint32_t n = g * 32 + (lane & 31);
@@ -724,8 +710,8 @@ __device__ __forceinline__ void store_swiglu(const GemmArgs &a, uint32_t g, uint
             const uint32_t m = m0 + out_row(mt, v, lane);
             if (!(lane & 1) && m < a.rows && n + 1 < a.n) {
                 const float act = mine * (1.0f / (1.0f + expf(-mine))) * other;
-                if (a.c_f16) ((uint16_t *)a.c)[(size_t)m * half + n / 2] = f2h_bits(act);
-                else ((float *)a.c)[(size_t)m * half + n / 2] = act;
+                if constexpr (F32OUT) ((float *)a.c)[(size_t)m * half + n / 2] = act;
+                else ((uint16_t *)a.c)[(size_t)m * half + n / 2] = f2h_bits(act);
             }
         }
 }
@@ -847,7 +833,7 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_mfma_kernel(GemmArgs a) 
     }
     if (kw != 0 || !active) return;
     if (a.ksplit == 1 && !a.to_ws) {
-        if (a.swiglu) store_swiglu<MT>(a, g, 0, lane, acc);
+        if (a.swiglu) store_swiglu<MT, false>(a, g, 0, lane, acc);
         else store_tile<MT>(a, g, 0, lane, acc);
         return;
     }
@@ -860,6 +846,8 @@ __global__ __launch_bounds__(64 * WAVES * KW) void gemm_mfma_kernel(GemmArgs a) 
         for (int v = 0; v < 16; ++v)
             __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * Mpad + out_row(mt, v, lane)) * Npad + n);
 }
+
+constexpr int kWideKR = 128;   // pass length of the forms that take several M tiles
 
 // Bytes of one staging buffer of gemm_pipe_kernel: the activations (three
 // bfloat16 planes with X32) and, where the format needs them, the per-block sums.
@@ -911,13 +899,13 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     // weight tile are consecutive on one XCD (workgroup ids go round the 8
     // XCDs), so they share the tile's weights in that XCD's L2.
     uint32_t tile = blockIdx.x, mtile = 0;
-    if (a.mtiles > 1) {
+    if (KR == kWideKR && a.mtiles > 1) {
         const uint32_t local = blockIdx.x >> 3;
         tile = (local / a.mtiles) * 8 + (blockIdx.x & 7u);
         mtile = local % a.mtiles;
         if (tile >= a.tiles) return;
     }
-    const uint32_t g = tile * NW + rgw, ks = blockIdx.y, m0 = mtile * MP;
+    const uint32_t g = tile * NW + rgw, ks = blockIdx.y, m0 = KR == kWideKR ? mtile * MP : 0;
     const bool active = g < G;
     const uint32_t p_begin = ks * a.passes_per_wg;
     const uint32_t p_end = min(a.total_passes, p_begin + a.passes_per_wg);
@@ -1037,7 +1025,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
             // one or two M tiles the branches keep the chunks' order for less.
             if ((WIDE && decltype(load_next)::value) || cw + i < c1) {
                 if constexpr (X32)
-                    F::template mma_x32<MT, WIDE, VN>(w[i], As, PLANE, PITCH, (uint32_t)(kw * CPW + i) * F::CK,
+                    F::template mma_x32<MT, true, VN>(w[i], As, PLANE, PITCH, (uint32_t)(kw * CPW + i) * F::CK,
                                             FLAG ? inf : cw + i, lane, Ss, part, pend);
                 else if constexpr (Defers<F>::value)
                     F::template mma_deferred<MT, WIDE, VN>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, acc, pend);
@@ -1102,16 +1090,17 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     }
     if (kw != 0 || !active) return;
     if (a.ksplit == 1 && !a.to_ws) {
-        if (a.swiglu) store_swiglu<MT>(a, g, m0, lane, acc);
+        if (a.swiglu) store_swiglu<MT, X32>(a, g, m0, lane, acc);
         else store_tile<MT>(a, g, m0, lane, acc);
         return;
     }
     const uint32_t Npad = G * 32, n = g * 32 + (lane & 31);
+    const uint32_t mpad = MT * 32 * (KR == kWideKR ? a.mtiles : 1);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int v = 0; v < VN; ++v)
-            __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * (MT * 32) * a.mtiles + m0 + out_row(mt, v, lane)) * Npad + n);
+            __builtin_nontemporal_store(acc[mt][v], a.ws + ((size_t)ks * mpad + m0 + out_row(mt, v, lane)) * Npad + n);
 }
 
 // LDS bytes of gemm_pipe_kernel: two staging buffers, at least the K-slice
@@ -1609,7 +1598,7 @@ int launch_x32_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, Gemm
 // x 2 K slices and 186 with MT = 2; binary32 rows 411 us (875 TFLOP/s of
 // MFMA) against 464, and 556 with MT = 3. A product with too few tiles for
 // the CUs splits K over workgroups.
-constexpr int kWideKR = 128, kWideNW = 8;
+constexpr int kWideNW = 8;
 
 template <class F, int MT, bool X32, int NW = kWideNW, int KW = 1>
 int launch_wide_mt(janus_ctx *ctx, GemmArgs a, const janus_weight *w, GemmPartials *parts) {
