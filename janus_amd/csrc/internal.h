@@ -138,6 +138,18 @@ int hip_fail(janus_ctx *ctx, hipError_t e, const char *what);
 inline bool is_act_dtype(int dt) { return dt == JANUS_DT_F32 || dt == JANUS_DT_F16; }
 inline size_t act_bytes(int dt) { return dt == JANUS_DT_F16 ? 2 : 4; }
 
+// Makes a device current and the one before it again at the end.
+struct DeviceGuard {
+    int prev = -1;
+    explicit DeviceGuard(int dev) {
+        if (hipGetDevice(&prev) == hipSuccess && prev != dev) (void)hipSetDevice(dev);
+        else prev = -1;
+    }
+    ~DeviceGuard() {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+};
+
 // Grows the context's attention workspace to at least `bytes`.
 int ensure_attn_ws(janus_ctx *ctx, size_t bytes);
 // Grows the small-M GEMM split-K partials to at least `bytes`.

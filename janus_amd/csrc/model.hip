@@ -48,6 +48,16 @@ struct RowDev {
 enum { EOS_IGNORE = 0, EOS_STOP_DROP = 1, EOS_STOP_KEEP = 2 };
 
 constexpr int kMaxRows = 64;
+constexpr uint32_t kLoopSteps = 16;   // steps of a generation loop between two looks at its rows
+
+// A row's state as the loops' host side reads it, written into pinned host
+// memory by collect_kernel.
+struct RowReport {
+    RowDev row;
+    int32_t pos;
+    int32_t token;                // d_tokens
+    int32_t recent[kLoopSteps];   // the last min(nout, kLoopSteps) generated tokens, in order
+};
 
 }  // namespace
 
@@ -99,6 +109,11 @@ struct janus_model {
         int32_t token;
     } *h_stream = nullptr;
     hipEvent_t stream_ev[2] = {nullptr, nullptr};
+    // pinned host memory of the loops: the rows' reports and one prompt on its
+    // way to the device (prompt_busy: its copy may not have run yet)
+    RowReport *h_report = nullptr;
+    int32_t *h_prompt = nullptr;
+    bool prompt_busy = false;
     // prompt chunks (prefill_chunk): activations of up to `rows` prompt tokens,
     // allocated with the first prompt that uses them
     struct Prefill {
@@ -483,9 +498,56 @@ int upload_step(janus_model *m, const uint32_t *tokens, const uint32_t *position
     return set_rows(m, in);
 }
 
+__global__ void set_sampler_kernel(SamplerDev s, SamplerDev *out) { *out = s; }
+
 int upload_sampler(janus_model *m) {
-    JANUS_HIP_CHECK(m->ctx, hipMemcpyAsync(m->d_sampler, &m->h_sampler, sizeof(SamplerDev), hipMemcpyHostToDevice,
-                                           m->ctx->stream));
+    hipLaunchKernelGGL(set_sampler_kernel, dim3(1), dim3(1), 0, m->ctx->stream, m->h_sampler, m->d_sampler);
+    JANUS_LAUNCH_CHECK(m->ctx);
+    return JANUS_OK;
+}
+
+// One workgroup per row, a thread per token: a row's report into pinned host
+// memory. A loop's look at its rows is this launch and one wait; copies of the
+// control blocks, the positions and the tokens to pageable memory each cost a
+// host round trip of 30 to 45 us, four of them around a prompt of one chunk.
+__global__ __launch_bounds__(64) void collect_kernel(const RowDev *rows, const int32_t *pos, const int32_t *tokens,
+                                                     const int32_t *out, uint32_t max_seq, RowReport *report) {
+    const uint32_t r = blockIdx.x, t = threadIdx.x;
+    const RowDev c = rows[r];
+    const uint32_t n = min((uint32_t)c.nout, max_seq), cnt = min(n, kLoopSteps);
+    if (t < cnt) report[r].recent[t] = out[(size_t)r * max_seq + n - cnt + t];
+    if (t == 0) {
+        report[r].row = c;
+        report[r].pos = pos[r];
+        report[r].token = tokens[r];
+    }
+}
+
+// Waits for everything enqueued and reports rows 0 .. n-1 in m->h_report.
+int collect(janus_model *m, uint32_t n) {
+    janus_ctx *ctx = m->ctx;
+    if (int e = need_device(ctx)) return e;
+    DeviceGuard g(ctx->device);
+    if (n) {
+        void *d = nullptr;
+        JANUS_HIP_CHECK(ctx, hipHostGetDevicePointer(&d, m->h_report, 0));
+        hipLaunchKernelGGL(collect_kernel, dim3(n), dim3(64), 0, ctx->stream, m->d_rows, m->d_pos, m->d_tokens,
+                           m->d_out, m->cfg.max_seq_len, (RowReport *)d);
+        JANUS_LAUNCH_CHECK(ctx);
+    }
+    JANUS_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    m->prompt_busy = false;
+    return JANUS_OK;
+}
+
+// Enqueues the copy of a prompt (n <= max_seq_len) to d_prompts[slot].
+int upload_prompt(janus_model *m, uint32_t slot, const uint32_t *prompt, uint32_t n) {
+    janus_ctx *ctx = m->ctx;
+    if (m->prompt_busy) JANUS_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));   // the prompt before this one
+    std::memcpy(m->h_prompt, prompt, (size_t)n * 4);
+    m->prompt_busy = true;
+    JANUS_HIP_CHECK(ctx, hipMemcpyAsync(m->d_prompts + (size_t)slot * m->cfg.max_seq_len, m->h_prompt, (size_t)n * 4,
+                                        hipMemcpyHostToDevice, ctx->stream));
     return JANUS_OK;
 }
 
@@ -761,14 +823,10 @@ int check_request(janus_model *m, const Request &q) {
 // Puts request q into row r of `in`: its prompt copied to the device and put
 // through the layers in chunks where that pays, its occurrence counts cleared,
 // its next token and position in KV slot r.
-int admit_row(janus_model *m, uint32_t r, const Request &q, uint32_t max_tokens, int eos_mode, RowInit &in,
-              std::vector<int32_t> &tmp) {
+int admit_row(janus_model *m, uint32_t r, const Request &q, uint32_t max_tokens, int eos_mode, RowInit &in) {
     janus_ctx *ctx = m->ctx;
     const janus_model_config &c = m->cfg;
-    tmp.assign(q.prompt, q.prompt + q.n);
-    JANUS_HIP_CHECK(ctx, hipMemcpyAsync(m->d_prompts + (size_t)r * c.max_seq_len, tmp.data(), q.n * 4,
-                                        hipMemcpyHostToDevice, ctx->stream));
-    JANUS_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));   // tmp is reused
+    if (int e = upload_prompt(m, r, q.prompt, q.n)) return e;
     JANUS_HIP_CHECK(ctx, hipMemsetAsync(m->d_counts + (size_t)r * c.vocab, 0, (size_t)c.vocab * 4, ctx->stream));
     // the whole prompt when a position is left for the re-fed last token (which
     // the row then starts with), else all but the last prompt token
@@ -802,7 +860,7 @@ int run_requests(janus_model *m, const std::vector<Request> &reqs, uint32_t max_
     std::vector<uint8_t> parked(B, 0);
     std::vector<RowDev> hrows(B);
     std::vector<int32_t> hpos(B, 0);
-    std::vector<int32_t> tmp;
+    std::vector<std::vector<int32_t>> made(B);   // the rows' tokens so far
     size_t next_req = 0;
     for (;;) {
         // admission: free rows take the next requests
@@ -814,7 +872,8 @@ int run_requests(janus_model *m, const std::vector<Request> &reqs, uint32_t max_
             if (row_req[r] >= 0) continue;
             row_req[r] = (int)next_req;
             parked[r] = 0;
-            if (int e = admit_row(m, r, reqs[next_req++], max_tokens, eos_mode, in, tmp)) return e;
+            if (int e = admit_row(m, r, reqs[next_req++], max_tokens, eos_mode, in)) return e;
+            made[r].clear();
             hrows[r] = in.ctl[r];
             hpos[r] = in.pos[r];
             any_new = true;
@@ -841,7 +900,7 @@ int run_requests(janus_model *m, const std::vector<Request> &reqs, uint32_t max_
             if (int e = set_rows(m, in)) return e;
         // steps until the first row can be done without an EOS: its prompt,
         // its tokens, or its capacity
-        uint32_t k = 16;
+        uint32_t k = kLoopSteps;
         for (uint32_t r = 0; r < nrows; ++r) {
             if (row_req[r] < 0 || hrows[r].done) continue;
             const int64_t left_prompt = hrows[r].prompt_len - hpos[r];   // steps still prefilling
@@ -855,22 +914,24 @@ int run_requests(janus_model *m, const std::vector<Request> &reqs, uint32_t max_
         int32_t top = 0;
         for (uint32_t r = 0; r < nrows; ++r) top = hpos[r] > top ? hpos[r] : top;
         if (int e = replay(m, nrows, k, (uint32_t)top + 1)) return e;
-        JANUS_HIP_CHECK(ctx, hipMemcpyAsync(hrows.data(), m->d_rows, nrows * sizeof(RowDev), hipMemcpyDeviceToHost,
-                                            ctx->stream));
-        JANUS_HIP_CHECK(ctx, hipMemcpyAsync(hpos.data(), m->d_pos, nrows * 4, hipMemcpyDeviceToHost, ctx->stream));
-        JANUS_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+        if (int e = collect(m, nrows)) return e;
+        for (uint32_t r = 0; r < nrows; ++r) {
+            const RowReport &t = m->h_report[r];
+            // the k <= kLoopSteps steps added at most the tokens of the report
+            const int32_t have = t.row.nout < (int32_t)kLoopSteps ? t.row.nout : (int32_t)kLoopSteps;
+            const int32_t add = t.row.nout - hrows[r].nout;
+            if (add > 0 && add <= have) made[r].insert(made[r].end(), t.recent + have - add, t.recent + have);
+            hrows[r] = t.row;
+            hpos[r] = t.pos;
+        }
         for (uint32_t r = 0; r < nrows; ++r)
             if (row_req[r] >= 0 && hrows[r].nan) return nan_fail(ctx, r);
         // retirement: finished rows hand back their tokens and free the row
         for (uint32_t r = 0; r < nrows; ++r) {
             if (row_req[r] < 0 || !hrows[r].done) continue;
             const int i = row_req[r];
-            const uint32_t n = (uint32_t)hrows[r].nout < max_tokens ? (uint32_t)hrows[r].nout : max_tokens;
-            tmp.resize(n ? n : 1);
-            if (n)
-                JANUS_HIP_CHECK(ctx, hipMemcpy(tmp.data(), m->d_out + (size_t)r * c.max_seq_len, n * 4,
-                                               hipMemcpyDeviceToHost));
-            for (uint32_t t = 0; t < n; ++t) out_tokens[(size_t)i * max_tokens + t] = (uint32_t)tmp[t];
+            const uint32_t n = made[r].size() < max_tokens ? (uint32_t)made[r].size() : max_tokens;
+            for (uint32_t t = 0; t < n; ++t) out_tokens[(size_t)i * max_tokens + t] = (uint32_t)made[r][t];
             n_out[i] = n;
             row_req[r] = -1;
         }
@@ -899,8 +960,7 @@ int run_stream(janus_model *m, const Request &q, uint32_t max_tokens, janus_toke
     RowInit in;
     std::memset(&in, 0, sizeof(in));
     in.set_ctl = 1;
-    std::vector<int32_t> tmp;
-    if (int e = admit_row(m, 0, q, max_tokens, EOS_STOP_DROP, in, tmp)) return e;
+    if (int e = admit_row(m, 0, q, max_tokens, EOS_STOP_DROP, in)) return e;
     if (int e = set_rows(m, in)) return e;
     // every bucket the request can reach, captured before the first step so
     // that no capture stalls the stream of tokens
@@ -995,7 +1055,9 @@ int janus_model_create(janus_ctx *ctx, const janus_model_config *cfg, janus_mode
               alloc((void **)&m->d_rowbase, kMaxRows * 4) && alloc((void **)&m->d_rows, kMaxRows * sizeof(RowDev)) &&
               alloc((void **)&m->d_prompts, B * S * 4) && alloc((void **)&m->d_out, B * S * 4) &&
               alloc((void **)&m->d_counts, B * c.vocab * 4) && alloc((void **)&m->d_best, kMaxRows * 8) &&
-              alloc((void **)&m->d_sampler, sizeof(SamplerDev));
+              alloc((void **)&m->d_sampler, sizeof(SamplerDev)) &&
+              hipHostMalloc((void **)&m->h_report, kMaxRows * sizeof(RowReport), hipHostMallocDefault) == hipSuccess &&
+              hipHostMalloc((void **)&m->h_prompt, S * 4, hipHostMallocDefault) == hipSuccess;
     ok = ok && hipMemset(m->d_best, 0, kMaxRows * 8) == hipSuccess &&
          hipMemset(m->d_rows, 0, kMaxRows * sizeof(RowDev)) == hipSuccess &&
          hipMemset(m->d_counts, 0, B * c.vocab * 4) == hipSuccess &&
@@ -1045,6 +1107,8 @@ void janus_model_destroy(janus_model *m) {
     for (hipEvent_t ev : m->stream_ev)
         if (ev) (void)hipEventDestroy(ev);
     if (m->h_stream) (void)hipHostFree(m->h_stream);
+    if (m->h_report) (void)hipHostFree(m->h_report);
+    if (m->h_prompt) (void)hipHostFree(m->h_prompt);
     prefill_free(m);
     for (auto &L : m->layers) {
         for (janus_weight *w : {L.q, L.k, L.v, L.o, L.gate, L.up, L.down, L.qkv, L.gu}) janus_weight_free(m->ctx, w);
@@ -1246,10 +1310,7 @@ int janus_model_generate(janus_model *m, const uint32_t *prompt, uint32_t n_prom
         uint32_t done = 0;
         if (n_prompt > kPrefillMin && janus_model_validate(m) == JANUS_OK &&
             check_request(m, Request{prompt, n_prompt}) == JANUS_OK) {
-            std::vector<int32_t> ids(prompt, prompt + n_prompt);
-            JANUS_HIP_CHECK(m->ctx, hipMemcpyAsync(m->d_prompts, ids.data(), (size_t)n_prompt * 4, hipMemcpyHostToDevice,
-                                                   m->ctx->stream));
-            JANUS_HIP_CHECK(m->ctx, hipStreamSynchronize(m->ctx->stream));   // ids goes out of scope
+            if (int e = upload_prompt(m, 0, prompt, n_prompt)) return e;
             m->graph_nseq = 0;   // d_prompts no longer holds a running loop's prompt
             if (int e = prefill(m, 0, n_prompt - 1, &done)) return e;
         }
@@ -1344,16 +1405,17 @@ int janus_model_graph_run(janus_model *m, uint32_t steps) {
     if (int e = replay(m, n, steps, top + 1)) return e;
     for (auto &p : m->h_pos) p += steps;
     // a row whose step met NaN logits is stopped on the device; report it
-    RowDev rows[kMaxRows];
-    if (int e = janus_d2h(m->ctx, rows, m->d_rows, (size_t)n * sizeof(RowDev))) return e;
+    if (int e = collect(m, n)) return e;
     for (uint32_t r = 0; r < n; ++r)
-        if (rows[r].nan) return nan_fail(m->ctx, r);
+        if (m->h_report[r].row.nan) return nan_fail(m->ctx, r);
     return JANUS_OK;
 }
 
 int janus_model_graph_read_tokens(janus_model *m, uint32_t *h_tokens, uint32_t nseq) {
     if (!m || !h_tokens || nseq > m->cfg.max_batch) return JANUS_E_INVALID_ARG;
-    return janus_d2h(m->ctx, h_tokens, m->d_tokens, (size_t)nseq * 4);
+    if (int e = collect(m, nseq)) return e;
+    for (uint32_t r = 0; r < nseq; ++r) h_tokens[r] = (uint32_t)m->h_report[r].token;
+    return JANUS_OK;
 }
 
 int janus_model_read_generated(janus_model *m, uint32_t row, uint32_t *h_tokens, uint32_t cap, uint32_t *n) {

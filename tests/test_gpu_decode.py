@@ -501,3 +501,19 @@ def test_prompt_attention_head_layouts(engine, act, heads, kv_heads, hd):
         for x, r in zip(kv, rows):
             assert float((x[:, :n].double() - r).norm() / r.norm()) <= tol, n
     m.close()
+
+
+@pytest.mark.parametrize("count", [1, 15, 16, 17, 33])
+def test_loops_hand_over_every_token_at_chunk_edges(engine, count):
+    """Token counts around the 16 steps between two looks at the rows: the
+    tokens generate collects per look, those of five requests over three rows
+    (prompts of several requests staged in one round), and those of the
+    captured loop's reads, against the streaming loop's one token per step."""
+    s = _prompt_model(synth.Q4_0)
+    m = Model(engine, s, max_seq_len=90, max_batch=3)
+    prompts = [_prompt(80 + n, n, s.vocab) for n in (3, 40, 1, 21, 70)]
+    want = [m.generate_with_callback(p, count) for p in prompts]
+    assert [m.generate(p, count) for p in prompts] == want
+    assert m.generate_batch(prompts, count) == want
+    assert [len(w) for w in want] == [min(count, 90 - len(p)) for p in prompts]
+    m.close()
