@@ -17,6 +17,11 @@
 //    MfmaAttn), P into hi + lo parts of 2^14 p (22 bits, as in
 //    attn_rows_kernel); V is transposed on its way into LDS.
 //  * binary32 caches: v_mfma_f32_32x32x2_f32, nothing split or rounded.
+//
+// Bound by the longest row tile's chain of K/V tiles (a 512-row chunk is 128
+// workgroups of four heads, so CUs are idle): 33 us for 512 binary16 rows at
+// 32/8/128 heads against 160 through the decode kernels, 25 us for 133
+// binary32 rows at 32/32/128.
 #include <type_traits>
 
 #include "internal.h"
@@ -58,6 +63,50 @@ template <int D> struct Tile<float, D> {
     static constexpr uint32_t K = PT * KP * 4, BYTES = K + PT * VP * 4;
     static constexpr int SEG = 4;
 };
+
+// The positions of a V tile (bit i: position i) that hold an infinity or NaN
+// in some dim.
+template <typename KV, int D>
+__device__ __forceinline__ uint32_t nonfinite_positions(const unsigned char *vt, int lane) {
+    typedef Tile<KV, D> T;
+    uint32_t bad = 0;
+    if constexpr (std::is_same<KV, _Float16>::value) {
+#pragma unroll 1
+        for (int i = 0; i < D / 64; ++i)   // dim lane + 64 i, 4 positions at a time
+#pragma unroll 2
+            for (int j = 0; j < PT / 4; ++j) {
+                const uint2 v = *(const uint2 *)(vt + ((size_t)(lane + 64 * i) * T::VP + 4 * j) * 2);
+                const uint32_t b = (uint32_t)((v.x & 0x7c00u) == 0x7c00u) | (uint32_t)((v.x & 0x7c000000u) == 0x7c000000u) << 1 |
+                                   (uint32_t)((v.y & 0x7c00u) == 0x7c00u) << 2 | (uint32_t)((v.y & 0x7c000000u) == 0x7c000000u) << 3;
+                bad |= b << (4 * j);
+            }
+    } else {
+#pragma unroll 2
+        for (int i = 0; i < PT * D / 256; ++i) {   // 16-byte segments, whole rows of D
+            const ju4 v = *(const ju4 *)(vt + (size_t)(i * 64 + lane) * 16);
+            bool b = false;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) b = b || (v[k] & 0x7f800000u) == 0x7f800000u;
+            bad |= (uint32_t)b << ((i * 64 + lane) / (D / 4));
+        }
+    }
+    if (!__any(bad != 0)) return 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) bad |= (uint32_t)__shfl_xor((int)bad, o, 64);
+    return __builtin_amdgcn_readfirstlane(bad);
+}
+
+// The finite values of 8 binary16, others as 0.
+__device__ __forceinline__ ph8 finite_only(ph8 x) {
+    const uint4 v = __builtin_bit_cast(uint4, x);
+    uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if ((u[i] & 0x7c00u) == 0x7c00u) u[i] &= 0xffff0000u;
+        if ((u[i] & 0x7c000000u) == 0x7c000000u) u[i] &= 0xffffu;
+    }
+    return __builtin_bit_cast(ph8, make_uint4(u[0], u[1], u[2], u[3]));
+}
 
 // HW: heads of a KV head that a workgroup's wavefronts take (1, 2 or 4); the
 // other factor of 4 is row tiles.
@@ -238,6 +287,17 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
                 for (int d = 0; d < ND; ++d)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+            // A probability of 0 does not mask an infinity or NaN of V. Where some
+            // query does not see all positions of the tile (the last tile or two
+            // of a wavefront), such values are kept out of the MFMAs and the
+            // queries that see them become NaN (about 5 us of a 580 us prompt of
+            // 512 tokens).
+            uint32_t bad = 0;
+            if (p + PT > a.p0 + q0 + 1) {
+                bad = nonfinite_positions<KV, D>(vt, lane);
+                const uint32_t seen = my_end - min(my_end, p);
+                if (bad & (seen >= 32 ? ~0u : (1u << seen) - 1u)) l = NAN;
+            }
             if constexpr (F16) {
                 // 16 positions per step: half h holds 4 h + 0..3 and 8 + 4 h + 0..3 of them
 #pragma unroll
@@ -254,7 +314,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
                     for (int d = 0; d < ND; ++d) {
                         const unsigned char *vp = vt + ((size_t)(32 * d + col) * T::VP + 16 * t + 4 * h) * 2;
                         const uint2 v0 = *(const uint2 *)vp, v1 = *(const uint2 *)(vp + 16);
-                        const ph8 v = __builtin_bit_cast(ph8, make_uint4(v0.x, v0.y, v1.x, v1.y));
+                        ph8 v = __builtin_bit_cast(ph8, make_uint4(v0.x, v0.y, v1.x, v1.y));
+                        if (bad) v = finite_only(v);
                         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, lo, o[d], 0, 0, 0);
                         o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, hi, o[d], 0, 0, 0);
                     }
@@ -265,7 +326,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
                 for (int v = 0; v < 16; ++v)
 #pragma unroll
                     for (int d = 0; d < ND; ++d) {
-                        const float x = *(const float *)(vt + ((size_t)(8 * (v >> 2) + 4 * h + (v & 3)) * T::VP + 32 * d + col) * 4);
+                        float x = *(const float *)(vt + ((size_t)(8 * (v >> 2) + 4 * h + (v & 3)) * T::VP + 32 * d + col) * 4);
+                        if (bad && (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u) x = 0.0f;
                         o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, s[v], o[d], 0, 0, 0);
                     }
             }
@@ -275,7 +337,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
     }
     if (q0 + col >= a.n) return;
     float lt = l + swap32(l);
-    const float inv = (F16 ? 1.0f / 16384.0f : 1.0f) / fmaxf(lt, 1e-20f);
+    const float inv = (F16 ? 1.0f / 16384.0f : 1.0f) / (lt < 1e-20f ? 1e-20f : lt);   // a NaN stays
     const size_t at = ((size_t)(q0 + col) * a.heads + head) * D + 4 * h;
 #pragma unroll
     for (int d = 0; d < ND; ++d)

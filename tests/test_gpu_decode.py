@@ -517,3 +517,46 @@ def test_loops_hand_over_every_token_at_chunk_edges(engine, count):
     assert m.generate_batch(prompts, count) == want
     assert [len(w) for w in want] == [min(count, 90 - len(p)) for p in prompts]
     m.close()
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", [(4, 1, 128), (4, 4, 128), (8, 2, 64), (2, 2, 64)])
+def test_an_overflowed_value_reaches_only_the_rows_that_see_it(engine, heads, kv_heads, hd):
+    """A prompt token whose V overflows binary16: the rows before it keep the
+    K/V of token-by-token steps (one binary16 rounding per value, as in
+    test_prompt_chunks_match_token_by_token), also those of its own 32-row
+    tile, and the same rows are not finite from it on."""
+    hidden, vocab, n, bad = heads * hd, 300, 60, 37
+    s = synth.make_model(95, hidden, heads, kv_heads, 256, vocab, 2, synth.F16, 1e-5, 10000.0, embed_type=synth.F16,
+                         head_type=synth.F16)
+    rng = np.random.default_rng(96)
+    emb = rng.standard_normal((vocab, hidden), dtype=np.float32)
+    emb[:, 0] = 0
+    emb[7] = 0
+    emb[7, 0] = 8   # token 7 alone has feature 0, which layer 0's V takes times 60000
+    v = rng.standard_normal((kv_heads * hd, hidden), dtype=np.float32) * np.float32(0.02)
+    v[:, 0] = 60000
+    for t in s.tensors:
+        if t.name == "token_embd.weight":
+            t.data = synth.f16_bits(emb)
+        elif t.name == "blk.0.attn_v.weight":
+            t.data = synth.f16_bits(v)
+    prompt = [8 + p * 5 % 290 for p in range(n)]
+    prompt[bad] = 7
+    caches = []
+    for chunked in (False, True):
+        m = Model(engine, s, max_seq_len=64, kv_dtype=_lib.DT_F16)
+        kv = [torch.zeros(2, 64, kv_heads, hd, dtype=torch.float16, device=DEV) for _ in range(2)]
+        m.set_kv_cache(*kv)
+        if chunked:
+            m.generate(prompt, 0)
+        else:
+            for p, t in enumerate(prompt):
+                m.forward([t], [p])
+        torch.cuda.synchronize()
+        caches.append([x.double() for x in kv])
+        m.close()
+    for r, x in zip(*caches):
+        assert torch.equal(r[:, :n].isfinite().all(-1), x[:, :n].isfinite().all(-1))
+        assert bool(x[:, :bad].isfinite().all())
+        assert float((x[:, :bad] - r[:, :bad]).norm() / r[:, :bad].norm()) <= 2e-3
+    assert not bool(caches[1][1][0, bad].isfinite().any())
