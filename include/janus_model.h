@@ -74,7 +74,7 @@ const float *janus_model_logits(const janus_model *m);        /* device pointer 
 void *janus_model_kv_cache(const janus_model *m, int which);  /* 0 = K, 1 = V; [layers][rows][kvh][hd] */
 int janus_model_read_logits(janus_model *m, float *h_out, uint32_t nseq);
 /* Greedy generation with the reference's loop semantics (generation.rs:129-323):
- * prefill token by token, then re-feed the last prompt token at position n
+ * prefill (in chunks of up to 512 tokens), then re-feed the last prompt token at position n
  * and sample as Sampler::sample does with temperature 0 (model/sampler.rs:
  * 146-209): with |repetition_penalty - 1| < 0.01 the GPU argmax and its tie
  * rule (shaders/argmax.wgsl:26-126), otherwise the penalty over the generated
@@ -112,7 +112,7 @@ int janus_model_generate_stream(janus_model *m, const uint32_t *prompt, uint32_t
 /* Model::generate_batch (generation.rs:673-870) with continuous batching:
  * request i is prompt_lens[i] token ids, the prompts back to back in
  * `prompts`. Up to max_batch requests run at once, each in its own KV slot
- * and at its own position (prefill token by token, then the re-fed last
+ * and at its own position (prefill in chunks, then the re-fed last
  * prompt token, then decode). A request leaves when it has max_tokens
  * tokens, hits 128001/128009 (kept in its output, as the reference pushes
  * it before the check, generation.rs:810-833) or fills max_seq_len, and a

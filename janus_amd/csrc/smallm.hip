@@ -1,5 +1,5 @@
-// smallm.hip -- products with 2..64 activation rows (ragged decode batches):
-// the dequant-fused MFMA GEMM, on binary16 activations or on binary32 ones
+// smallm.hip -- products with 2..64 activation rows (ragged decode batches)
+// and with any number of them (prompt chunks): the dequant-fused MFMA GEMM, on binary16 activations or on binary32 ones
 // split into three bfloat16 parts.
 //
 // Replaces the reference's M>1 quantised path, which hands quantised bytes
