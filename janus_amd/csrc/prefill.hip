@@ -51,49 +51,28 @@ __device__ __forceinline__ float swap32(float v) {   // value of lane ^ 32
 
 // LDS of one K/V tile. binary16: K rows padded to D + 8 halves; V transposed,
 // [dim][position] rows padded to PT + 4 halves (8-byte reads of 4 positions).
-// binary32: K rows padded to D + 4 floats, V rows as they are.
+// binary32: K rows padded to D + 4 floats, V rows as they are. Behind them one
+// word per wavefront: whether it stored an infinity or NaN of V.
 template <typename KV, int D> struct Tile;
 template <int D> struct Tile<_Float16, D> {
     static constexpr int KP = D + 8, VP = PT + 4;
-    static constexpr uint32_t K = PT * KP * 2, BYTES = K + D * VP * 2;
+    static constexpr uint32_t K = PT * KP * 2, FLAGS = K + D * VP * 2, BYTES = FLAGS + 16;
     static constexpr int SEG = 8;   // elements of a 16-byte segment
 };
 template <int D> struct Tile<float, D> {
     static constexpr int KP = D + 4, VP = D;
-    static constexpr uint32_t K = PT * KP * 4, BYTES = K + PT * VP * 4;
+    static constexpr uint32_t K = PT * KP * 4, FLAGS = K + PT * VP * 4, BYTES = FLAGS + 16;
     static constexpr int SEG = 4;
 };
 
-// The positions of a V tile (bit i: position i) that hold an infinity or NaN
-// in some dim.
-template <typename KV, int D>
-__device__ __forceinline__ uint32_t nonfinite_positions(const unsigned char *vt, int lane) {
-    typedef Tile<KV, D> T;
-    uint32_t bad = 0;
-    if constexpr (std::is_same<KV, _Float16>::value) {
-#pragma unroll 1
-        for (int i = 0; i < D / 64; ++i)   // dim lane + 64 i, 4 positions at a time
-#pragma unroll 2
-            for (int j = 0; j < PT / 4; ++j) {
-                const uint2 v = *(const uint2 *)(vt + ((size_t)(lane + 64 * i) * T::VP + 4 * j) * 2);
-                const uint32_t b = (uint32_t)((v.x & 0x7c00u) == 0x7c00u) | (uint32_t)((v.x & 0x7c000000u) == 0x7c000000u) << 1 |
-                                   (uint32_t)((v.y & 0x7c00u) == 0x7c00u) << 2 | (uint32_t)((v.y & 0x7c000000u) == 0x7c000000u) << 3;
-                bad |= b << (4 * j);
-            }
-    } else {
-#pragma unroll 2
-        for (int i = 0; i < PT * D / 256; ++i) {   // 16-byte segments, whole rows of D
-            const ju4 v = *(const ju4 *)(vt + (size_t)(i * 64 + lane) * 16);
-            bool b = false;
+// Whether the 16 bytes hold an infinity or NaN.
+template <typename KV> __device__ __forceinline__ bool nonfinite(const ju4 &v) {
+    uint32_t b = 0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) b = b || (v[k] & 0x7f800000u) == 0x7f800000u;
-            bad |= (uint32_t)b << ((i * 64 + lane) / (D / 4));
-        }
-    }
-    if (!__any(bad != 0)) return 0;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) bad |= (uint32_t)__shfl_xor((int)bad, o, 64);
-    return __builtin_amdgcn_readfirstlane(bad);
+    for (int i = 0; i < 4; ++i)
+        // adding one to an exponent of all ones carries into the sign's place
+        b |= std::is_same<KV, _Float16>::value ? (v[i] & 0x7c007c00u) + 0x04000400u : (v[i] & 0x7f800000u) + 0x00800000u;
+    return (b & (std::is_same<KV, _Float16>::value ? 0x80008000u : 0x80000000u)) != 0;
 }
 
 // The finite values of 8 binary16, others as 0.
@@ -106,6 +85,34 @@ __device__ __forceinline__ ph8 finite_only(ph8 x) {
         if ((u[i] & 0x7c000000u) == 0x7c000000u) u[i] &= 0xffffu;
     }
     return __builtin_bit_cast(ph8, make_uint4(u[0], u[1], u[2], u[3]));
+}
+
+// o[d] += p * V over the infinities and NaN of a V tile (the products left them
+// out): position j of the tile for the queries that see it (j < seen), so they
+// reach the dims that hold them and no other row or dim. s: probabilities of
+// the lane's positions. A tile that holds none does not come here.
+template <typename KV, int D>
+__device__ __forceinline__ void add_nonfinite(const unsigned char *vt, const pf16 &s, uint32_t seen, int h,
+                                              pf16 (&o)[D / 32]) {
+    typedef Tile<KV, D> T;
+#pragma unroll 1
+    for (uint32_t j = 0; j < PT; ++j) {
+        const int at = (int)(j >> 3) * 4 + (int)(j & 3);   // position j is s[at] of half (j / 4) % 2
+        float mine = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) mine = v == at ? s[v] : mine;
+        const float other = swap32(mine), p = (int)((j >> 2) & 1) == h ? mine : other;
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const uint32_t dim = 32 * d + 8 * (v >> 2) + 4 * h + (v & 3);
+                float x;
+                if constexpr (std::is_same<KV, _Float16>::value) x = (float)((const _Float16 *)vt)[dim * T::VP + j];
+                else x = ((const float *)vt)[j * T::VP + dim];
+                if (j < seen && (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u) o[d][v] = fmaf(p, x, o[d][v]);
+            }
+    }
 }
 
 // HW: heads of a KV head that a workgroup's wavefronts take (1, 2 or 4); the
@@ -155,6 +162,11 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         }
     };
     auto store = [&](unsigned char *t) {
+        bool odd = false;
+#pragma unroll
+        for (int j = 0; j < LD; ++j) odd = odd || nonfinite<KV>(vr[j]);
+        const bool any = __any(odd);
+        if (lane == 0) *(uint32_t *)(t + T::FLAGS + 4 * wave) = any;
 #pragma unroll
         for (int j = 0; j < LD; ++j)
             *(ju4 *)(t + ((size_t)row_of(j, false) * T::KP + seg_of(j, false) * SEG) * sizeof(KV)) = kr[j];
@@ -287,17 +299,12 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
                 for (int d = 0; d < ND; ++d)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
-            // A probability of 0 does not mask an infinity or NaN of V. Where some
-            // query does not see all positions of the tile (the last tile or two
-            // of a wavefront), such values are kept out of the MFMAs and the
-            // queries that see them become NaN (about 5 us of a 580 us prompt of
-            // 512 tokens).
-            uint32_t bad = 0;
-            if (p + PT > a.p0 + q0 + 1) {
-                bad = nonfinite_positions<KV, D>(vt, lane);
-                const uint32_t seen = my_end - min(my_end, p);
-                if (bad & (seen >= 32 ? ~0u : (1u << seen) - 1u)) l = NAN;
-            }
+            // A probability of 0 does not mask an infinity or NaN of V, and one
+            // split into parts turns an infinity into a NaN: such values stay
+            // out of the MFMAs and are added on their own. They are noticed as
+            // the tile is stored (about a dozen instructions per 16 bytes).
+            const uint4 f = *(const uint4 *)(kt + T::FLAGS);
+            const uint32_t bad = __builtin_amdgcn_readfirstlane(f.x | f.y | f.z | f.w);
             if constexpr (F16) {
                 // 16 positions per step: half h holds 4 h + 0..3 and 8 + 4 h + 0..3 of them
 #pragma unroll
@@ -331,6 +338,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
                         o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, s[v], o[d], 0, 0, 0);
                     }
             }
+            if (bad) add_nonfinite<KV, D>(vt, s, my_end - min(my_end, p), h, o);
         }
         buf ^= 1u;
         store(smem + buf * T::BYTES);   // last read before the barrier above
