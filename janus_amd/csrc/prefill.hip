@@ -242,6 +242,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] = (pf16){};
     float m = -INFINITY, l = 0.0f;
+    bool lost = false;
     const uint32_t my_end = a.p0 + q0 + col + 1;                         // this lane's query sees [0, my_end)
     const uint32_t wave_end = q0 < a.n ? a.p0 + min(q0 + QT, a.n) : 0;   // uniform
 
@@ -286,6 +287,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
             bm = fmaxf(bm, swap32(bm));
             const float mn = fmaxf(m, bm);
             const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            // the maxima pass over a NaN: while there is no other score, it is kept here
+            if (__any(mn == -INFINITY) && mn == -INFINITY)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) lost = lost || s[v] != s[v];
             float sum = 0.0f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
@@ -344,6 +349,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         store(smem + buf * T::BYTES);   // last read before the barrier above
     }
     if (q0 + col >= a.n) return;
+    // a row whose scores are all NaN stays 0, as in the decode kernels
+    const float other = swap32(lost ? 1.0f : 0.0f);
+    if ((lost || other != 0.0f) && m != -INFINITY) l = NAN;
     float lt = l + swap32(l);
     const float inv = (F16 ? 1.0f / 16384.0f : 1.0f) / (lt < 1e-20f ? 1e-20f : lt);   // a NaN stays
     const size_t at = ((size_t)(q0 + col) * a.heads + head) * D + 4 * h;

@@ -85,3 +85,25 @@ def test_nonfinite_values_reach_their_dim_of_the_rows_that_see_them(engine, head
         v[p0 + 37, kv_heads - 1, hd - 1] = float("nan")
         v[p0 + n - 1, 0, 9] = float("inf")
         _same_where_finite(_prompt_attention(engine, q, k, v, p0), _exact(q, k, v, p0))
+
+
+@pytest.mark.parametrize("kv", [torch.float16, torch.float32])
+@pytest.mark.parametrize("heads,kv_heads,hd", LAYOUTS)
+def test_nan_scores_are_not_passed_over(engine, heads, kv_heads, hd, kv):
+    """NaN in K rows with V finite. One such row: NaN from its position on.
+    The whole first tile: NaN for every later row, whose other scores are
+    finite. Rows without any other score (also a NaN q) are what the decode
+    kernels make of them."""
+    n, rep = 75, heads // kv_heads
+    q, k, v = _inputs(1, n, 0, heads, kv_heads, hd, kv)
+    k[2, 0, 1] = float("nan")
+    _same_where_finite(_prompt_attention(engine, q, k, v, 0), _exact(q, k, v, 0))
+    k[:32, 0] = float("nan")
+    got, one = _prompt_attention(engine, q, k, v, 0), _decode_attention(engine, q, k, v, 0)
+    assert bool(got[32:, :rep].isnan().all()) and bool(got[:, rep:].isfinite().all())
+    assert torch.equal(got[:32, :rep], one[:32, :rep])
+    q, k, v = _inputs(1, n, 0, heads, kv_heads, hd, kv)
+    want = _prompt_attention(engine, q, k, v, 0)
+    q[70, heads - 1] = float("nan")
+    want[70, heads - 1] = _decode_attention(engine, q, k, v, 0)[70, heads - 1]
+    assert torch.equal(_prompt_attention(engine, q, k, v, 0), want)
