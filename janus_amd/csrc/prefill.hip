@@ -52,7 +52,8 @@ __device__ __forceinline__ float swap32(float v) {   // value of lane ^ 32
 // LDS of one K/V tile. binary16: K rows padded to D + 8 halves; V transposed,
 // [dim][position] rows padded to PT + 4 halves (8-byte reads of 4 positions).
 // binary32: K rows padded to D + 4 floats, V rows as they are. Behind them one
-// word per wavefront: whether it stored an infinity or NaN of V.
+// word per wavefront: whether it stored an infinity or NaN of V (bit 0) and of
+// K (bit 1).
 template <typename KV, int D> struct Tile;
 template <int D> struct Tile<_Float16, D> {
     static constexpr int KP = D + 8, VP = PT + 4;
@@ -115,6 +116,22 @@ __device__ __forceinline__ void add_nonfinite(const unsigned char *vt, const pf1
     }
 }
 
+// The scores of a tile with q in one piece: s[v] = qs * (q . K row of the
+// lane's position v), 8 (v / 4) + 4 h + v % 4.
+template <int D>
+__device__ __forceinline__ void whole_scores(const unsigned char *kt, const float *q, float qs, int h, pf16 &s) {
+    s = (pf16){};
+#pragma unroll 1
+    for (int d = 0; d < D; ++d) {
+        const float x = q[d];
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+            s[v] = fmaf(x, (float)((const _Float16 *)kt)[(8 * (v >> 2) + 4 * h + (v & 3)) * Tile<_Float16, D>::KP + d], s[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] *= qs;
+}
+
 // HW: heads of a KV head that a workgroup's wavefronts take (1, 2 or 4); the
 // other factor of 4 is row tiles.
 template <typename KV, int D, int HW>
@@ -162,10 +179,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         }
     };
     auto store = [&](unsigned char *t) {
-        bool odd = false;
+        bool oddv = false, oddk = false;
 #pragma unroll
-        for (int j = 0; j < LD; ++j) odd = odd || nonfinite<KV>(vr[j]);
-        const bool any = __any(odd);
+        for (int j = 0; j < LD; ++j) {
+            oddv = oddv || nonfinite<KV>(vr[j]);
+            if (F16) oddk = oddk || nonfinite<KV>(kr[j]);
+        }
+        const uint32_t any = (uint32_t)(__any(oddv) != 0) | (uint32_t)(__any(oddk) != 0) << 1;
         if (lane == 0) *(uint32_t *)(t + T::FLAGS + 4 * wave) = any;
 #pragma unroll
         for (int j = 0; j < LD; ++j)
@@ -201,7 +221,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
     // 16-wide step as three parts; binary32: dims 8 s + 4 h + 0..3
     const uint32_t qi = min(q0 + col, a.n - 1);
     const float *qp = a.q + ((size_t)qi * a.heads + head) * D;
-    float sc2 = a.scale2;
+    float sc2 = a.scale2, qs = 1.0f;   // q's parts are those of q * qs
+    bool q_inf = false;
     ph8 qh[F16 ? D / 16 : 1], qm[F16 ? D / 16 : 1], ql[F16 ? D / 16 : 1];
     jf4 qf[F16 ? 1 : D / 8];
     if constexpr (F16) {
@@ -216,7 +237,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         int qe = 0;
         (void)frexpf(qmax, &qe);                  // qmax < 2^qe
         const int sh = qe > 15 ? qe - 15 : 0;     // |q| 2^-sh < 2^15
-        const float qs = ldexpf(1.0f, -sh);
+        qs = ldexpf(1.0f, -sh);
+        q_inf = __any(qmax == INFINITY);
         sc2 *= ldexpf(1.0f, sh);
         asm volatile("" : "+v"(qp));   // q is read again (from cache) rather than held beside its parts
 #pragma unroll
@@ -253,6 +275,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         __syncthreads();
         const unsigned char *kt = smem + buf * T::BYTES, *vt = kt + T::K;
         if (p < wave_end) {
+            const uint4 f = *(const uint4 *)(kt + T::FLAGS);
+            const uint32_t flags = __builtin_amdgcn_readfirstlane(f.x | f.y | f.z | f.w);
             // two chains, so that an MFMA need not wait for the one before it
             pf16 s = (pf16){}, s2 = (pf16){};
             if constexpr (F16) {
@@ -276,6 +300,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
             }
 #pragma unroll
             for (int v = 0; v < 16; ++v) s[v] += s2[v];
+            // An infinity times a part of q that is 0 or of the other sign would
+            // make a NaN of an infinite score: such tiles take q whole.
+            if (F16 && (q_inf || (flags & 2u))) whole_scores<D>(kt, qp, qs, h, s);
             // s[4 j + i]: position p + 8 j + 4 h + i
             float bm = -INFINITY;
 #pragma unroll
@@ -308,8 +335,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
             // split into parts turns an infinity into a NaN: such values stay
             // out of the MFMAs and are added on their own. They are noticed as
             // the tile is stored (about a dozen instructions per 16 bytes).
-            const uint4 f = *(const uint4 *)(kt + T::FLAGS);
-            const uint32_t bad = __builtin_amdgcn_readfirstlane(f.x | f.y | f.z | f.w);
+            const bool bad = flags & 1u;
             if constexpr (F16) {
                 // 16 positions per step: half h holds 4 h + 0..3 and 8 + 4 h + 0..3 of them
 #pragma unroll

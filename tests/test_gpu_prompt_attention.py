@@ -107,3 +107,25 @@ def test_nan_scores_are_not_passed_over(engine, heads, kv_heads, hd, kv):
     q[70, heads - 1] = float("nan")
     want[70, heads - 1] = _decode_attention(engine, q, k, v, 0)[70, heads - 1]
     assert torch.equal(_prompt_attention(engine, q, k, v, 0), want)
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", LAYOUTS)
+def test_infinite_keys_and_queries(engine, heads, kv_heads, hd):
+    """Infinities in K of a binary16 cache (overflowed) and in q, where q runs
+    in parts: a score of minus infinity takes its position out, one of plus
+    infinity makes the row NaN, as q in one piece has it."""
+    n = 75
+    q, k, v = _inputs(2, n, 0, heads, kv_heads, hd, torch.float16)
+    k[2, 0, 1] = float("-inf")
+    k[40, 0, 7] = float("inf")
+    q[:, 0, 1], q[:, 0, 7] = q[:, 0, 1].abs(), -q[:, 0, 7].abs()      # head 0: minus infinity both times
+    want = _exact(q, k, v, 0)
+    assert bool(want[:, 0].isfinite().all()) and (heads == kv_heads or bool(want.isnan().any()))
+    _same_where_finite(_prompt_attention(engine, q, k, v, 0), want)
+    q, k, v = _inputs(3, n, 0, heads, kv_heads, hd, torch.float16)
+    k[:, 0, 5] = -k[:, 0, 5].abs()
+    k[9, 0, 5] = 1.0
+    q[4, 0, 5], q[50, 0, 5] = float("inf"), float("-inf")
+    want = _exact(q, k, v, 0)
+    want[4, 0] = _decode_attention(engine, q, k, v, 0)[4, 0].double().cpu()   # no score but minus infinity
+    _same_where_finite(_prompt_attention(engine, q, k, v, 0), want)
