@@ -13,15 +13,23 @@
 // are per lane; the probabilities are P.V's B operand as they lie, with the
 // position order of V's operand chosen to match.
 //  * binary16 caches: v_mfma_f32_32x32x16_f16. q is split into binary16
-//    hi + mid + lo parts after a power-of-two prescale (33 bits, as in
-//    MfmaAttn), P into hi + lo parts of 2^14 p (22 bits, as in
-//    attn_rows_kernel); V is transposed on its way into LDS.
-//  * binary32 caches: v_mfma_f32_32x32x2_f32, nothing split or rounded.
+//    hi + mid + lo parts after a power-of-two prescale of its largest element
+//    to 2^14 .. 2^15 (33 bits of that element, a fixed 2^-39 of it for the
+//    others), P into three parts of 2^14 p (every bit down to 2^-38); V is
+//    transposed on its way into LDS.
+//  * binary32 caches: v_mfma_f32_32x32x2_f32 (a chain of two FMAs), nothing
+//    split or rounded.
+// Sums run as short chains joined as equals (four dims of a score, eight
+// positions of P.V; four tiles of output before they join the running one), a
+// score is scaled after the maximum is taken off and l is a double: against 64 bits the
+// output is as close as the decode kernels' (rms 0.8 to 1.02 of their error over
+// up to 512 positions; with one chain per score and output, two parts of P and
+// q scaled down only, it was 1.1 to 2.2, and 120 where q was small).
 //
 // Bound by the longest row tile's chain of K/V tiles (a 512-row chunk is 128
-// workgroups of four heads, so CUs are idle): 33 us for 512 binary16 rows at
-// 32/8/128 heads against 160 through the decode kernels, 25 us for 133
-// binary32 rows at 32/32/128.
+// workgroups of four heads, so CUs are idle). Per call, back to back: 49 us for
+// 512 binary16 rows at 32/8/128 heads against 160 through the decode kernels,
+// 45 us for 133 binary32 rows at 32/32/128 (38 and 33 with the longer chains).
 #include <type_traits>
 
 #include "internal.h"
@@ -76,42 +84,42 @@ template <typename KV> __device__ __forceinline__ bool nonfinite(const ju4 &v) {
     return (b & (std::is_same<KV, _Float16>::value ? 0x80008000u : 0x80000000u)) != 0;
 }
 
-// The finite values of 8 binary16, others as 0.
-__device__ __forceinline__ ph8 finite_only(ph8 x) {
-    const uint4 v = __builtin_bit_cast(uint4, x);
-    uint32_t u[4] = {v.x, v.y, v.z, v.w};
+// The finite values of the 16 bytes, others as 0.
+template <typename KV> __device__ __forceinline__ ju4 finite_only(ju4 v) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        if ((u[i] & 0x7c00u) == 0x7c00u) u[i] &= 0xffff0000u;
-        if ((u[i] & 0x7c000000u) == 0x7c000000u) u[i] &= 0xffffu;
+        if constexpr (std::is_same<KV, _Float16>::value) {
+            if ((v[i] & 0x7c00u) == 0x7c00u) v[i] &= 0xffff0000u;
+            if ((v[i] & 0x7c000000u) == 0x7c000000u) v[i] &= 0xffffu;
+        } else if ((v[i] & 0x7f800000u) == 0x7f800000u) {
+            v[i] = 0u;
+        }
     }
-    return __builtin_bit_cast(ph8, make_uint4(u[0], u[1], u[2], u[3]));
+    return v;
 }
 
-// o[d] += p * V over the infinities and NaN of a V tile (the products left them
-// out): position j of the tile for the queries that see it (j < seen), so they
-// reach the dims that hold them and no other row or dim. s: probabilities of
-// the lane's positions. A tile that holds none does not come here.
+// o[d] += p * V over the infinities and NaN of a tile of V (rows of kvrow
+// elements from `v` on, `rows` of them in the cache; LDS has zeros in their
+// place): position j of the tile for the queries that see it (j < seen), so
+// they reach the dims that hold them and no other row or dim. s: probabilities
+// of the lane's positions. A tile that holds none does not come here.
 template <typename KV, int D>
-__device__ __forceinline__ void add_nonfinite(const unsigned char *vt, const pf16 &s, uint32_t seen, int h,
-                                              pf16 (&o)[D / 32]) {
-    typedef Tile<KV, D> T;
+__device__ __forceinline__ void add_nonfinite(const KV *v, uint32_t kvrow, uint32_t rows, const pf16 &s, uint32_t seen,
+                                              int h, pf16 (&o)[D / 32]) {
 #pragma unroll 1
     for (uint32_t j = 0; j < PT; ++j) {
         const int at = (int)(j >> 3) * 4 + (int)(j & 3);   // position j is s[at] of half (j / 4) % 2
         float mine = 0.0f;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) mine = v == at ? s[v] : mine;
+        for (int i = 0; i < 16; ++i) mine = i == at ? s[i] : mine;
         const float other = swap32(mine), p = (int)((j >> 2) & 1) == h ? mine : other;
+        const KV *row = v + (size_t)min(j, rows - 1) * kvrow;
 #pragma unroll
         for (int d = 0; d < D / 32; ++d)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const uint32_t dim = 32 * d + 8 * (v >> 2) + 4 * h + (v & 3);
-                float x;
-                if constexpr (std::is_same<KV, _Float16>::value) x = (float)((const _Float16 *)vt)[dim * T::VP + j];
-                else x = ((const float *)vt)[j * T::VP + dim];
-                if (j < seen && (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u) o[d][v] = fmaf(p, x, o[d][v]);
+            for (int i = 0; i < 16; ++i) {
+                const float x = (float)row[32 * d + 8 * (i >> 2) + 4 * h + (i & 3)];
+                if (j < seen && (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u) o[d][i] = fmaf(p, x, o[d][i]);
             }
     }
 }
@@ -133,9 +141,10 @@ __device__ __forceinline__ void whole_scores(const unsigned char *kt, const floa
 }
 
 // HW: heads of a KV head that a workgroup's wavefronts take (1, 2 or 4); the
-// other factor of 4 is row tiles.
+// other factor of 4 is row tiles. A chunk seldom has more workgroups than there
+// are CUs (4 per query head at most), so a wavefront may take a SIMD's registers.
 template <typename KV, int D, int HW>
-__global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(256, 1) void prefill_attn_kernel(PrefillArgs a) {
     constexpr bool F16 = std::is_same<KV, _Float16>::value;
     typedef Tile<KV, D> T;
     constexpr int SEG = T::SEG, SROW = D / SEG;       // 16-byte segments per row
@@ -187,6 +196,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         }
         const uint32_t any = (uint32_t)(__any(oddv) != 0) | (uint32_t)(__any(oddk) != 0) << 1;
         if (lane == 0) *(uint32_t *)(t + T::FLAGS + 4 * wave) = any;
+        // A probability of 0 does not mask an infinity or NaN of V, and one
+        // split into parts turns an infinity into a NaN: such values stay out of
+        // the MFMAs and are added on their own (the look at a tile takes about
+        // a dozen instructions per 16 bytes).
+        if (any & 1u)
+#pragma unroll
+            for (int j = 0; j < LD; ++j) vr[j] = finite_only<KV>(vr[j]);
 #pragma unroll
         for (int j = 0; j < LD; ++j)
             *(ju4 *)(t + ((size_t)row_of(j, false) * T::KP + seg_of(j, false) * SEG) * sizeof(KV)) = kr[j];
@@ -236,7 +252,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         qmax = fmaxf(qmax, swap32(qmax));
         int qe = 0;
         (void)frexpf(qmax, &qe);                  // qmax < 2^qe
-        const int sh = qe > 15 ? qe - 15 : 0;     // |q| 2^-sh < 2^15
+        const int sh = max(qe - 15, -100);        // 2^14 <= |qmax| 2^-sh < 2^15 (below 2^-85 no score counts)
         qs = ldexpf(1.0f, -sh);
         q_inf = __any(qmax == INFINITY);
         sc2 *= ldexpf(1.0f, sh);
@@ -260,10 +276,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         for (int s = 0; s < D / 8; ++s) qf[s] = *(const jf4 *)(qp + 8 * s + 4 * h);
     }
 
-    pf16 o[ND];   // O^T: dims 32 d + 8 j + 4 h + i of query col (binary16 caches: times 2^14)
+    // O^T: dims 32 d + 8 j + 4 h + i of query col (binary16 caches: times 2^14).
+    // o4 is the sum over the last tiles (up to four), which then joins o.
+    pf16 o[ND], o4[ND];
 #pragma unroll
-    for (int d = 0; d < ND; ++d) o[d] = (pf16){};
-    float m = -INFINITY, l = 0.0f;
+    for (int d = 0; d < ND; ++d) o[d] = o4[d] = (pf16){};
+    float m = -INFINITY;
+    double l = 0.0;
     bool lost = false;
     const uint32_t my_end = a.p0 + q0 + col + 1;                         // this lane's query sees [0, my_end)
     const uint32_t wave_end = q0 < a.n ? a.p0 + min(q0 + QT, a.n) : 0;   // uniform
@@ -277,25 +296,36 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
         if (p < wave_end) {
             const uint4 f = *(const uint4 *)(kt + T::FLAGS);
             const uint32_t flags = __builtin_amdgcn_readfirstlane(f.x | f.y | f.z | f.w);
-            // two chains, so that an MFMA need not wait for the one before it
+            // Short chains, then sums of equals: a chain over all dims would round
+            // every term at the size of the whole score.
             pf16 s = (pf16){}, s2 = (pf16){};
             if constexpr (F16) {
+                pf16 sm = (pf16){};   // the small parts
 #pragma unroll
                 for (int t = 0; t < D / 16; ++t) {
                     const ph8 k = *(const ph8 *)(kt + ((size_t)col * T::KP + 16 * t + 8 * h) * 2);
-                    s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, ql[t], s2, 0, 0, 0);
-                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, qh[t], s, 0, 0, 0);
-                    s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, qm[t], s2, 0, 0, 0);
+                    sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, ql[t], sm, 0, 0, 0);
+                    if (t & 1) s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, qh[t], s2, 0, 0, 0);
+                    else s = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, qh[t], s, 0, 0, 0);
+                    sm = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, qm[t], sm, 0, 0, 0);
                 }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) s2[v] += sm[v];
             } else {
 #pragma unroll
-                for (int t = 0; t < D / 8; ++t) {
-                    const jf4 k = *(const jf4 *)(kt + ((size_t)col * T::KP + 8 * t + 4 * h) * 4);
+                for (int t = 0; t < D / 8; t += 2) {   // 16 dims as a tree over chains of four
+                    pf16 c[4];
 #pragma unroll
-                    for (int i = 0; i < 4; i += 2) {
-                        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i], qf[t][i], s, 0, 0, 0);
-                        s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i + 1], qf[t][i + 1], s2, 0, 0, 0);
+                    for (int u = 0; u < 2; ++u) {
+                        const jf4 k = *(const jf4 *)(kt + ((size_t)col * T::KP + 8 * (t + u) + 4 * h) * 4);
+                        c[2 * u] = __builtin_amdgcn_mfma_f32_32x32x2f32(k[0], qf[t + u][0], (pf16){}, 0, 0, 0);
+                        c[2 * u + 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(k[2], qf[t + u][2], (pf16){}, 0, 0, 0);
+                        c[2 * u] = __builtin_amdgcn_mfma_f32_32x32x2f32(k[1], qf[t + u][1], c[2 * u], 0, 0, 0);
+                        c[2 * u + 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(k[3], qf[t + u][3], c[2 * u + 1], 0, 0, 0);
                     }
+                    pf16 &to = t & 2 ? s2 : s;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) to[v] += (c[0][v] + c[1][v]) + (c[2][v] + c[3][v]);
                 }
             }
 #pragma unroll
@@ -308,68 +338,93 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const bool live = p + 8 * (v >> 2) + 4 * h + (v & 3) < my_end;
-                s[v] = live ? s[v] * sc2 : -INFINITY;
+                s[v] = live ? s[v] : -INFINITY;
                 bm = fmaxf(bm, s[v]);
             }
             bm = fmaxf(bm, swap32(bm));
+            // m is in the scores' unit: their differences are exact near the
+            // maximum and are scaled after
             const float mn = fmaxf(m, bm);
-            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * sc2);
             // the maxima pass over a NaN: while there is no other score, it is kept here
             if (__any(mn == -INFINITY) && mn == -INFINITY)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) lost = lost || s[v] != s[v];
-            float sum = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                s[v] = mn == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[v] - mn);
-                sum += s[v];
-            }
-            l = l * alpha + sum;
+            for (int v = 0; v < 16; ++v) s[v] = mn == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((s[v] - mn) * sc2);
+            float sum[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum[v] = (s[4 * v] + s[4 * v + 1]) + (s[4 * v + 2] + s[4 * v + 3]);
+            l = fma(l, (double)alpha, (double)((sum[0] + sum[1]) + (sum[2] + sum[3])));
             m = mn;
             if (__any(alpha != 1.0f))   // after the first tiles the maximum rarely moves
 #pragma unroll
                 for (int d = 0; d < ND; ++d)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
-            // A probability of 0 does not mask an infinity or NaN of V, and one
-            // split into parts turns an infinity into a NaN: such values stay
-            // out of the MFMAs and are added on their own. They are noticed as
-            // the tile is stored (about a dozen instructions per 16 bytes).
-            const bool bad = flags & 1u;
+                    for (int v = 0; v < 16; ++v) {
+                        o[d][v] *= alpha;
+                        o4[d][v] *= alpha;
+                    }
+            // the tile's sums are made on their own and then added to o4
             if constexpr (F16) {
                 // 16 positions per step: half h holds 4 h + 0..3 and 8 + 4 h + 0..3 of them
+                ph8 pp[2][3];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    ph8 hi, lo;
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const float x = s[8 * t + e] * 16384.0f;
-                        const _Float16 xh = (_Float16)x;
-                        hi[e] = xh;
-                        lo[e] = (_Float16)(x - (float)xh);
+                        const _Float16 hi = (_Float16)x;
+                        const float r = x - (float)hi;
+                        const _Float16 mid = (_Float16)r;
+                        pp[t][0][e] = hi;
+                        pp[t][1][e] = mid;
+                        pp[t][2][e] = (_Float16)(r - (float)mid);
                     }
 #pragma unroll
-                    for (int d = 0; d < ND; ++d) {
+                for (int d = 0; d < ND; ++d) {
+                    ph8 v[2];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
                         const unsigned char *vp = vt + ((size_t)(32 * d + col) * T::VP + 16 * t + 4 * h) * 2;
                         const uint2 v0 = *(const uint2 *)vp, v1 = *(const uint2 *)(vp + 16);
-                        ph8 v = __builtin_bit_cast(ph8, make_uint4(v0.x, v0.y, v1.x, v1.y));
-                        if (bad) v = finite_only(v);
-                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, lo, o[d], 0, 0, 0);
-                        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, hi, o[d], 0, 0, 0);
+                        v[t] = __builtin_bit_cast(ph8, make_uint4(v0.x, v0.y, v1.x, v1.y));
                     }
+                    pf16 c = (pf16){};
+#pragma unroll
+                    for (int i = 2; i >= 0; --i) {
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[0], pp[0][i], c, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[1], pp[1][i], c, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) o4[d][i] += c[i];
                 }
             } else {
                 // step v: positions 8 (v / 4) + v % 4 (half 0) and that plus 4 (half 1)
 #pragma unroll
-                for (int v = 0; v < 16; ++v)
+                for (int d = 0; d < ND; ++d) {
+                    pf16 c[4];
 #pragma unroll
-                    for (int d = 0; d < ND; ++d) {
-                        float x = *(const float *)(vt + ((size_t)(8 * (v >> 2) + 4 * h + (v & 3)) * T::VP + 32 * d + col) * 4);
-                        if (bad && (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u) x = 0.0f;
-                        o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, s[v], o[d], 0, 0, 0);
+                    for (int j = 0; j < 4; ++j) {
+                        c[j] = (pf16){};
+#pragma unroll
+                        for (int v = 4 * j; v < 4 * j + 4; ++v) {
+                            const float x = *(const float *)(vt + ((size_t)(8 * j + 4 * h + (v & 3)) * T::VP + 32 * d + col) * 4);
+                            c[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, s[v], c[j], 0, 0, 0);
+                        }
                     }
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) o4[d][i] += (c[0][i] + c[1][i]) + (c[2][i] + c[3][i]);
+                }
             }
-            if (bad) add_nonfinite<KV, D>(vt, s, my_end - min(my_end, p), h, o);
+            if (flags & 1u) add_nonfinite<KV, D>(vc + (size_t)p * kvrow, kvrow, end_all - p, s, my_end - min(my_end, p), h, o4);
+            if ((p / PT) % 4 == 3 || p + PT >= wave_end)
+#pragma unroll
+                for (int d = 0; d < ND; ++d) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) o[d][v] += o4[d][v];
+                    o4[d] = (pf16){};
+                }
         }
         buf ^= 1u;
         store(smem + buf * T::BYTES);   // last read before the barrier above
@@ -378,15 +433,21 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(PrefillArgs a) {
     // a row whose scores are all NaN stays 0, as in the decode kernels
     const float other = swap32(lost ? 1.0f : 0.0f);
     if ((lost || other != 0.0f) && m != -INFINITY) l = NAN;
-    float lt = l + swap32(l);
-    const float inv = (F16 ? 1.0f / 16384.0f : 1.0f) / (lt < 1e-20f ? 1e-20f : lt);   // a NaN stays
+    float lt = (float)l + swap32((float)l);
+    lt = lt < 1e-20f ? 1e-20f : lt;   // a NaN stays
+    const float inv = 1.0f / lt;
+    auto divide = [&](float x) {   // x / lt: the remainder corrects the last bit
+        if (F16) x *= 1.0f / 16384.0f;
+        const float r = x * inv, rest = fmaf(-r, lt, x);
+        return rest == rest ? fmaf(rest, inv, r) : r;
+    };
     const size_t at = ((size_t)(q0 + col) * a.heads + head) * D + 4 * h;
 #pragma unroll
     for (int d = 0; d < ND; ++d)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float x0 = o[d][4 * j] * inv, x1 = o[d][4 * j + 1] * inv, x2 = o[d][4 * j + 2] * inv,
-                        x3 = o[d][4 * j + 3] * inv;
+            const float x0 = divide(o[d][4 * j]), x1 = divide(o[d][4 * j + 1]), x2 = divide(o[d][4 * j + 2]),
+                        x3 = divide(o[d][4 * j + 3]);
             const size_t i = at + 32 * d + 8 * j;
             if (a.out_f16)
                 *(uint2 *)((uint16_t *)a.out + i) = make_uint2((uint32_t)f2h_bits(x0) | ((uint32_t)f2h_bits(x1) << 16),

@@ -129,3 +129,22 @@ def test_infinite_keys_and_queries(engine, heads, kv_heads, hd):
     want = _exact(q, k, v, 0)
     want[4, 0] = _decode_attention(engine, q, k, v, 0)[4, 0].double().cpu()   # no score but minus infinity
     _same_where_finite(_prompt_attention(engine, q, k, v, 0), want)
+
+
+@pytest.mark.parametrize("kv", [torch.float16, torch.float32])
+@pytest.mark.parametrize("heads,kv_heads,hd", LAYOUTS)
+@pytest.mark.parametrize("q_scale,k_scale", [(2.0, 1.0), (2.0 ** -10, 2.0 ** 10), (2.0 ** -14, 2.0 ** 12), (2.0 ** 40, 2.0 ** -12)])
+def test_as_close_to_64_bits_as_the_decode_kernels(engine, heads, kv_heads, hd, kv, q_scale, k_scale):
+    """The root-mean-square error over a prompt's rows is that of the decode
+    kernels on the same rows, which hold q and the probabilities in binary32
+    (1.25 of it: the ratio of two samples of rounding errors), whatever the
+    sizes of q and K. A huge q leaves one position per row: its V exactly."""
+    ours = theirs = 0.0
+    for n, p0 in ((130, 0), (60, 100)):
+        q, k, v = _inputs(n + hd, n, p0, heads, kv_heads, hd, torch.float32)
+        q, k, v = q * q_scale, (k * k_scale).to(kv), v.to(kv)
+        want = _exact(q, k, v, p0)
+        got, one = (f(engine, q, k, v, p0).double().cpu() for f in (_prompt_attention, _decode_attention))
+        ours += float((got - want).square().sum())
+        theirs += float((one - want).square().sum())
+    assert ours <= 1.25 ** 2 * theirs, math.sqrt(ours / theirs)
