@@ -887,6 +887,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     constexpr int SPT = (MP * SEGS + NT - 1) / NT;   // segments per thread
     constexpr bool PART = SPT * NT != MP * SEGS;     // the last wavefronts stage nothing
     static_assert(CPW >= 1 && CPW * KW == PC && (!PART || SPT == 1) && MP * SEGS % 64 == 0, "pass shape");
+    static_assert(!X32 || !std::is_same<F, GF16>::value || CPW % 4 == 0, "parts of 64 of K");
     constexpr uint32_t PLANE = (uint32_t)MP * PITCH;   // halves of one staged part
     constexpr uint32_t ABYTES = PLANE * 2 * (X32 ? 3 : 1);
     constexpr uint32_t BUF = pipe_buf<F, MT, KR, X32, VN>();
@@ -918,11 +919,27 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
     for (int mt = 0; mt < MT; ++mt) pend.t[mt] = (f16x){};
     pend.d = 0.0f;
     // X32: 256 of K are summed on their own (part) and then added to acc, so
-    // the sum over K takes one long rounding per 256 and not one per block
+    // the sum over K takes one long rounding per 256 and not one per block.
     f16x part[MT];
     if constexpr (X32)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) part[mt] = (f16x){};
+    // F16 weights: part holds 64 of K and mid up to 8 of those, as the products
+    // themselves leave less room there (rms error 1.04 of the row kernels' over
+    // 32000x4096 at 40 rows without mid, 0.92 with it).
+    constexpr bool FINE = X32 && std::is_same<F, GF16>::value;
+    f16x mid[FINE ? MT : 1];
+    if constexpr (FINE)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) mid[mt] = (f16x){};
+    auto join = [&](f16x (&to)[MT], f16x (&from)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+            for (int v = 0; v < VN; ++v) to[mt][v] += from[mt][v];
+            from[mt] = (f16x){};
+        }
+    };
     typename F::W w[CPW];
     uint4 sv[SPT * (X32 ? 2 : 1)];
 
@@ -1032,17 +1049,17 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
                 else
                     F::template mma<MT, WIDE, VN>(w[i], As, PITCH, (uint32_t)(kw * CPW + i) * F::CK, lane, Ss, p * PC, acc);
             }
+            if constexpr (FINE)
+                if (i % 4 == 3) join(mid, part);
             if (decltype(load_next)::value) w[i] = F::load(a, gl, chunk_of(p + 1, i), lane);
             if constexpr (WIDE) __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (X32)
-            if (KR >= 256 || ((p - p_begin) & 1u) || !decltype(load_next)::value)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-                    for (int v = 0; v < VN; ++v) acc[mt][v] += part[mt][v];
-                    part[mt] = (f16x){};
-                }
+        if constexpr (FINE) {
+            constexpr uint32_t N = 32 / CPW;   // passes to 8 parts
+            if ((p - p_begin) % N == N - 1 || !decltype(load_next)::value) join(acc, mid);
+        } else if constexpr (X32) {
+            if (KR >= 256 || ((p - p_begin) & 1u) || !decltype(load_next)::value) join(acc, part);
+        }
     };
 
     if (p_begin < p_end) {
@@ -1155,12 +1172,17 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, uint32_t M
     const uint32_t m = (uint32_t)(idx / a.n), n = (uint32_t)(idx % a.n);
     const float *p = a.ws + (size_t)m * Npad + n;
     const size_t stride = (size_t)Mpad * Npad;
-    // split order; the loads of 8 splits are issued together
+    // split order; the loads of 8 splits are issued together, and on binary32
+    // activations they are also summed as equals before they join the rest
     float s = 0.0f;
     for (uint32_t j0 = 0; j0 < a.ksplit; j0 += 8) {
         float u[8];
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj) u[jj] = j0 + jj < a.ksplit ? p[(j0 + jj) * stride] : 0.0f;
+        if (a.a32) {
+            s += ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
+            continue;
+        }
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj)
             if (j0 + jj < a.ksplit) s += u[jj];
@@ -1644,9 +1666,12 @@ int launch_wide(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, GemmPa
             const uint64_t ks = a.swiglu || wgs > cus ? 1 : cus / wgs;
             return unit * (float)((wgs * ks + cus - 1) / cus) / (float)ks;
         };
-        const float t2 = time(64, 8, 1.0f), t3 = time(96, 8, 1.45f), t4 = time(64, 4, 0.57f);
-        if (t2 <= t3 && t2 <= t4) return launch_wide_mt<F, 2, true>(ctx, a, w, parts);
-        return t3 <= t4 ? launch_wide_mt<F, 3, true>(ctx, a, w, parts) : launch_wide_mt<F, 2, true, 4, 2>(ctx, a, w, parts);
+        const float t2 = time(64, 8, 1.0f), t4 = time(64, 4, 0.57f);
+        if constexpr (!std::is_same<F, GF16>::value) {   // F16's sums of 96 rows do not fit the registers
+            const float t3 = time(96, 8, 1.45f);
+            if (t3 < t2 && t3 <= t4) return launch_wide_mt<F, 3, true>(ctx, a, w, parts);
+        }
+        return t2 <= t4 ? launch_wide_mt<F, 2, true>(ctx, a, w, parts) : launch_wide_mt<F, 2, true, 4, 2>(ctx, a, w, parts);
     }
     // the M tile with the least padded work (per workgroup, unpacking and
     // staging cost about what 0.7 of an M subtile does)
