@@ -107,10 +107,10 @@ __device__ __forceinline__ h8 unpack_i8x8(uint32_t lo, uint32_t hi) {
 }
 
 // ---- binary32 activations: three bfloat16 parts ---------------------------------
-// A finite binary32 x is exactly x1 + x2 + x3 with bfloat16 parts of 8
-// significant bits each (x1 = the upper 16 bits of x, x2 those of x - x1, x3
-// the rest), over the whole binary32 range, and the quantised weights are
-// exact bfloat16 integers. So a product of binary32 activations is three
+// A finite binary32 x of at least 2^-110 (K-quants 2^-105) is exactly
+// x1 + x2 + x3 with bfloat16 parts of 8 significant bits each (x1 = the upper 16
+// bits of x, x2 those of x - x1, x3 the rest; what lies below 2^-133, K-quants
+// 2^-128, is cut off), and the quantised weights are exact bfloat16 integers. So a product of binary32 activations is three
 // v_mfma_f32_32x32x16_bf16 per operand pair, every partial product exact and
 // every sum binary32, with nothing rounded on the way in: the weights are read
 // once for all rows instead of once per row by the M = 1 kernel.
@@ -339,6 +339,7 @@ struct GQ4_0 {
     static constexpr bool DEFER = true;
     static constexpr bool ORDER4 = true;
     static constexpr float XSUM = -8.0f;   // X32: per-block sums are staged times this
+    static constexpr float XMUL = 1.0f;    // X32: and x times this
     struct W { uint4 q; uint32_t s; };
     // One chunk on binary32 activations: As holds their three bfloat16 parts
     // (`plane` halves apart). The offset -8 enters as the first accumulator,
@@ -414,6 +415,7 @@ struct GQ8_0 {
     static constexpr int CK = 32;
     static constexpr bool ORDER4 = false;
     static constexpr float XSUM = 0.0f;   // no sums
+    static constexpr float XMUL = 1.0f;
     struct W { uint4 q; uint16_t s; };
     // see GQ4_0::mma_x32
     template <int MT, bool PIN = false, int VN = 16>
@@ -458,13 +460,14 @@ struct GQ8_0 {
 struct GQ4_K {
     static constexpr int CK = 64;
     static constexpr bool ORDER4 = true;
-    static constexpr float XSUM = -8.0f;
+    static constexpr float XSUM = -8.0f, XMUL = 1.0f / 16.0f;
     struct W { uint4 q; uint4 hdr; };
     // binary32 activations (three bfloat16 parts, GQ4_0::mma_x32). The staged
     // sums are -8 sum(x) (Q5_K: -16), so the MFMA result is that of the centred
     // values q - 8 and ds * (q . x) - dm * sum(x) = ds * t + (dm - 8 ds) / 8 * staged:
     // the two large terms of a block mostly cancel before they are rounded.
-    // c: chunk of the row group.
+    // x is staged times XMUL, so that the staged sums stay finite wherever the
+    // row kernel's sums over 16 do (1/32 for Q5_K). c: chunk of the row group.
     template <int MT, bool PIN = false, int VN = 16, class G = GQ4_K>
     __device__ static void mma_x32(const typename G::W &w, const _Float16 *As, uint32_t plane, uint32_t pitch,
                                    uint32_t kl, uint32_t c, int lane, const float *Ss, f16x (&acc)[MT],
@@ -476,8 +479,9 @@ struct GQ4_K {
         for (int b = 0; b < 2; ++b) {
             float sc, mn;
             scale_min(w.hdr, 2 * j + b, sc, mn);
-            const float ds = d * sc, dm = dmin * mn;
-            const float cs = fmaf(G::XSUM, ds, dm) * (-1.0f / G::XSUM);   // the power of two is exact
+            // powers of two are exact
+            const float ds = d * sc * (1.0f / G::XMUL), dm = dmin * mn * (1.0f / G::XMUL);
+            const float cs = fmaf(G::XSUM, ds, dm) * (-1.0f / G::XSUM);
             b8 b0, b1;
             G::unpack_b(w, b, b0, b1);
 #pragma unroll
@@ -550,7 +554,7 @@ struct GQ4_K {
 struct GQ5_K {
     static constexpr int CK = 64;
     static constexpr bool ORDER4 = true;
-    static constexpr float XSUM = -16.0f;
+    static constexpr float XSUM = -16.0f, XMUL = 1.0f / 32.0f;
     struct W { uint4 q; uint4 hdr; uint32_t fifth; };
     template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
@@ -624,7 +628,7 @@ template <> struct NeedsSums<GQ5_K> { static constexpr bool value = true; };
 struct GF16 {
     static constexpr int CK = 16;
     static constexpr bool ORDER4 = false;
-    static constexpr float XSUM = 0.0f;
+    static constexpr float XSUM = 0.0f, XMUL = 1.0f;
     struct W { uint4 q; };
     // binary32 activations: the weight is two bfloat16 parts, so a 16-wide
     // chunk is six MFMAs. The product of the two leading parts goes to acc,
@@ -984,7 +988,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
                 const uint32_t u[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
                 float x[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = ok ? __uint_as_float(u[e]) : 0.0f;
+                for (int e = 0; e < 8; ++e) x[e] = ok ? __uint_as_float(u[e]) * F::XMUL : 0.0f;
                 uint4 part[3];
                 const bool inf = split_x8<F::ORDER4>(x, part);
                 if (FLAG && inf) *(uint32_t *)(smem + (p & 1) * BUF + ABYTES) = 1u;

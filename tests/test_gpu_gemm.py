@@ -304,3 +304,32 @@ def test_f32_rows_on_mfma_are_as_close_as_single_rows(engine, ggml_type, rows, n
     upper = lambda t: (t.view(torch.int32) & -65536).view(torch.float32)
     x12 = upper(x).double() + upper(x - upper(x)).double()
     assert float((x12 @ w.dequant().double().T.contiguous() - want).norm()) > 1.5 * single
+
+
+@pytest.mark.parametrize("ggml_type", [12, 13])
+@pytest.mark.parametrize("rows", [5, 40])
+def test_f32_rows_on_mfma_at_the_top_of_the_range(engine, ggml_type, rows):
+    """K-quant blocks whose six-bit scales and mins are 1 and x near the top of
+    binary32: a block's sum of x times 8 or 16 exceeds it, the row kernel's sums
+    do not, and neither do these. A row of 2^-124: each x keeps what is not
+    below 2^-128 (its last part is a bfloat16, of 2^-133, of x / 32)."""
+    n, k = 64, 512
+    rng = np.random.default_rng(3)
+    blocks = np.zeros((n * k // 256, 144 if ggml_type == 12 else 176), np.uint8)
+    blocks[:, 0:4] = np.array([2.0 ** -14, 2.0 ** -12], np.float16).view(np.uint8)   # d, dmin
+    blocks[:, 4:12], blocks[:, 12:16] = 1, 0x11
+    blocks[:, -128:] = rng.integers(0, 256, (len(blocks), 128)) & 0x11               # q of 0 or 1
+    w = ops.GpuTensor(engine, ggml_type, n, k, blocks)
+    x = torch.full((rows, k), 2.0 ** 122)
+    x[1] = torch.randn(k, generator=torch.Generator().manual_seed(4)) * 2.0 ** -124
+    x[:, 300:] *= -0.75
+    a, c = x.to(DEV), torch.empty(rows, n, device=DEV)
+    ops.gemm_auto(engine, a, w, c, rows, 1, k, n)
+    y = torch.empty(n, device=DEV)
+    ops.gemm_auto(engine, a[0], w, y, 1, 1, k, n)
+    assert bool(y.isfinite().all()) and bool(c.isfinite().all())
+    keep = [0] + list(range(2, rows))
+    _check_f32_against_f64(c[keep], w.dequant().cpu().numpy(), x[keep])
+    wf = w.dequant().cpu().double()
+    err = (c[1].double().cpu() - x[1].double() @ wf.T).abs()
+    assert bool((err <= 1.01 * 2.0 ** -128 * wf.abs().sum(1)).all())
