@@ -114,7 +114,8 @@ struct janus_weight {
     const uint8_t *t32_side = nullptr;
     const uint32_t *t32_q5h = nullptr;   // Q5_K: the fifth bits, one word per lane and chunk
     uint32_t t32_chunks = 0;
-    bool t32_nonfinite = false;          // F16: some weight is infinite or NaN
+    bool t32_nonfinite = false;          // F16: some weight is infinite or NaN (known once a copy was made)
+    bool t32_denied = false;             // no memory for a copy that was not indispensable: not asked for again
 };
 
 namespace janus {

@@ -707,8 +707,8 @@ bool prefill_ready(janus_model *m) {
         split = split || !L.qkv || !L.gu;
         for (const janus_weight *w : ws) {
             if (!w->t32) built.push_back(w);
-            ok = ok && mfma_gemm_supported(JANUS_DT_F16, w) && mfma_gemm_prepare(ctx, w) == JANUS_OK &&
-                 mfma_rows_supported(c.act_dtype, w);
+            ok = ok && mfma_rows_supported(c.act_dtype, w) && mfma_gemm_prepare(ctx, w) == JANUS_OK &&
+                 mfma_rows_supported(c.act_dtype, w);   // F16 on binary32 rows: known with the copy
         }
     }
     const size_t R = c.max_seq_len < kPrefillRows ? c.max_seq_len : kPrefillRows, kvd = (size_t)c.kv_heads * c.head_dim;

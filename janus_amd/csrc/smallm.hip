@@ -1344,9 +1344,11 @@ uint32_t chunk_k(int type) {
     }
 }
 
-// Builds the weight's T32 copy (device memory, kept with the weight).
-int t32_ensure(janus_ctx *ctx, janus_weight *w) {
-    if (w->t32) return JANUS_OK;
+// Builds the weight's T32 copy (device memory, kept with the weight). exact:
+// only a copy with exact parts is of use; for a weight that has none,
+// t32_nonfinite is set and nothing kept.
+int t32_ensure(janus_ctx *ctx, janus_weight *w, bool exact = false) {
+    if (w->t32 || (exact && w->t32_nonfinite)) return JANUS_OK;
     const uint32_t G = (w->n + 31) / 32, ck = chunk_k(w->type);
     const uint32_t C = (w->k + ck - 1) / ck;
     const size_t qbytes = (size_t)G * C * 64 * 16;
@@ -1391,12 +1393,16 @@ int t32_ensure(janus_ctx *ctx, janus_weight *w) {
         (void)hipFree(mem);   // already failing: the repack error is the one reported
         return hip_fail(ctx, e, "t32 repack");
     }
-    w->t32 = mem;
+    w->t32_nonfinite = bad != 0;
+    if (exact && bad) {
+        (void)hipFree(mem);
+        return JANUS_OK;
+    }
     w->t32_qs = dq;
     w->t32_side = ds;
     w->t32_q5h = fifth ? df : nullptr;
     w->t32_chunks = C;
-    w->t32_nonfinite = bad != 0;
+    w->t32 = mem;
     return JANUS_OK;
 }
 
@@ -1918,7 +1924,6 @@ void mfma_gemm_release(const janus_weight *cw) {
     w->t32_qs = w->t32_side = nullptr;
     w->t32_q5h = nullptr;
     w->t32_chunks = 0;
-    w->t32_nonfinite = false;
 }
 
 int smallm_gemm_launch(janus_ctx *ctx, const void *a, int a_dt, const janus_weight *w, void *c, int c_dt,
@@ -1933,15 +1938,13 @@ int smallm_gemm_launch(janus_ctx *ctx, const void *a, int a_dt, const janus_weig
     // capture; a binary16 weight with an infinity or NaN has no exact parts),
     // else one GEMV launch per row
     if (a_dt == JANUS_DT_F32 && mfma_gemm_supported(JANUS_DT_F16, w) && x32_pays(w, rows)) {
-        bool tiles = w->t32 != nullptr;
-        if (!tiles && !capturing(ctx)) {
-            tiles = mfma_gemm_prepare(ctx, w) == JANUS_OK;
-            if (!tiles) {   // no memory for the copy
-                (void)hipGetLastError();
-                ctx->last_error.clear();
-            }
+        janus_weight *mw = const_cast<janus_weight *>(w);
+        if (!w->t32 && !w->t32_nonfinite && !w->t32_denied && !capturing(ctx) && t32_ensure(ctx, mw, true)) {
+            mw->t32_denied = true;
+            (void)hipGetLastError();
+            ctx->last_error.clear();
         }
-        if (tiles && !w->t32_nonfinite) {
+        if (w->t32 && !w->t32_nonfinite) {
             GemmArgs g = make_args(w, nullptr, c, c_dt == JANUS_DT_F16, rows, residual);
             g.a32 = (const float *)a;
             bool ran = false;

@@ -333,3 +333,28 @@ def test_f32_rows_on_mfma_at_the_top_of_the_range(engine, ggml_type, rows):
     wf = w.dequant().cpu().double()
     err = (c[1].double().cpu() - x[1].double() @ wf.T).abs()
     assert bool((err <= 1.01 * 2.0 ** -128 * wf.abs().sum(1)).all())
+
+
+def test_f32_rows_keep_no_copy_of_a_weight_without_exact_parts(engine):
+    """The tile copy of a binary16 weight (its size again) stays with the
+    weight where binary32 rows run on it, and not where an infinity keeps them
+    on the row kernels; binary16 rows may still build it."""
+    n, k, rows = 8192, 4096, 5   # 64 MiB
+    bits = synth.f16_bits(np.full((n, k), 0.02, np.float32)).reshape(n, k).copy()
+    a, c = torch.randn(rows, k, device=DEV), torch.empty(rows, n, device=DEV)
+    for kept, value in ((True, bits[3, 3]), (False, 0x7C00)):
+        bits[3, 3] = value
+        w = ops.GpuTensor(engine, 1, n, k, bits)
+        ops.gemm_auto(engine, a[:1], w, c[:1], 1, 1, k, n)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        for _ in range(2):
+            ops.gemm_auto(engine, a, w, c, rows, 1, k, n)
+        torch.cuda.synchronize()
+        assert (free - torch.cuda.mem_get_info()[0] > 32 << 20) == kept
+        h = torch.empty(rows, n, device=DEV)
+        ops.gemm_auto(engine, a.half(), w, h, rows, 1, k, n)
+        torch.cuda.synchronize()
+        assert free - torch.cuda.mem_get_info()[0] > 32 << 20
+        assert bool(h.isfinite().all(0)[3]) == kept and bool(h[:, 4:].isfinite().all())
+        w.free()
