@@ -3,9 +3,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <type_traits>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -108,14 +110,16 @@ struct janus_weight {
     size_t bytes = 0;
     const uint8_t *qs = nullptr;
     const uint16_t *sc = nullptr;
-    // MFMA tile copy for the small-M GEMM (smallm.hip), built on first use.
-    void *t32 = nullptr;
+    // MFMA tile copy for the small-M GEMM (smallm.hip), built on first use under
+    // t32_mu; t32 is set last, so whoever sees it sees the rest.
+    std::mutex t32_mu;
+    std::atomic<void *> t32{nullptr};
     const uint8_t *t32_qs = nullptr;
     const uint8_t *t32_side = nullptr;
     const uint32_t *t32_q5h = nullptr;   // Q5_K: the fifth bits, one word per lane and chunk
     uint32_t t32_chunks = 0;
-    bool t32_nonfinite = false;          // F16: some weight is infinite or NaN (known once a copy was made)
-    bool t32_denied = false;             // no memory for a copy that was not indispensable: not asked for again
+    std::atomic<bool> t32_nonfinite{false};   // F16: some weight is infinite or NaN (known once a copy was made)
+    std::atomic<bool> t32_denied{false};      // no memory for a copy that was not indispensable: not asked for again
 };
 
 namespace janus {

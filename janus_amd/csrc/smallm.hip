@@ -1344,10 +1344,13 @@ uint32_t chunk_k(int type) {
     }
 }
 
-// Builds the weight's T32 copy (device memory, kept with the weight). exact:
-// only a copy with exact parts is of use; for a weight that has none,
-// t32_nonfinite is set and nothing kept.
+// Builds the weight's T32 copy (device memory, kept with the weight). Several
+// threads, each with its context, may come here with one weight. exact: only a
+// copy with exact parts is of use; for a weight that has none, t32_nonfinite is
+// set and nothing kept.
 int t32_ensure(janus_ctx *ctx, janus_weight *w, bool exact = false) {
+    if (w->t32) return JANUS_OK;
+    std::lock_guard<std::mutex> lock(w->t32_mu);
     if (w->t32 || (exact && w->t32_nonfinite)) return JANUS_OK;
     const uint32_t G = (w->n + 31) / 32, ck = chunk_k(w->type);
     const uint32_t C = (w->k + ck - 1) / ck;

@@ -8,6 +8,8 @@ match the M=1 kernel on the same binary16 row, and both must match an f64
 product of the bit-exact dequantised weights within
 |y - y64| <= 2e-5 * sum_i |w_i x_i|   (exact products, fp32 accumulation).
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -358,3 +360,39 @@ def test_f32_rows_keep_no_copy_of_a_weight_without_exact_parts(engine):
         assert free - torch.cuda.mem_get_info()[0] > 32 << 20
         assert bool(h.isfinite().all(0)[3]) == kept and bool(h[:, 4:].isfinite().all())
         w.free()
+
+
+def test_f32_rows_of_several_threads_on_one_weight():
+    """Threads with a context and a stream each make the first call with
+    several binary32 rows on a weight at the same time: the tile copy is built
+    once, and all get the result of a call alone."""
+    n, k, rows, count = 4096, 2048, 9, 6
+    engines = [ops.ComputeEngine(0) for _ in range(count)]
+    streams = [torch.cuda.Stream() for _ in range(count)]
+    a = torch.randn(rows, k, device=DEV)
+    outs = [torch.zeros(rows, n, device=DEV) for _ in range(count)]
+    for e, s in zip(engines, streams):
+        e.bind_stream(s)
+    for turn in range(4):
+        _, w = _weight(engines[0], 2, n, k, turn)
+        torch.cuda.synchronize()
+        start = threading.Barrier(count)
+
+        def call(i):
+            start.wait()
+            ops.gemm_auto(engines[i], a, w, outs[i], rows, 1, k, n)
+            engines[i].sync()
+
+        threads = [threading.Thread(target=call, args=(i,)) for i in range(count)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        want = torch.empty(rows, n, device=DEV)
+        torch.cuda.synchronize()
+        ops.gemm_auto(engines[0], a, w, want, rows, 1, k, n)
+        engines[0].sync()
+        assert all(torch.equal(o, want) for o in outs)
+        w.free()
+    for e in engines:
+        e.close()
