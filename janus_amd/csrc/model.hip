@@ -501,6 +501,7 @@ int upload_step(janus_model *m, const uint32_t *tokens, const uint32_t *position
 __global__ void set_sampler_kernel(SamplerDev s, SamplerDev *out) { *out = s; }
 
 int upload_sampler(janus_model *m) {
+    DeviceGuard g(m->ctx->device);   // janus_model_set_sampler works whatever device is current
     hipLaunchKernelGGL(set_sampler_kernel, dim3(1), dim3(1), 0, m->ctx->stream, m->h_sampler, m->d_sampler);
     JANUS_LAUNCH_CHECK(m->ctx);
     return JANUS_OK;
