@@ -560,3 +560,67 @@ def test_an_overflowed_value_reaches_only_the_rows_that_see_it(engine, heads, kv
         assert bool(x[:, :bad].isfinite().all())
         assert float((x[:, :bad] - r[:, :bad]).norm() / r[:, :bad].norm()) <= 2e-3
     assert not bool(caches[1][1][0, bad].isfinite().any())
+
+
+def _eager_cache(m, kv, prompt):
+    for x in kv:
+        x.zero_()
+    for p, t in enumerate(prompt):
+        m.forward([t], [p])
+    torch.cuda.synchronize()
+    return [x.clone() for x in kv]
+
+
+def test_a_weight_without_exact_parts_keeps_prompts_token_by_token(engine):
+    """A binary16 layer weight with an infinity on binary32 activations: found
+    after the other weights' tile copies were built, which are given back
+    (their 50 MB), and prompts run as before: the K/V rows are those of eager
+    steps bit for bit (chunks sum in another order), over two length buckets."""
+    s = synth.make_model(101, 512, 4, 4, 8192, 300, 2, synth.F16, 1e-5, 10000.0, embed_type=synth.F16,
+                         head_type=synth.F16)
+    t = [t for t in s.tensors if t.name == "blk.1.ffn_down.weight"][0]   # after the last K/V rows
+    t.data = np.array(t.data, dtype=np.uint16, copy=True).reshape(s.hidden, s.ffn)
+    t.data[5, 17] = 0x7C00
+    prompt = _prompt(102, 300, s.vocab)
+    m = Model(engine, s, max_seq_len=310)
+    kv = [torch.zeros(2, 310, 4, 128, device=DEV) for _ in range(2)]
+    m.set_kv_cache(*kv)
+    want = _eager_cache(m, kv, prompt)
+    free = torch.cuda.mem_get_info()[0]
+    for x in kv:
+        x.zero_()
+    m.generate(prompt, 1, 1.0)   # the GPU argmax: NaN logits are not refused
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 25 << 20
+    assert not bool(torch.from_numpy(m.logits()).isfinite().all())
+    for x, w in zip(kv, want):
+        assert torch.equal(x[:, :300], w[:, :300])
+    m.close()
+
+
+def test_long_prompts_token_by_token_in_every_loop(monkeypatch):
+    """Prompts across two length buckets without chunks (JANUS_FUSED=0): K/V
+    rows of generate, its streaming form and generate_batch (two rows, the
+    shorter prompt decoding while the longer one still prefills) are those of
+    eager steps up to the order of binary32 sums (attention planned for the
+    bucket), and their tokens agree with eager steps' or part at a near tie."""
+    s = _prompt_model(synth.Q4_0)
+    monkeypatch.setenv("JANUS_FUSED", "0")
+    eng = ops.ComputeEngine(0)
+    m = Model(eng, s, max_seq_len=330, max_batch=2)
+    kv = [torch.zeros(2, 2 * 330, s.kv_heads, 128, device=DEV) for _ in range(2)]
+    m.set_kv_cache(*kv)
+    prompts = [_prompt(103, 300, s.vocab), _prompt(104, 40, s.vocab)]
+    want = [_eager_tokens(m, p, 12, 1.15) for p in prompts]
+    rows = _eager_cache(m, kv, prompts[0])
+    for run in (lambda: m.generate(prompts[0], 12), lambda: m.generate_with_callback(prompts[0], 12)):
+        for x in kv:
+            x.zero_()
+        assert_same_or_near_tie(run(), *want[0], 1.15)
+        torch.cuda.synchronize()
+        for x, w in zip(kv, rows):
+            assert float((x[:, :300] - w[:, :300]).norm() / w[:, :300].norm()) <= 1e-5
+    for got, w in zip(m.generate_batch(prompts, 12), want):
+        assert_same_or_near_tie(got, *w, 1.15)
+    m.close()
+    eng.close()
