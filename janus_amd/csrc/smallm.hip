@@ -107,18 +107,18 @@ __device__ __forceinline__ h8 unpack_i8x8(uint32_t lo, uint32_t hi) {
 }
 
 // ---- binary32 activations: three bfloat16 parts ---------------------------------
-// A finite binary32 x of at least 2^-110 (K-quants 2^-105) is exactly
-// x1 + x2 + x3 with bfloat16 parts of 8 significant bits each (x1 = the upper 16
-// bits of x, x2 those of x - x1, x3 the rest; what lies below 2^-133, K-quants
-// 2^-128, is cut off), and the quantised weights are exact bfloat16 integers. So a product of binary32 activations is three
+// A finite binary32 x of at least 2^-110 (Q5_K 2^-105) is exactly x1 + x2 + x3
+// with bfloat16 parts of 8 significant bits each (x1 = the upper 16 bits of x,
+// x2 those of x - x1, x3 the rest; what lies below 2^-133, Q5_K 2^-128, is cut
+// off), and the quantised weights are exact bfloat16 integers. So a product of binary32 activations is three
 // v_mfma_f32_32x32x16_bf16 per operand pair, every partial product exact and
 // every sum binary32, with nothing rounded on the way in: the weights are read
 // once for all rows instead of once per row by the M = 1 kernel.
 
-// Bytes (b0, b1) / (b2, b3) of v (each below 16) as exact bfloat16 integers
-// (OCP e4m3 byte b < 16 is b * 2^-9; the conversion scales it by 512).
-template <bool HI> __device__ __forceinline__ b2 nib8_bf16(uint32_t v) {
-    return __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f, HI);
+// Bytes (b0, b1) / (b2, b3) of v (each below 16) times `unit`, a power of two, as
+// exact bfloat16 (OCP e4m3 byte b < 16 is b * 2^-9; the conversion scales it).
+template <bool HI> __device__ __forceinline__ b2 nib8_bf16(uint32_t v, float unit) {
+    return __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 512.0f * unit, HI);
 }
 
 // The upper halves of two floats as a bfloat16 pair (exact for integers below 256).
@@ -126,12 +126,13 @@ __device__ __forceinline__ uint32_t pack_hi16(float lo, float hi) {
     return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
 
-// A T32 word of 8 nibbles -> 8 bfloat16 integers in the order e0 e4 e1 e5 e2
+// A T32 word of 8 nibbles -> 8 bfloat16 integers (times `unit`) in the order e0 e4 e1 e5 e2
 // e6 e3 e7 (the byte order of the word's low and high nibbles); the
 // activations are staged in the same order (SplitOrder).
-__device__ __forceinline__ b8 unpack_nib8_b(uint32_t u) {
+__device__ __forceinline__ b8 unpack_nib8_b(uint32_t u, float unit = 1.0f) {
     const uint32_t lo = u & 0x0f0f0f0fu, hi = (u >> 4) & 0x0f0f0f0fu;
-    const b2 p0 = nib8_bf16<false>(lo), p1 = nib8_bf16<true>(lo), p2 = nib8_bf16<false>(hi), p3 = nib8_bf16<true>(hi);
+    const b2 p0 = nib8_bf16<false>(lo, unit), p1 = nib8_bf16<true>(lo, unit), p2 = nib8_bf16<false>(hi, unit),
+             p3 = nib8_bf16<true>(hi, unit);
     return (b8){p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
 }
 
@@ -339,7 +340,8 @@ struct GQ4_0 {
     static constexpr bool DEFER = true;
     static constexpr bool ORDER4 = true;
     static constexpr float XSUM = -8.0f;   // X32: per-block sums are staged times this
-    static constexpr float XMUL = 1.0f;    // X32: and x times this
+    static constexpr float XMUL = 1.0f;    // X32: x is staged times this
+    static constexpr float WMUL = 1.0f;    // X32: and the weights' integers are times this, and the sums too
     struct W { uint4 q; uint32_t s; };
     // One chunk on binary32 activations: As holds their three bfloat16 parts
     // (`plane` halves apart). The offset -8 enters as the first accumulator,
@@ -415,7 +417,7 @@ struct GQ8_0 {
     static constexpr int CK = 32;
     static constexpr bool ORDER4 = false;
     static constexpr float XSUM = 0.0f;   // no sums
-    static constexpr float XMUL = 1.0f;
+    static constexpr float XMUL = 1.0f, WMUL = 1.0f;
     struct W { uint4 q; uint16_t s; };
     // see GQ4_0::mma_x32
     template <int MT, bool PIN = false, int VN = 16>
@@ -460,14 +462,17 @@ struct GQ8_0 {
 struct GQ4_K {
     static constexpr int CK = 64;
     static constexpr bool ORDER4 = true;
-    static constexpr float XSUM = -8.0f, XMUL = 1.0f / 16.0f;
+    static constexpr float XSUM = -8.0f, XMUL = 1.0f, WMUL = 1.0f / 16.0f;
     struct W { uint4 q; uint4 hdr; };
     // binary32 activations (three bfloat16 parts, GQ4_0::mma_x32). The staged
     // sums are -8 sum(x) (Q5_K: -16), so the MFMA result is that of the centred
     // values q - 8 and ds * (q . x) - dm * sum(x) = ds * t + (dm - 8 ds) / 8 * staged:
     // the two large terms of a block mostly cancel before they are rounded.
-    // x is staged times XMUL, so that the staged sums stay finite wherever the
-    // row kernel's sums over 16 do (1/32 for Q5_K). c: chunk of the row group.
+    // Products and sums are made 16 times smaller (Q5_K: 32), so that the sums
+    // stay finite wherever the row kernel's over 16 elements do: by the
+    // conversion of the nibbles, in Q5_K, whose five bits have none, by x as it
+    // is staged (either is within the spread of 63 us, 11008x4096 and back at 16
+    // rows). c: chunk of the row group.
     template <int MT, bool PIN = false, int VN = 16, class G = GQ4_K>
     __device__ static void mma_x32(const typename G::W &w, const _Float16 *As, uint32_t plane, uint32_t pitch,
                                    uint32_t kl, uint32_t c, int lane, const float *Ss, f16x (&acc)[MT],
@@ -480,7 +485,8 @@ struct GQ4_K {
             float sc, mn;
             scale_min(w.hdr, 2 * j + b, sc, mn);
             // powers of two are exact
-            const float ds = d * sc * (1.0f / G::XMUL), dm = dmin * mn * (1.0f / G::XMUL);
+            constexpr float up = 1.0f / (G::XMUL * G::WMUL);
+            const float ds = d * sc * up, dm = dmin * mn * up;
             const float cs = fmaf(G::XSUM, ds, dm) * (-1.0f / G::XSUM);
             b8 b0, b1;
             G::unpack_b(w, b, b0, b1);
@@ -496,8 +502,8 @@ struct GQ4_K {
         }
     }
     __device__ static void unpack_b(const W &w, int b, b8 &b0, b8 &b1) {
-        b0 = unpack_nib8_b(b ? w.q.z : w.q.x);
-        b1 = unpack_nib8_b(b ? w.q.w : w.q.y);
+        b0 = unpack_nib8_b(b ? w.q.z : w.q.x, WMUL);
+        b1 = unpack_nib8_b(b ? w.q.w : w.q.y, WMUL);
     }
     __device__ static W load(const GemmArgs &a, uint32_t g, uint32_t c, int lane) {
         const size_t ch = (size_t)g * a.chunks + c;
@@ -554,7 +560,7 @@ struct GQ4_K {
 struct GQ5_K {
     static constexpr int CK = 64;
     static constexpr bool ORDER4 = true;
-    static constexpr float XSUM = -16.0f, XMUL = 1.0f / 32.0f;
+    static constexpr float XSUM = -16.0f, XMUL = 1.0f / 32.0f, WMUL = 1.0f;
     struct W { uint4 q; uint4 hdr; uint32_t fifth; };
     template <int MT, bool PIN = false, int VN = 16>
     __device__ static void mma_x32(const W &w, const _Float16 *As, uint32_t plane, uint32_t pitch, uint32_t kl,
@@ -628,7 +634,7 @@ template <> struct NeedsSums<GQ5_K> { static constexpr bool value = true; };
 struct GF16 {
     static constexpr int CK = 16;
     static constexpr bool ORDER4 = false;
-    static constexpr float XSUM = 0.0f, XMUL = 1.0f;
+    static constexpr float XSUM = 0.0f, XMUL = 1.0f, WMUL = 1.0f;
     struct W { uint4 q; };
     // binary32 activations: the weight is two bfloat16 parts, so a 16-wide
     // chunk is six MFMAs. The product of the two leading parts goes to acc,
@@ -996,7 +1002,7 @@ __global__ __launch_bounds__(64 * NW * KW) void gemm_pipe_kernel(GemmArgs a) {
 #pragma unroll
                 for (int j = 0; j < 3; ++j) *(uint4 *)(at + j * PLANE) = part[j];
                 if constexpr (F::XSUM != 0.0f)
-                    put_sum(p, s, F::XSUM * (((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]))));
+                    put_sum(p, s, F::XSUM * F::WMUL * (((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]))));
                 continue;
             }
             const uint4 v = ok ? sv[i] : make_uint4(0u, 0u, 0u, 0u);

@@ -314,7 +314,7 @@ def test_f32_rows_on_mfma_at_the_top_of_the_range(engine, ggml_type, rows):
     """K-quant blocks whose six-bit scales and mins are 1 and x near the top of
     binary32: a block's sum of x times 8 or 16 exceeds it, the row kernel's sums
     do not, and neither do these. A row of 2^-124: each x keeps what is not
-    below 2^-128 (its last part is a bfloat16, of 2^-133, of x / 32)."""
+    below 2^-133, the last place of a bfloat16 (Q5_K: of x / 32)."""
     n, k = 64, 512
     rng = np.random.default_rng(3)
     blocks = np.zeros((n * k // 256, 144 if ggml_type == 12 else 176), np.uint8)
@@ -334,7 +334,8 @@ def test_f32_rows_on_mfma_at_the_top_of_the_range(engine, ggml_type, rows):
     _check_f32_against_f64(c[keep], w.dequant().cpu().numpy(), x[keep])
     wf = w.dequant().cpu().double()
     err = (c[1].double().cpu() - x[1].double() @ wf.T).abs()
-    assert bool((err <= 1.01 * 2.0 ** -128 * wf.abs().sum(1)).all())
+    last = 2.0 ** (-133 if ggml_type == 12 else -128)
+    assert bool((err <= 1.01 * last * wf.abs().sum(1)).all())
 
 
 def test_f32_rows_keep_no_copy_of_a_weight_without_exact_parts(engine):
