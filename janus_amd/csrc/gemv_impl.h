@@ -1693,9 +1693,9 @@ int launch_lds32(janus_ctx *ctx, const GemvArgs &a, bool norm) {
 // ffn_down loaded from Q6_K): the whole row is in flight at once,
 // single-buffered, and x is read from LDS at use. They took the per-launch
 // kernel, which stages x behind four rows' loads in every 256-thread
-// workgroup: 4096x14336 43.0 -> 22.5 us (5.2 TB/s), 4096x11008 34.2 -> 17.9,
-// 4096x8192 unchanged at 13.7. (With binary16 x the register kernel holds
-// such rows' x and is as fast: 21.7 us at 4096x14336.)
+// workgroup: 4096x14336 41.3 -> 22.5 us (5.2 TB/s), 4096x11008 34.2 -> 18.6,
+// 4096x8192 unchanged at 13.9. (With binary16 x the register kernel holds
+// such rows' x and is as fast: 21.0 us at 4096x14336.)
 inline int launch_f16_long(janus_ctx *ctx, const GemvArgs &a, int bpl, bool &done) {
     done = bpl <= 32;
     if (!done) return JANUS_OK;

@@ -940,8 +940,9 @@ int run_requests(janus_model *m, const std::vector<Request> &reqs, uint32_t max_
     return JANUS_OK;
 }
 
-// The streaming form of run_requests for one request in row 0: the prompt
-// on replays of the captured step, then one replay per token with the row's
+// The streaming form of run_requests for one request in row 0: the prompt in
+// chunks (what they leave of it on replays of the captured step), then one
+// replay per token with the row's
 // control block and its token copied behind it to pinned host memory; the
 // host hands step i's token to the callback while step i + 1 runs.
 int run_stream(janus_model *m, const Request &q, uint32_t max_tokens, janus_token_callback cb, void *user,

@@ -1174,7 +1174,9 @@ void launch_pipe_rows(janus_ctx *ctx, dim3 grid, const GemmArgs &a) {
     launch_pipe<F, MT, KW, KR, X32>(ctx, grid, a);
 }
 
-// Sums the split-K partials in split order and applies the epilogue.
+// Sums the split-K partials in split order and applies the epilogue. X32
+// (binary32 activations): eight at a time as equals before they join the rest.
+template <bool X32>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, uint32_t Mpad) {
     const uint32_t Npad = (a.n + 31) / 32 * 32;
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -1182,14 +1184,13 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, uint32_t M
     const uint32_t m = (uint32_t)(idx / a.n), n = (uint32_t)(idx % a.n);
     const float *p = a.ws + (size_t)m * Npad + n;
     const size_t stride = (size_t)Mpad * Npad;
-    // split order; the loads of 8 splits are issued together, and on binary32
-    // activations they are also summed as equals before they join the rest
+    // split order; the loads of 8 splits are issued together
     float s = 0.0f;
     for (uint32_t j0 = 0; j0 < a.ksplit; j0 += 8) {
         float u[8];
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj) u[jj] = j0 + jj < a.ksplit ? p[(j0 + jj) * stride] : 0.0f;
-        if (a.a32) {
+        if constexpr (X32) {
             s += ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
             continue;
         }
@@ -1422,7 +1423,9 @@ constexpr int gemm_kw() {
 
 int launch_reduce(janus_ctx *ctx, const GemmArgs &a, uint32_t mpad) {
     const size_t total = (size_t)a.rows * a.n;
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, a, mpad);
+    const dim3 grid((unsigned)((total + 255) / 256));
+    if (a.a32) hipLaunchKernelGGL(gemm_reduce_kernel<true>, grid, dim3(256), 0, ctx->stream, a, mpad);
+    else hipLaunchKernelGGL(gemm_reduce_kernel<false>, grid, dim3(256), 0, ctx->stream, a, mpad);
     JANUS_LAUNCH_CHECK(ctx);
     return JANUS_OK;
 }
@@ -1631,14 +1634,17 @@ int launch_x32_mt(janus_ctx *ctx, const GemmArgs &a, const janus_weight *w, Gemm
 // ---- more than 64 rows (prompts) -----------------------------------------------
 // gemm_pipe_kernel over M tiles of 32 MT rows with 8 row groups per workgroup
 // (256 weight rows) and no K slices: a staged activation tile serves all 8
-// wavefronts, and a weight chunk is unpacked once for MT MFMA pairs. MT = 4
-// for binary16 rows (2 x 35 KB of LDS), 2 for three bfloat16 parts (2 x 52 KB).
-// Bound by the VALU (one scale FMA per weight and 32 rows, 0.4 more to unpack)
-// on binary16 rows and by LDS reads of the parts on binary32 rows. Q4_0
-// 28672x4096 at 512 rows: 167 us (721 TFLOP/s) against 229 with 4 row groups
-// x 2 K slices and 186 with MT = 2; binary32 rows 411 us (875 TFLOP/s of
-// MFMA) against 464, and 556 with MT = 3. A product with too few tiles for
-// the CUs splits K over workgroups.
+// wavefronts, and a weight chunk is unpacked once for MT MFMA pairs. MT = 4 or 3
+// for binary16 rows (2 x 35 KB of LDS at 4); three bfloat16 parts take 64 rows
+// (MT = 2, 2 x 52 KB), 96 (MT = 3, not for F16 weights) or 64 with 4 row groups
+// and two K slices, whichever launch_wide reckons the fastest. Bound by the
+// VALU (one scale FMA per weight and 32 rows, 0.4 more to unpack) on binary16
+// rows and by LDS reads of the parts on binary32 rows. Q4_0 28672x4096 at 512
+// rows: 167 us when the forms were compared (178 in a traced prompt) against
+// 229 with 4 row groups x 2 K slices and 186 with MT = 2; binary32 rows 411 us
+// with MT = 2, 464 with 4 row groups, and 556 with MT = 3, which pays only where
+// it saves a round of workgroups. A product with too few tiles for the CUs
+// splits K over workgroups.
 constexpr int kWideNW = 8;
 
 template <class F, int MT, bool X32, int NW = kWideNW, int KW = 1>
