@@ -47,13 +47,19 @@ HIP_FLAGS = [
 ]
 
 
+# Flags of single sources. prefill.hip: a wavefront may take 512 registers there
+# (one workgroup per CU), where the compiler otherwise puts every MFMA result in
+# accumulation registers and moves it back for each add.
+SRC_FLAGS = {"prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+
+
 def _sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
 
 def _compile(src: Path, out_dir: Path = BUILD, extra: tuple = ()) -> Path:
     obj = out_dir / (src.stem + ".o")
-    cmd = [HIPCC, *HIP_FLAGS, *extra, "-c", str(src), "-o", str(obj)]
+    cmd = [HIPCC, *HIP_FLAGS, *SRC_FLAGS.get(src.stem, []), *extra, "-c", str(src), "-o", str(obj)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{res.stdout}\n{res.stderr}")

@@ -21,15 +21,18 @@
 //    split or rounded.
 // Sums run as short chains joined as equals (four dims of a score, eight
 // positions of P.V; four tiles of output before they join the running one), a
-// score is scaled after the maximum is taken off and l is a double: against 64 bits the
-// output is as close as the decode kernels' (rms 0.8 to 1.02 of their error over
-// up to 512 positions; with one chain per score and output, two parts of P and
-// q scaled down only, it was 1.1 to 2.2, and 120 where q was small).
+// score is scaled after the maximum is taken off and l is a double: against 64
+// bits the output is as close as the decode kernels' (rms 0.8 to 1.02 of their
+// error over up to 512 positions; with one chain per score and output, two parts
+// of P and q scaled down only, it was 1.1 to 2.2, and 120 where q was small).
 //
 // Bound by the longest row tile's chain of K/V tiles (a 512-row chunk is 128
-// workgroups of four heads, so CUs are idle). Per call, back to back: 49 us for
+// workgroups of four heads, so CUs are idle). Per call, back to back: 50 us for
 // 512 binary16 rows at 32/8/128 heads against 160 through the decode kernels,
-// 45 us for 133 binary32 rows at 32/32/128 (38 and 33 with the longer chains).
+// 38 us for 133 binary32 rows at 32/32/128 (38 and 33 with the longer chains).
+// Built with MFMA results in vector registers: the compiler's choice for
+// wavefronts of 512 registers, accumulation registers, takes a move per add
+// (45 us for the binary32 rows).
 #include <type_traits>
 
 #include "internal.h"
