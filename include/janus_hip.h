@@ -82,7 +82,12 @@ const char *janus_status_string(int status);
 int janus_abi_version(void);
 /* Run subsequent calls on `hip_stream` (a hipStream_t) exactly as given:
  * NULL selects the legacy default stream. A new context runs on its own
- * non-blocking stream, which janus_get_stream returns before any change. */
+ * non-blocking stream, which janus_get_stream returns before any change.
+ * The context's workspaces (attention and matrix products, also those of
+ * graphs captured from its calls) are shared by all its calls: work enqueued
+ * on the stream before must be ordered ahead of what follows on this one, and
+ * a captured graph ahead of eager calls. Work that overlaps takes a context
+ * of its own. */
 int janus_set_stream(janus_ctx *ctx, void *hip_stream);
 void *janus_get_stream(janus_ctx *ctx);
 int janus_sync(janus_ctx *ctx);                      /* device.poll(wait) */
@@ -134,7 +139,16 @@ int janus_weight_dequant(janus_ctx *ctx, const janus_weight *w, float *d_out);
  * (F32 rows as three exact bfloat16 parts; two F32 rows, or three of a small
  * product, run the GEMV kernels row by row)
  * (the reference's M>1 quantized fallback, quantized.rs:77-90, is replaced
- * by a correct product). k and n must match the weight. */
+ * by a correct product). k and n must match the weight.
+ *
+ * The first call on a weight that takes the MFMA GEMM, outside any capture,
+ * makes a copy of the weight in that kernel's layout: it allocates about the
+ * weight's size again, kept until janus_weight_free, and waits for the stream.
+ * F32 rows do without it, on the row kernels, where it cannot be had (inside a
+ * capture, or no memory: not asked for again) or is of no use (a binary16
+ * weight with an infinity or NaN). Products whose K is split grow and use the
+ * context's workspace (janus_set_stream). A weight may be used by several
+ * contexts, each in its thread. */
 int janus_gemm_auto(janus_ctx *ctx, const void *a, int a_dtype, const janus_weight *w,
                     void *c, int c_dtype, uint32_t batch, uint32_t m, uint32_t k,
                     uint32_t n);
